@@ -99,28 +99,27 @@ int launch_bmt_dma_grid_t(const exc_dev &d, const kdesc *ks, const mt_item *item
   return EXC_OK;
 }
 
-__global__ __launch_bounds__(lo_dev::kRows * lo_dev::kSlots) void blo_apw_kernel(const kdesc *__restrict__ ks, int naa,
-                                                                                  int maxnlo, int nlomax, int apwordmax,
-                                                                                  int nlotot,
-                                                                                  const lo_desc *__restrict__ lod,
-                                                                                  const cplx *__restrict__ loa,
-                                                                                  const double *__restrict__ oalo,
-                                                                                  const double *__restrict__ h1loa) {
+template <int MAXLO>
+__global__ __launch_bounds__(lo_dev::kThreads) void blo_kernel(
+    const kdesc *__restrict__ ks, int naa, int maxnlo, int nlomax, int apwordmax, int nlotot,
+    const int *__restrict__ dlo, const lo_desc *__restrict__ lod, const cplx *__restrict__ loa,
+    const double *__restrict__ oalo, const double *__restrict__ h1loa, const cplx *__restrict__ lolo,
+    const double *__restrict__ ololo, const double *__restrict__ h1lolo) {
   __shared__ lo_dev::ApwLoShared sh;
   const kdesc k = ks[blockIdx.z];
-  if ((int)blockIdx.x * lo_dev::kRows >= k.ngp) return;
-  lo_dev::lo_apw_body(sh, blockIdx.x, blockIdx.y, k.ngp, naa, maxnlo, nlomax, apwordmax, nlotot, lod, k.apwalm, k.ldg,
-                      loa, oalo, h1loa, k.h, k.o, k.ldh);
+  if (blockIdx.x == 0)
+    lo_dev::lo_lo_atom(blockIdx.y, dlo, k.ngp, nlotot, maxnlo, nlomax, lod, lolo, ololo, h1lolo, k.h, k.o, k.ldh);
+  else
+    lo_dev::lo_apw_body<MAXLO>(sh, blockIdx.x - 1, blockIdx.y, k.ngp, naa, maxnlo, nlomax, apwordmax, dlo, lod,
+                               k.apwalm, k.ldg, loa, oalo, h1loa, k.h, k.o, k.ldh);
 }
 
-__global__ __launch_bounds__(lo_dev::kLoThreads) void blo_lo_kernel(const kdesc *__restrict__ ks, int nlotot, int maxnlo,
-                                                                     int nlomax, const lo_desc *__restrict__ lod,
-                                                                     const cplx *__restrict__ lolo,
-                                                                     const double *__restrict__ ololo,
-                                                                     const double *__restrict__ h1lolo) {
-  const kdesc k = ks[blockIdx.z];
-  lo_dev::lo_lo_body(blockIdx.x * lo_dev::kLoThreads + threadIdx.x, blockIdx.y, k.ngp, nlotot, maxnlo, nlomax, lod,
-                     lolo, ololo, h1lolo, k.h, k.o, k.ldh);
+template <int MAXLO>
+void launch_blo_t(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hipStream_t s) {
+  const dim3 grid(1 + (maxngp + lo_dev::kRows - 1) / lo_dev::kRows, d.natm, nk);
+  hipLaunchKernelGGL(blo_kernel<MAXLO>, grid, dim3(lo_dev::kThreads), 0, s, ks, d.naa, d.maxnlo, d.nlomax,
+                     d.apwordmax, d.nlotot, d.dm_lo, d.lod, d.loa, d.oalo, (d.iora & 2) ? d.h1loa : nullptr, d.lolo,
+                     d.ololo, (d.iora & 2) ? d.h1lolo : nullptr);
 }
 
 }  // namespace
@@ -176,15 +175,9 @@ int exc_launch_bmt(const exc_dev &d, const kdesc *ks, const mt_item *items, int 
 int exc_launch_blo(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hipStream_t s) {
   if (nk <= 0 || d.nlotot == 0) return EXC_OK;
   if (d.maxnlo > lo_dev::kMaxLo) return EXC_ERR_UNSUPPORTED;
-  if (maxngp > 0) {
-    dim3 grid((maxngp + lo_dev::kRows - 1) / lo_dev::kRows, d.natm, nk);
-    hipLaunchKernelGGL(blo_apw_kernel, grid, dim3(lo_dev::kRows * lo_dev::kSlots), 0, s, ks, d.naa, d.maxnlo, d.nlomax,
-                       d.apwordmax, d.nlotot, d.lod, d.loa, d.oalo, (d.iora & 2) ? d.h1loa : nullptr);
-    EXC_CHECK(hipGetLastError());
-  }
-  dim3 grid2((d.nlotot + lo_dev::kLoThreads - 1) / lo_dev::kLoThreads, d.nlotot, nk);
-  hipLaunchKernelGGL(blo_lo_kernel, grid2, dim3(lo_dev::kLoThreads), 0, s, ks, d.nlotot, d.maxnlo, d.nlomax, d.lod,
-                     d.lolo, d.ololo, (d.iora & 2) ? d.h1lolo : nullptr);
+  if (d.dm_maxlo <= 4) launch_blo_t<4>(d, nk, maxngp, ks, s);
+  else if (d.dm_maxlo <= 8) launch_blo_t<8>(d, nk, maxngp, ks, s);
+  else launch_blo_t<16>(d, nk, maxngp, ks, s);
   EXC_CHECK(hipGetLastError());
   return EXC_OK;
 }
