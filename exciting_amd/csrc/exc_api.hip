@@ -221,15 +221,15 @@ int exc_ctx_set_variant(exc_ctx *c, int stage, int variant) {
   if (!c) return EXC_ERR_ARG;
   switch (stage) {
     case EXC_STAGE_YSTAGE:
-      if (variant < -1 || variant >= kYstageVariants) return EXC_ERR_ARG;
+      if (variant < -1 || (variant >= kYstageVariants && variant != kYWave1 && variant != kYWave2)) return EXC_ERR_ARG;
       c->y_variant = variant;
       return EXC_OK;
     case EXC_STAGE_MT:
-      if (variant < -1 || variant >= kMtVariants) return EXC_ERR_ARG;
+      if (variant < -1 || (variant >= kMtVariants && variant != kMtWave1 && variant != kMtWave2)) return EXC_ERR_ARG;
       c->mt_variant = variant;
       return EXC_OK;
     case EXC_STAGE_BMT:
-      if (variant < -1 || variant >= kBmtVariants) return EXC_ERR_ARG;
+      if (variant < -1 || (variant >= kBmtVariants && variant != kMtWave1 && variant != kMtWave2)) return EXC_ERR_ARG;
       c->bmt_variant = variant;
       return EXC_OK;
     case EXC_STAGE_BSPLIT:
@@ -612,6 +612,28 @@ int exc_match(exc_ctx *c, int ngp, int ngkmax, const double *gpc, const double *
 
 namespace {
 
+// Tiles of the Y stage and the muffin-tin stage by the number of 64-wide ones a call has: below
+// about half the CUs the 16-wide tiles of mt_wave.h (their four waves also split the sum over
+// k), up to two per CU the 32-wide ones, beyond that the 64-wide ones, whose operands are
+// read a quarter as often.  Measured on 256 CUs, MT stage (us; 64-, 16-, 32-wide): 24 tiles
+// (2 atoms, N = 97, 8 k-points) 48, 12, 22; 90 (5 atoms, N = 260, 8 k) 113, 55, 74; 175 (16 k)
+// 115, 98, 110; 190 (8 atoms, N = 1200, 1 k) 262, 255, 231; 528 (5 atoms, N = 700, 8 k) 431, 444,
+// 405; 741 (8 atoms, N = 1200, 4 k) 739, 1004, 870.  The count is H's alone, so that H does not
+// depend on whether O is formed with it.
+int mt_narrow(const exc_ctx *c, long tiles, int wide) {
+  return 2 * tiles <= c->ncu ? kMtWave1 : tiles <= 2 * c->ncu ? kMtWave2 : wide;
+}
+
+// The Y stage by its 64 x 128 tiles: 16-wide ones up to three quarters of the CUs.  Measured
+// (us; wide, 16-wide): 8 tiles (2 atoms, N = 97) 46, 8; 50 (5 atoms, N = 260) 48, 19; 200 (4 k) 50,
+// 48; 400 (8 k) 83, 88.
+int y_narrow(const exc_ctx *c, long tiles, int wide) { return 4 * tiles <= 3 * c->ncu ? kYWave1 : wide; }
+
+long tri_tiles(int ngp, int t) {
+  const long n = (ngp + t - 1) / t;
+  return n * (n + 1) / 2;
+}
+
 // H (h given), O (o given) or both of one k-point from device arrays
 // ws: the Y stage's workspace; NULL takes the context's grow-only buffer.  With a caller's
 // workspace nothing is allocated and no stage timer runs (a timer may create its events).
@@ -625,10 +647,13 @@ int setup_dev_sel(exc_ctx *c, int ngp, int ngkmax, const double *apwalm, const i
   if (rc) return rc;
   const bool untimed = ws != nullptr;   // a StageTimer of stage -1 records nothing
   if (ngp > 0) {
-    // defaults from the autotuner's sweep on MI355X (64x64 MT and Y tiles, LDS filled by DMA;
-    // the MT tile with Gauss's three real products per complex product)
-    const int yv = c->y_variant >= 0 ? c->y_variant : 3;
-    const int mv = c->mt_variant >= 0 ? c->mt_variant : 0;
+    // defaults: the narrow tiles at small sizes (the per-k call has H's and O's tiles: twice
+    // H's count), else from the autotuner's sweep on MI355X (64x64 MT and Y tiles, LDS filled
+    // by DMA; the MT tile with Gauss's three real products per complex product).  MT at N = 97
+    // (2 atoms) 47 -> 10 us, N = 260 (5 atoms) 110 -> 26; Y 28 -> 8, 30 -> 18
+    const long ytiles = (long)((ngp + 63) / 64) * ((c->d.naa + 127) / 128) * c->d.natm;
+    const int yv = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, 3);
+    const int mv = c->mt_variant >= 0 ? c->mt_variant : mt_narrow(c, 2 * tri_tiles(ngp, 64), 0);
     cplx *yt = ws;
     if (h) {   // the Y stage feeds only H
       if (!ws) {
@@ -865,8 +890,14 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   // defaults: the fastest variants measured on MI355X for N = 1150..5000 (grouped MT: 64x64
   // tile, 8 waves, two LDS stages filled by DMA, one item per workgroup; split: 64x64 tile,
   // LDS filled by DMA)
-  const int bv = split ? (c->bsplit_variant >= 0 ? c->bsplit_variant : 3) : (c->bmt_variant >= 0 ? c->bmt_variant : 0);
-  const int yv = c->y_variant >= 0 ? c->y_variant : 0;     // 64x128 Y tiles, DMA-staged, 3 real products
+  long mtiles = 0, ytiles = 0;
+  for (int k = 0; k < nk; ++k) {
+    mtiles += tri_tiles(ks[k].ngp, 64);
+    ytiles += (long)((ks[k].ngp + 63) / 64) * ((c->d.naa + 127) / 128) * c->d.natm;
+  }
+  const int bv = split ? (c->bsplit_variant >= 0 ? c->bsplit_variant : 3)
+                       : (c->bmt_variant >= 0 ? c->bmt_variant : mt_narrow(c, mtiles, 0));
+  const int yv = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, 0);   // 64x128 Y tiles, DMA-staged, 3 products
   // residue GEMM: the register-pipelined 256 x 256 form from N = 2048, 128 x 128 tiles below
   int maxn = 0;
   for (int k = 0; k < nk; ++k) maxn = std::max(maxn, ks[k].ngp);
@@ -903,7 +934,7 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   // (64 x 64 three-product tiles, 5.7 against 6.7 ms at workload 3; the dense Y stage keeps
   // 64 x 128, 8.8 against 9.1 ms)
   const bool etri = gram && c->gram_tri;
-  const int ye = c->y_variant >= 0 ? c->y_variant : (etri ? 4 : 0);
+  const int ye = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, etri ? 4 : 0);
   int tail[10] = {nk, flags, bv, yv, crt ? cv : -1, (crt ? nmod : -1) + 100 * ov, fv, gram, etri, ye};
   std::vector<char> sig(sizeof(exc_kpoint_dev) * nk + sizeof(tail));
   memcpy(sig.data(), ks, sizeof(exc_kpoint_dev) * nk);

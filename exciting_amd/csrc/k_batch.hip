@@ -9,6 +9,7 @@
 #include "match_dev.h"
 #include "setup_dev.h"
 #include "mt_dma.h"
+#include "mt_wave.h"
 
 namespace {
 
@@ -99,6 +100,54 @@ int launch_bmt_dma_grid_t(const exc_dev &d, const kdesc *ks, const mt_item *item
   return EXC_OK;
 }
 
+// narrow tiles (mt_wave.h)
+template <int TB>
+__global__ __launch_bounds__(256) void bystage_wave_kernel(const kdesc *__restrict__ ks, int natm, int naa,
+                                                           const cplx *__restrict__ haa,
+                                                           const int *__restrict__ fperm, int tri) {
+  using T = YTileWave<TB>;
+  __shared__ typename T::C::Red red;
+  const int ias = blockIdx.z % natm;
+  const kdesc k = ks[blockIdx.z / natm];
+  const int row0 = blockIdx.x * T::C::T, col0 = blockIdx.y * T::C::T;
+  if (row0 >= k.ngp) return;
+  T::run(red, k.ngp, naa, k.apwalm + (size_t)k.ldg * naa * ias, k.ldg, haa + (size_t)naa * naa * ias,
+         k.yt + (size_t)k.ldy * naa * ias, k.ldy, row0, col0, fperm, tri ? min(col0, naa) : 0);
+}
+
+template <int TB>
+int launch_bystage_wave_t(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hipStream_t s) {
+  constexpr int T = 16 * TB;
+  hipLaunchKernelGGL(bystage_wave_kernel<TB>, dim3((maxngp + T - 1) / T, (d.naa + T - 1) / T, d.natm * nk), dim3(256),
+                     0, s, ks, d.natm, d.naa, d.haa, d.fperm, d.ytri);
+  EXC_CHECK(hipGetLastError());
+  return EXC_OK;
+}
+
+template <int TB>
+__global__ __launch_bounds__(256) void bmt_wave_kernel(const kdesc *__restrict__ ks,
+                                                       const mt_item *__restrict__ items, int nitems, int ktot,
+                                                       GTab gt, const int *__restrict__ kperm) {
+  using T = MtTileWave<TB>;
+  __shared__ typename T::C::Red red;
+  const int chunk = (nitems + 7) / 8;                   // XCD-contiguous items, as bmt_dma_grid_kernel
+  const int q = blockIdx.x / 8, it = (blockIdx.x % 8) * chunk + q;
+  if (q >= chunk || it >= nitems) return;
+  const mt_item w = items[it];
+  const kdesc k = ks[w.k];
+  T::run(red, k.ngp, ktot, k.apwalm, k.ldg, k.yt, k.ldy, k.igpig, k.vgpc, gt, k.h, k.o, k.ldh, kperm, w.ti, w.tj,
+         w.which);
+}
+
+template <int TB>
+int launch_bmt_wave_t(const exc_dev &d, const kdesc *ks, const mt_item *items, int nitems, hipStream_t s) {
+  const int chunk = (nitems + 7) / 8;
+  hipLaunchKernelGGL(bmt_wave_kernel<TB>, dim3(8 * chunk), dim3(256), 0, s, ks, items, nitems, d.natm * d.naa,
+                     make_gtab(d), d.kperm);
+  EXC_CHECK(hipGetLastError());
+  return EXC_OK;
+}
+
 template <int MAXLO>
 __global__ __launch_bounds__(lo_dev::kThreads) void blo_kernel(
     const kdesc *__restrict__ ks, int naa, int maxnlo, int nlomax, int apwordmax, int nlotot,
@@ -152,11 +201,13 @@ int exc_launch_bystage(const exc_dev &d, int nk, int maxngp, const kdesc *ks, in
     case 2: return launch_bystage_dma_t<64, 128, 8, 2, 2, 4>(d, nk, maxngp, ks, s);
     case 3: return launch_bystage_dma_t<64, 64, 16, 2, 2, 4>(d, nk, maxngp, ks, s);
     case 4: return launch_bystage_dma_t<64, 64, 8, 2, 2, 4, true>(d, nk, maxngp, ks, s);   // narrow, Gauss's form
+    case kYWave1: return launch_bystage_wave_t<1>(d, nk, maxngp, ks, s);
+    case kYWave2: return launch_bystage_wave_t<2>(d, nk, maxngp, ks, s);
     default: return EXC_ERR_ARG;
   }
 }
 
-int exc_bmt_tile(int variant) { return variant >= 0 && variant < kBmtVariants ? 64 : 0; }
+int exc_bmt_tile(int variant) { return variant == kMtWave1 ? 16 : variant == kMtWave2 ? 32 : 64; }
 
 // grouped MT variants: 64 x 64 tile, 8 waves; 0: BK 16, two DMA stages, Gauss's three real
 // products per complex product (the default); 1: the same with four products; 2: BK 8, four
@@ -168,6 +219,8 @@ int exc_launch_bmt(const exc_dev &d, const kdesc *ks, const mt_item *items, int 
     case 1: return launch_bmt_dma_grid_t<64, 16, 2, 2, 4>(d, ks, items, nitems, s);
     case 2: return launch_bmt_dma_grid_t<64, 8, 4, 2, 4, true>(d, ks, items, nitems, s);
     case 3: return launch_bmt_dma_grid_t<64, 16, 3, 2, 4, true>(d, ks, items, nitems, s);
+    case kMtWave1: return launch_bmt_wave_t<1>(d, ks, items, nitems, s);
+    case kMtWave2: return launch_bmt_wave_t<2>(d, ks, items, nitems, s);
     default: return EXC_ERR_ARG;
   }
 }

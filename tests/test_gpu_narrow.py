@@ -1,0 +1,60 @@
+"""The narrow muffin-tin and Y tiles (mt_wave.h) and the lo kernel at tile edges and remainders.
+
+H and O of the 16- and 32-wide tiles against the four-product 64-wide variants, which sum the
+same terms in another order: within 1e-14 relative (the bar of the other reorderings), and
+against the oracle to 1e-12.  Sizes around multiples of 16 and 32, the smallest basis, K not a
+multiple of the four waves' k-steps, and lo counts of every accumulator size (4, 8, 16)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,lmax,lo,natm", [(3, 1, (0,), (1,)), (15, 2, (0, 1), (1, 1)), (16, 3, (0, 1, 1), (2,)),
+                                            (17, 3, (0, 1), (1, 2)), (33, 4, (0, 0, 1, 1), (1, 1)),
+                                            (64, 5, (0, 1, 2, 2), (1, 2)), (97, 2, (), (1, 1)), (130, 8, (0, 1), (1, 2))])
+def test_narrow_tiles(n, lmax, lo, natm):
+    import torch
+    from exciting_amd import lapw, synth
+    from oracle import lapw_ref as R
+    w = synth.make_small(natm_per_species=natm, lmax=lmax, lorbl=lo or (0,), n_target=n, nk=3, seed=11 + n,
+                         cell=(9.0, 9.5, 10.0))
+    cr = w.crystal
+    s = torch.cuda.Stream()
+    ctx = lapw.Context(cr, stream=s)
+    with torch.cuda.stream(s):
+        b = lapw.DeviceBatch(cr, w.kpoints)
+
+        def perk():
+            for i, d in enumerate(b.dks):
+                ctx.match_dev(d.ngp, d.ngkmax, d.gpc, d.tpgpc, d.sfacgp, b.apw[i])
+                ctx.setup_dev(d.ngp, d.ngkmax, b.apw[i], d.igpig, d.vgpc, b.nmat[i], b.H[i], b.O[i])
+
+        def grouped():
+            ctx.setup_batched_dev(b, lapw.EXC_BATCH_MATCH)
+
+        def result(run):
+            for t in b.H + b.O:
+                t.fill_(float("nan"))
+            run()
+            torch.cuda.synchronize()
+            return [(h.cpu().numpy().T, o.cpu().numpy().T) for h, o in zip(b.H, b.O)]
+
+        ctx.set_variant("mt", 1)
+        ctx.set_variant("ystage", 3)
+        ref = result(perk)
+        for i, kp in enumerate(w.kpoints):
+            for m, mr in zip(ref[i], R.setup(cr, kp)[:2]):
+                assert np.linalg.norm(m - mr) <= 1e-12 * np.linalg.norm(mr)
+        for v in (-1, 16, 17):
+            for stage in ("mt", "bmt", "ystage"):
+                ctx.set_variant(stage, v)
+            for name, run in (("per-k", perk), ("grouped", grouped)):
+                print(f"N={n} lmax={lmax} {name} variant {v}", flush=True)
+                for (h, o), (h0, o0) in zip(result(run), ref):
+                    assert np.linalg.norm(h - h0) <= 1e-14 * np.linalg.norm(h0)
+                    assert np.linalg.norm(o - o0) <= 1e-14 * np.linalg.norm(o0)
+                    il = np.tril_indices(h.shape[0], -1)       # the strict lower triangle, as copy_UL leaves it
+                    assert np.array_equal(h[il], h.T[il].conj()) and np.array_equal(o[il], o.T[il].conj())
+    ctx.status()
+    ctx.close()
