@@ -138,8 +138,10 @@ int exc_launch_blo(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hipStr
 size_t exc_vjp_work_elems(const exc_dev &d, int ngp, int nst);
 int exc_launch_vjp(const exc_dev &d, int ngp, int nst, const cplx *apwalm, int ldg, const int *igpig,
                    const double *vgpc, const cplx *sfacgp, const cplx *evec, int ldc, const double *wh,
-                   const double *wo, cplx *work, double *dedtau, double *dedv, hipStream_t s);   // uv in work first
-int exc_launch_vjp_qscale(int ngp, int nst, const cplx *evec, int ldc, const double *vgpc, cplx *cs, hipStream_t s);
+                   const double *wo, cplx *work, double *dedtau, double *dedv, int ncu, int yv, hipStream_t s);
+// out[b os + i si + j] = sum_k X(k, i) Y(k, j) (k_atc.hip)
+int exc_launch_xty(int nb, int n, const cplx *X, int ldx, int ni, size_t xs, const cplx *Y, int ldy, int nj, size_t ys,
+                   cplx *out, size_t si, size_t os, int ncu, hipStream_t s);
 // split-BF16 muffin-tin stage
 constexpr int kSplitKB = 256;       // APW functions per atom block, padded (naa <= 256)
 constexpr int kSplitPlanes = 6;     // 3 slices x (re, im)
