@@ -221,7 +221,7 @@ int exc_ctx_set_variant(exc_ctx *c, int stage, int variant) {
   if (!c) return EXC_ERR_ARG;
   switch (stage) {
     case EXC_STAGE_YSTAGE:
-      if (variant < -1 || (variant >= kYstageVariants && variant != kYWave1 && variant != kYWave2)) return EXC_ERR_ARG;
+      if (variant < -1 || (variant >= kYstageVariants && (variant < kYWave1 || variant > kYDirect))) return EXC_ERR_ARG;
       c->y_variant = variant;
       return EXC_OK;
     case EXC_STAGE_MT:
@@ -229,7 +229,7 @@ int exc_ctx_set_variant(exc_ctx *c, int stage, int variant) {
       c->mt_variant = variant;
       return EXC_OK;
     case EXC_STAGE_BMT:
-      if (variant < -1 || (variant >= kBmtVariants && variant != kMtWave1 && variant != kMtWave2)) return EXC_ERR_ARG;
+      if (variant < -1 || (variant >= kBmtVariants && (variant < kMtWave1 || variant > kMtWave2))) return EXC_ERR_ARG;
       c->bmt_variant = variant;
       return EXC_OK;
     case EXC_STAGE_BSPLIT:
@@ -612,22 +612,25 @@ int exc_match(exc_ctx *c, int ngp, int ngkmax, const double *gpc, const double *
 
 namespace {
 
-// Tiles of the Y stage and the muffin-tin stage by the number of 64-wide ones a call has: below
-// about half the CUs the 16-wide tiles of mt_wave.h (their four waves also split the sum over
-// k), up to two per CU the 32-wide ones, beyond that the 64-wide ones, whose operands are
-// read a quarter as often.  Measured on 256 CUs, MT stage (us; 64-, 16-, 32-wide): 24 tiles
-// (2 atoms, N = 97, 8 k-points) 48, 12, 22; 90 (5 atoms, N = 260, 8 k) 113, 55, 74; 175 (16 k)
-// 115, 98, 110; 190 (8 atoms, N = 1200, 1 k) 262, 255, 231; 528 (5 atoms, N = 700, 8 k) 431, 444,
-// 405; 741 (8 atoms, N = 1200, 4 k) 739, 1004, 870.  The count is H's alone, so that H does not
-// depend on whether O is formed with it.
+// Tiles of the muffin-tin stage by the number of 64-wide ones a call has: below about half the
+// CUs the 16-wide tiles of mt_wave.h (their four waves also split the sum over k), up to five per
+// two CUs the 32-wide ones, beyond that the 64-wide ones, whose operands are read half as
+// often.  Measured on 256 CUs (us; 64-, 16-, 32-wide): 24 tiles (2 atoms, N = 97, 8 k-points) 48, 12,
+// 20; 90 (5 atoms, N = 260, 8 k) 113, 55, 66; 175 (16 k) 115, 95, 98; 190 (8 atoms, N = 1200, 1 k) 262,
+// 256, 207; 528 (5 atoms, N = 700, 8 k) 434, 441, 360; 741 (8 atoms, N = 1200, 4 k) 729, 1010, 774.  The
+// count is H's alone, so that H does not depend on whether O is formed with it.
 int mt_narrow(const exc_ctx *c, long tiles, int wide) {
-  return 2 * tiles <= c->ncu ? kMtWave1 : tiles <= 2 * c->ncu ? kMtWave2 : wide;
+  return 2 * tiles <= c->ncu ? kMtWave1 : 2 * tiles <= 5 * c->ncu ? kMtWave2 : wide;
 }
 
-// The Y stage by its 64 x 128 tiles: 16-wide ones up to three quarters of the CUs.  Measured
-// (us; wide, 16-wide): 8 tiles (2 atoms, N = 97) 46, 8; 50 (5 atoms, N = 260) 48, 19; 200 (4 k) 50,
-// 48; 400 (8 k) 83, 88.
-int y_narrow(const exc_ctx *c, long tiles, int wide) { return 4 * tiles <= 3 * c->ncu ? kYWave1 : wide; }
+// The Y stage by its 64 x 128 tiles: 16-wide up to a quarter of the CUs, 32-wide up to two per CU,
+// the 64-wide ones without LDS up to five per CU.  Measured (us; wide, 16-, 32-, 64-wide direct): 8
+// tiles (2 atoms, N = 97) 46, 8, 12, 26; 64 (8 k) 48, 22, 19, 27; 200 (5 atoms, N = 260, 4 k) 50, 51, 36, 47;
+// 400 (8 k) 83, 93, 63, 66; 560 (5 atoms, N = 400, 8 k) 178, 225, 150, 147; 1216 (8 atoms, N = 1200, 4 k)
+// 304, 564, 308, 275; 4864 (16 k) 1054, -, 1188, 1049; 10240 (16 atoms, N = 2500, 8 k) 2101, -, 2488, 2221.
+int y_narrow(const exc_ctx *c, long tiles, int wide) {
+  return 4 * tiles <= c->ncu ? kYWave1 : tiles <= 2 * c->ncu ? kYWave2 : tiles <= 5 * c->ncu ? kYDirect : wide;
+}
 
 long tri_tiles(int ngp, int t) {
   const long n = (ngp + t - 1) / t;
@@ -650,7 +653,7 @@ int setup_dev_sel(exc_ctx *c, int ngp, int ngkmax, const double *apwalm, const i
     // defaults: the narrow tiles at small sizes (the per-k call has H's and O's tiles: twice
     // H's count), else from the autotuner's sweep on MI355X (64x64 MT and Y tiles, LDS filled
     // by DMA; the MT tile with Gauss's three real products per complex product).  MT at N = 97
-    // (2 atoms) 47 -> 10 us, N = 260 (5 atoms) 110 -> 26; Y 28 -> 8, 30 -> 18
+    // (2 atoms) 47 -> 10 us, N = 260 (5 atoms) 110 -> 24; Y 28 -> 8, 30 -> 18
     const long ytiles = (long)((ngp + 63) / 64) * ((c->d.naa + 127) / 128) * c->d.natm;
     const int yv = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, 3);
     const int mv = c->mt_variant >= 0 ? c->mt_variant : mt_narrow(c, 2 * tri_tiles(ngp, 64), 0);

@@ -125,9 +125,10 @@ int exc_launch_mt(const exc_dev &d, int ngp, const cplx *apwalm, int ldg, const 
 constexpr int kYstageVariants = 5;   // per-k and grouped Y stage (the same shapes)
 constexpr int kMtVariants = 3;       // per-k MT
 constexpr int kBmtVariants = 4;      // grouped MT
-// the narrow tiles of mt_wave.h, 16 and 32 wide (per-k and grouped), chosen by the built-in rules
-// at small sizes; they sum in another order than the variants counted above
-constexpr int kYWave1 = 16, kYWave2 = 17, kMtWave1 = 16, kMtWave2 = 17;
+// the tiles of mt_wave.h (per-k and grouped), chosen by the built-in rules at small sizes: 16 and
+// 32 wide with the sum split over the waves, and 64 wide without (Y stage); they sum in another
+// order than the variants counted above
+constexpr int kYWave1 = 16, kYWave2 = 17, kYDirect = 18, kMtWave1 = 16, kMtWave2 = 17;
 // Grouped launches over nk k-points described by ks (device memory); maxngp bounds the grids.
 int exc_launch_bmatch(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hipStream_t s);
 int exc_launch_bystage(const exc_dev &d, int nk, int maxngp, const kdesc *ks, int variant, hipStream_t s);

@@ -148,6 +148,25 @@ int launch_bmt_wave_t(const exc_dev &d, const kdesc *ks, const mt_item *items, i
   return EXC_OK;
 }
 
+// one 32 x 32 block per wave, operands straight to registers (mt_wave.h)
+__global__ __launch_bounds__(256, 2) void bystage_direct_kernel(const kdesc *__restrict__ ks, int natm, int naa,
+                                                                const cplx *__restrict__ haa,
+                                                                const int *__restrict__ fperm, int tri) {
+  const int ias = blockIdx.z % natm;
+  const kdesc k = ks[blockIdx.z / natm];
+  const int row0 = blockIdx.x * 64, col0 = blockIdx.y * 64;
+  if (row0 >= k.ngp) return;
+  YTileDirect::run(k.ngp, naa, k.apwalm + (size_t)k.ldg * naa * ias, k.ldg, haa + (size_t)naa * naa * ias,
+                   k.yt + (size_t)k.ldy * naa * ias, k.ldy, row0, col0, fperm, tri ? min(col0, naa) : 0);
+}
+
+int launch_bystage_direct(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hipStream_t s) {
+  hipLaunchKernelGGL(bystage_direct_kernel, dim3((maxngp + 63) / 64, (d.naa + 63) / 64, d.natm * nk), dim3(256), 0, s, ks,
+                     d.natm, d.naa, d.haa, d.fperm, d.ytri);
+  EXC_CHECK(hipGetLastError());
+  return EXC_OK;
+}
+
 template <int MAXLO>
 __global__ __launch_bounds__(lo_dev::kThreads) void blo_kernel(
     const kdesc *__restrict__ ks, int naa, int maxnlo, int nlomax, int apwordmax, int nlotot,
@@ -203,6 +222,7 @@ int exc_launch_bystage(const exc_dev &d, int nk, int maxngp, const kdesc *ks, in
     case 4: return launch_bystage_dma_t<64, 64, 8, 2, 2, 4, true>(d, nk, maxngp, ks, s);   // narrow, Gauss's form
     case kYWave1: return launch_bystage_wave_t<1>(d, nk, maxngp, ks, s);
     case kYWave2: return launch_bystage_wave_t<2>(d, nk, maxngp, ks, s);
+    case kYDirect: return launch_bystage_direct(d, nk, maxngp, ks, s);
     default: return EXC_ERR_ARG;
   }
 }

@@ -4,7 +4,7 @@
 // A workgroup takes one (16 TB) x (16 TB) tile; its 4 waves (one per SIMD) split the sum over
 // k and are added in wave order through LDS at the end.  The operands go from global memory
 // (L2) straight to registers in the MFMA layout (16 rows of 16 bytes contiguous per k), U
-// k-steps of 4 ahead of their use: no LDS staging and no barrier in the K loop, so a wave's time
+// to 2 U k-steps of 4 ahead of their use: no LDS staging and no barrier in the K loop, so a wave's time
 // is its MFMA chain plus one memory latency per U steps, and the interstitial values of the
 // elements a wave finishes are looked up before the K loop (three dependent loads).
 // Gauss's three real products per complex product, as the 64-wide default.
@@ -49,10 +49,17 @@ struct WaveCore {
   __device__ __forceinline__ static void run(const cplx *__restrict__ A, int lda, int row0, int mrows,
                                              const cplx *__restrict__ B, int ldb, int col0, int nrows, int ktot,
                                              const int *__restrict__ kperm, d4_t (&cr)[TB][TB], d4_t (&ci)[TB][TB]) {
-    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int per = (ktot + 15) / 16 * 4;          // k's per wave, whole k-steps
-    const int kb = wave * per, ke = min(ktot, kb + per);
+    sum(A, lda, row0, mrows, B, ldb, col0, nrows, ktot, wave * per, min(ktot, (wave + 1) * per), kperm, cr, ci);
+  }
+
+  // the same for k in [kb, ke)
+  __device__ __forceinline__ static void sum(const cplx *__restrict__ A, int lda, int row0, int mrows,
+                                             const cplx *__restrict__ B, int ldb, int col0, int nrows, int ktot, int kb,
+                                             int ke, const int *__restrict__ kperm, d4_t (&cr)[TB][TB],
+                                             d4_t (&ci)[TB][TB]) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
     const cplx *pa[TB], *pb[TB];
 #pragma unroll
     for (int i = 0; i < TB; ++i) {
@@ -66,16 +73,7 @@ struct WaveCore {
 #pragma unroll
       for (int j = 0; j < TB; ++j) p1[i][j] = p2[i][j] = p3[i][j] = d4_t{0.0, 0.0, 0.0, 0.0};
     const int klast = ktot - 1;
-    int kc[U];
-    Group g;
-    cols(kc, kperm, kb, klast);
-    load(g, kc, pa, lda, pb, ldb);
-    cols(kc, kperm, kb + 4 * U, klast);
-#pragma unroll 1
-    for (int k0 = kb; k0 < ke; k0 += 4 * U) {
-      Group n;
-      load(n, kc, pa, lda, pb, ldb);               // the next group's operands (past the end: the last k's again)
-      cols(kc, kperm, k0 + 8 * U, klast);
+    auto step = [&](const Group &g, int k0) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (k0 + 4 * u >= ke) break;
@@ -99,7 +97,25 @@ struct WaveCore {
             p3[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[i], bs[j], p3[i][j], 0, 0, 0);
           }
       }
-      g = n;
+    };
+    // two groups in turn, each refilled right after its use (a copy from one to the next would
+    // wait for the loads in flight); past the end they load the last k's again, unused
+    int kc[U];
+    Group g0, g1;
+    cols(kc, kperm, kb, klast);
+    load(g0, kc, pa, lda, pb, ldb);
+    cols(kc, kperm, kb + 4 * U, klast);
+    load(g1, kc, pa, lda, pb, ldb);
+    cols(kc, kperm, kb + 8 * U, klast);
+#pragma unroll 1
+    for (int k0 = kb; k0 < ke; k0 += 8 * U) {
+      step(g0, k0);
+      load(g0, kc, pa, lda, pb, ldb);
+      cols(kc, kperm, k0 + 12 * U, klast);
+      if (k0 + 4 * U >= ke) break;
+      step(g1, k0 + 4 * U);
+      load(g1, kc, pa, lda, pb, ldb);
+      cols(kc, kperm, k0 + 16 * U, klast);
     }
 #pragma unroll
     for (int i = 0; i < TB; ++i)
@@ -184,6 +200,32 @@ struct MtTileWave {
       out[r + (size_t)c * ldh] = cplx{re, im};
       if (r < c) out[c + (size_t)r * ldh] = cplx{re, -im};
     }
+  }
+};
+
+// one 64 x 64 tile of Yt_a with the waves 2 x 2 over the tile, each its 32 x 32 over all of k: the
+// 64-wide tile without LDS, operands shared between the waves through the CU's L1
+struct YTileDirect {
+  using C = WaveCore<2, false>;
+  __device__ static void run(int ngp, int naa, const cplx *__restrict__ A, int ldg, const cplx *__restrict__ ha,
+                             cplx *__restrict__ Y, int ldy, int row0, int col0, const int *__restrict__ fperm,
+                             int kfirst) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    row0 += 32 * (wave >> 1);
+    col0 += 32 * (wave & 1);
+    if (row0 >= ngp || col0 >= naa) return;
+    d4_t cr[2][2], ci[2][2];
+    C::sum(ha, naa, col0, naa, A, ldg, row0, ngp, naa - kfirst, 0, naa - kfirst, fperm + kfirst, cr, ci);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int e = 4 * (2 * i + j) + v;
+          const int c = col0 + C::row_of(e), r = row0 + C::col_of(e);
+          if (r < ngp && c < naa) Y[r + (size_t)c * ldy] = cplx{cr[i][j][v], ci[i][j][v]};
+        }
   }
 };
 
