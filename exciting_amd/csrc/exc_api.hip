@@ -182,7 +182,6 @@ int exc_ctx_destroy(exc_ctx *c) {
   if (c->crt_x) hipFree(c->crt_x);
   if (c->crt_parts) hipFree(c->crt_parts);
   if (c->gram_buf) hipFree(c->gram_buf);
-  if (c->gram_blas) rocblas_destroy_handle(c->gram_blas);
   if (c->gk_buf) hipFree(c->gk_buf);
   if (c->crt_res) hipFree(c->crt_res);
   if (c->d_citems) hipFree(c->d_citems);
@@ -731,75 +730,42 @@ int setup_host_sel(exc_ctx *c, int ngp, int ngkmax, const double *apwalm, const 
   return exc_ctx_status(c);
 }
 
-// The Gram form's table from every h_a (rocSOLVER, strided batches): the eigenvalues give
-// sigma = -min lambda (times 1 + 1e-6) when some lambda < 0, plus 1e-10 of the largest
-// |lambda| (h + sigma I is then positive definite beyond the eigensolver's rounding); the
-// table is the lower Cholesky factor of h + sigma I in the Y stage's summation order
-// (exc_launch_crt_gram_tri: a triangular table, whose Y stage skips the zero part), or, if
-// that factorization fails, conj(U) (Lambda + sigma)^(1/2) from the eigenvectors.  Once per
-// change of h_a; a failed eigensolve leaves the form unused.
+// The Gram form's table from every h_a (k_gram.hip): the extreme eigenvalues give sigma = -min
+// lambda (times 1 + 1e-6) when some lambda < 0, plus 1e-10 of the largest |lambda| (h + sigma I
+// is then positive definite beyond the eigenvalues' rounding); the table is conj(L), L the lower
+// Cholesky factor of h + sigma I in the Y stage's summation order, triangular, whose Y stage
+// skips the zero part.  Once per change of h_a; an h_a that is not finite, or a factorization
+// that fails, leaves the form unused.
 int gram_build(exc_ctx *c) {
   if (c->gram_valid) return EXC_OK;
   const int na = c->d.natm, n = c->d.naa;
   const size_t nn = (size_t)n * n * na;
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  const size_t o_u = al(sizeof(cplx) * nn), o_l = o_u + al(sizeof(cplx) * nn), o_e = o_l + al(8 * (size_t)n * na);
-  const size_t o_i = o_e + al(8 * (size_t)n * na), o_s = o_i + al(4 * (size_t)na);
-  const size_t o_m = o_s + al(8);
-  int rc = grow(&c->gram_buf, &c->gram_bytes, o_m + sizeof(cplx) * nn);
+  // the table, scratch, then (read back together) the extremes, sigma and the infos
+  const size_t o_w = al(sizeof(cplx) * nn), o_x = o_w + al(sizeof(cplx) * nn);
+  const size_t b_x = 8 * (2 * (size_t)na + 1) + 4 * (size_t)na;
+  int rc = grow(&c->gram_buf, &c->gram_bytes, o_x + b_x);
   if (rc) return rc;
   char *b = (char *)c->gram_buf;
-  cplx *T = (cplx *)b, *U = (cplx *)(b + o_u);
-  double *lam = (double *)(b + o_l), *E = (double *)(b + o_e), *dsig = (double *)(b + o_s);
-  int *info = (int *)(b + o_i);
-  cplx *Mp = (cplx *)(b + o_m);
-  c->gram_table = T;
-  c->gram_sig_dev = dsig;
-  EXC_CHECK(hipMemcpyAsync(U, c->d.haa, sizeof(cplx) * nn, hipMemcpyDeviceToDevice, c->stream));
-  // a handle of its own with the library-managed workspace (the eigensolve workers' handles
-  // hold fixed workspaces sized for their own calls); the stream is drained below
-  if (!c->gram_blas && rocblas_create_handle(&c->gram_blas) != rocblas_status_success) {
-    c->gram_blas = nullptr;
-    return EXC_ERR_HIP;
-  }
-  if (rocblas_set_stream(c->gram_blas, c->stream) != rocblas_status_success) return EXC_ERR_HIP;
-  const bool solved = rocsolver_zheevd_strided_batched(c->gram_blas, rocblas_evect_original, rocblas_fill_upper, n,
-                                                       (rocblas_double_complex *)U, n, (rocblas_stride)n * n, lam, n,
-                                                       E, n, info, na) == rocblas_status_success;
-  std::vector<double> hl((size_t)n * na);
-  std::vector<int> hi(na, 1);
-  if (solved) {
-    EXC_CHECK(hipMemcpyAsync(hl.data(), lam, 8 * hl.size(), hipMemcpyDeviceToHost, c->stream));
-    EXC_CHECK(hipMemcpyAsync(hi.data(), info, 4 * (size_t)na, hipMemcpyDeviceToHost, c->stream));
-  }
+  double *ext = (double *)(b + o_x);
+  c->gram_table = (cplx *)b;
+  c->gram_sig_dev = ext + 2 * na;
+  if ((rc = exc_launch_gram(c->d, (cplx *)(b + o_w), c->gram_table, ext, c->gram_sig_dev, (int *)(ext + 2 * na + 1),
+                            c->stream)))
+    return rc;
+  std::vector<char> back(b_x);
+  EXC_CHECK(hipMemcpyAsync(back.data(), ext, b_x, hipMemcpyDeviceToHost, c->stream));
   EXC_CHECK(hipStreamSynchronize(c->stream));
-  bool ok = solved;
-  double lmin = 0.0, lmax = 0.0;
-  for (int a = 0; a < na; ++a) ok = ok && hi[a] == 0;
-  for (double v : hl) {
-    ok = ok && std::isfinite(v);
-    lmin = std::min(lmin, v);
-    lmax = std::max(lmax, fabs(v));
+  const double *x = (const double *)back.data();
+  const int *info = (const int *)(x + 2 * na + 1);
+  bool ok = std::isfinite(x[2 * na]);
+  double lmax = 0.0;
+  for (int a = 0; a < na; ++a) {
+    ok = ok && info[a] == 0;
+    lmax = std::max(lmax, std::max(fabs(x[2 * a]), fabs(x[2 * a + 1])));
   }
-  c->gram_sigma = ok ? (lmin < 0.0 ? -lmin * (1.0 + 1e-6) : 0.0) + 1e-10 * lmax : HUGE_VAL;
+  c->gram_sigma = ok ? x[2 * na] : HUGE_VAL;
   c->gram_lmax = lmax;
-  c->gram_tri = false;
-  if (ok) {
-    if ((rc = exc_launch_crt_gram_perm(c->d, c->gram_sigma, Mp, c->stream))) return rc;
-    bool tri = rocsolver_zpotrf_strided_batched(c->gram_blas, rocblas_fill_lower, n, (rocblas_double_complex *)Mp, n,
-                                                (rocblas_stride)n * n, info, na) == rocblas_status_success;
-    if (tri) {
-      EXC_CHECK(hipMemcpyAsync(hi.data(), info, 4 * (size_t)na, hipMemcpyDeviceToHost, c->stream));
-      EXC_CHECK(hipStreamSynchronize(c->stream));
-      for (int a = 0; a < na; ++a) tri = tri && hi[a] == 0;
-    }
-    rc = tri ? exc_launch_crt_gram_tri(c->d, Mp, T, c->stream)
-             : exc_launch_crt_gram_table(c->d, U, lam, c->gram_sigma, T, c->stream);
-    if (rc) return rc;
-    c->gram_tri = tri;
-    EXC_CHECK(hipMemcpyAsync(dsig, &c->gram_sigma, 8, hipMemcpyHostToDevice, c->stream));
-    EXC_CHECK(hipStreamSynchronize(c->stream));
-  }
   c->gram_valid = true;
   return EXC_OK;
 }
@@ -936,9 +902,8 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   // the Gram form's E stage on its triangular table: narrow column tiles skip more of it
   // (64 x 64 three-product tiles, 5.7 against 6.7 ms at workload 3; the dense Y stage keeps
   // 64 x 128, 8.8 against 9.1 ms)
-  const bool etri = gram && c->gram_tri;
-  const int ye = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, etri ? 4 : 0);
-  int tail[10] = {nk, flags, bv, yv, crt ? cv : -1, (crt ? nmod : -1) + 100 * ov, fv, gram, etri, ye};
+  const int ye = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, 4);
+  int tail[9] = {nk, flags, bv, yv, crt ? cv : -1, (crt ? nmod : -1) + 100 * ov, fv, gram, ye};
   std::vector<char> sig(sizeof(exc_kpoint_dev) * nk + sizeof(tail));
   memcpy(sig.data(), ks, sizeof(exc_kpoint_dev) * nk);
   memcpy(sig.data() + sizeof(exc_kpoint_dev) * nk, tail, sizeof(tail));
@@ -1165,12 +1130,12 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
       if (hipEventRecord(c->ev_join, c->side) != hipSuccess) return EXC_ERR_HIP;
     }
     {
-      // the Gram form's E = A conj(U) (Lambda + sigma)^(1/2) is the Y stage on its table
+      // the Gram form's E = A conj(L) is the Y stage on its table
       StageTimer t(c, capture ? -1 : EXC_STAGE_YSTAGE);
       exc_dev dy = c->d;
       if (gram) {
         dy.haa = (cplx *)gram_t;
-        dy.ytri = etri ? 1 : 0;
+        dy.ytri = 1;
       }
       if ((r = exc_launch_bystage(dy, nk, c->batch_maxngp, c->d_ks, gram ? ye : yv, c->stream))) return r;
     }

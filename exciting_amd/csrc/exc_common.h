@@ -179,10 +179,8 @@ int exc_launch_crt_gemm(const exc_dev &d, const kdesc *ks, const mt_item *items,
                         const CrtTab &t, signed char *res, int variant, hipStream_t s);
 int exc_launch_crt_merge(const exc_dev &d, const kdesc *ks, const mt_item *items, int nitems, const CrtTab &t,
                          const signed char *res, int variant, const double *gsig, hipStream_t s);
-int exc_launch_crt_gram_table(const exc_dev &d, const cplx *U, const double *lam, double sigma, cplx *T,
-                              hipStream_t s);
-int exc_launch_crt_gram_perm(const exc_dev &d, double sigma, cplx *Mp, hipStream_t s);
-int exc_launch_crt_gram_tri(const exc_dev &d, const cplx *L, cplx *T, hipStream_t s);
+// the Gram form's table (k_gram.hip)
+int exc_launch_gram(const exc_dev &d, cplx *scratch, cplx *T, double *ext, double *sig, int *info, hipStream_t s);
 // generalized eigensolve helpers (k_eigen.hip)
 struct eig_kdesc {   // one k-point of a grouped solve: nmat n, device arrays
   const cplx *h, *o;

@@ -86,18 +86,16 @@ struct exc_ctx {
   void *gk_buf;               // G+k sets: k-point coordinates, counts, and the host entries' staging
   size_t gk_buf_bytes;
   double cfdamp_t1;           // gencfun's damping exponent cfdamp / gmaxvr (0: none)
-  // Gram form of the modular split: the table conj(U) (Lambda + sigma)^(1/2) per atom, the
-  // eigenvectors and values of h_a, sigma (host and device); valid until h_a changes
+  // Gram form of the modular split: the table conj(L) per atom (L L^H = h_a + sigma), sigma (host
+  // and device); valid until h_a changes
   int crt_form;               // -1 built-in (Gram where it applies), 0 A and Yt, 1 Gram
   int crt_last_form, crt_last_nmod;   // what the last modular-split setup used
   void *gram_buf;
   size_t gram_bytes;
-  rocblas_handle gram_blas;   // its own handle: the eigensolve workers pin their workspaces
-  cplx *gram_table;           // in gram_buf: the Y stage's table conj(U) (Lambda + sigma)^(1/2)
+  cplx *gram_table;           // in gram_buf: the Y stage's table
   double *gram_sig_dev;       // in gram_buf: sigma for the merge
   bool gram_valid;
-  double gram_sigma, gram_lmax;
-  bool gram_tri;              // the table is the triangular (Cholesky) one
+  double gram_sigma, gram_lmax;   // sigma infinite: no table (h_a not finite, or its factorization failed)
   signed char *crt_res;
   size_t crt_res_bytes;
   mt_item *d_citems;

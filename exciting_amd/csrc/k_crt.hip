@@ -28,9 +28,9 @@
 // same bits; the only rounding between the inputs and H_MT is that of the operands to
 // beta-bit integers and the final conversion.
 //
-// Gram form (the default where it applies): with h_a = U_a Lambda_a U_a^H and a shift
-// sigma >= -min lambda, E_a = A_a conj(U_a) (Lambda_a + sigma)^(1/2) (the Y stage on that
-// table instead of h_a) gives conj(E) E^T = conj(A) (h + sigma) A^T = H_MT + sigma O_APW, so
+// Gram form (the default where it applies): with a shift sigma >= -min lambda(h_a) and h_a +
+// sigma = L_a L_a^H, E_a = A_a conj(L_a) (the Y stage on that table instead of h_a, k_gram.hip)
+// gives conj(E) E^T = conj(A) (h + sigma) A^T = H_MT + sigma O_APW, so
 // H_MT = conj(E) E^T - sigma O_APW with O_APW the FP64 addition-theorem overlap (O minus
 // its interstitial term).  One operand is split instead of two, and the right operand's
 // planes are the left's swapped, as for O = conj(A) A^T; merge items of this form carry
@@ -841,71 +841,4 @@ int exc_launch_crt_merge(const exc_dev &d, const kdesc *ks, const mt_item *items
     case 12: return launch_merge_t<12>(d, ks, items, nitems, t, res, bt, wr, wc, gsig, s);
     default: return EXC_ERR_ARG;
   }
-}
-
-namespace {
-// T_a(r, f) = conj(U_a(f, r)) sqrt(lambda_r + sigma), column-major per atom: the table the Y
-// stage reads in h_a's place (it forms A_a T_a^T = A_a conj(U_a) (Lambda_a + sigma)^(1/2))
-__global__ __launch_bounds__(256) void crt_gram_table_kernel(int naa, const cplx *__restrict__ U,
-                                                             const double *__restrict__ lam, double sigma,
-                                                             cplx *__restrict__ T) {
-  const int r = blockIdx.x * 256 + threadIdx.x, f = blockIdx.y, a = blockIdx.z;
-  if (r >= naa) return;
-  const size_t o = (size_t)a * naa * naa;
-  const cplx u = U[o + f + (size_t)naa * r];
-  const double w = sqrt(fmax(lam[(size_t)a * naa + r] + sigma, 0.0));
-  T[o + r + (size_t)naa * f] = cplx{u.re * w, -u.im * w};
-}
-}  // namespace
-
-int exc_launch_crt_gram_table(const exc_dev &d, const cplx *U, const double *lam, double sigma, cplx *T,
-                              hipStream_t s) {
-  hipLaunchKernelGGL(crt_gram_table_kernel, dim3((d.naa + 255) / 256, d.naa, d.natm), dim3(256), 0, s, d.naa, U, lam,
-                     sigma, T);
-  EXC_CHECK(hipGetLastError());
-  return EXC_OK;
-}
-
-namespace {
-// M_p = P (h + sigma I) P^T per atom: h's rows and columns in the Y stage's summation order
-__global__ __launch_bounds__(256) void crt_gram_perm_kernel(int naa, const cplx *__restrict__ h,
-                                                            const int *__restrict__ fperm, double sigma,
-                                                            cplx *__restrict__ Mp) {
-  const int a = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y, at = blockIdx.z;
-  if (a >= naa) return;
-  const size_t o = (size_t)at * naa * naa;
-  cplx v = h[o + fperm[a] + (size_t)naa * fperm[b]];
-  if (a == b) v.re += sigma;
-  Mp[o + a + (size_t)naa * b] = v;
-}
-
-// T(r, fperm[kk]) = conj(L(kk, r)) for kk >= r and 0 above, L the lower Cholesky factor of M_p:
-// the Y stage on T forms E = A_p conj(L), conj(E) E^T = conj(A) (h + sigma) A^T, and the sum of
-// a column tile starting at r0 may start at position r0 of the order
-__global__ __launch_bounds__(256) void crt_gram_tri_kernel(int naa, const cplx *__restrict__ L,
-                                                           const int *__restrict__ fperm, cplx *__restrict__ T) {
-  const int r = blockIdx.x * 256 + threadIdx.x, kk = blockIdx.y, at = blockIdx.z;
-  if (r >= naa) return;
-  const size_t o = (size_t)at * naa * naa;
-  cplx v = {0.0, 0.0};
-  if (kk >= r) {
-    const cplx l = L[o + kk + (size_t)naa * r];
-    v = cplx{l.re, -l.im};
-  }
-  T[o + r + (size_t)naa * fperm[kk]] = v;
-}
-}  // namespace
-
-int exc_launch_crt_gram_perm(const exc_dev &d, double sigma, cplx *Mp, hipStream_t s) {
-  hipLaunchKernelGGL(crt_gram_perm_kernel, dim3((d.naa + 255) / 256, d.naa, d.natm), dim3(256), 0, s, d.naa, d.haa,
-                     d.fperm, sigma, Mp);
-  EXC_CHECK(hipGetLastError());
-  return EXC_OK;
-}
-
-int exc_launch_crt_gram_tri(const exc_dev &d, const cplx *L, cplx *T, hipStream_t s) {
-  hipLaunchKernelGGL(crt_gram_tri_kernel, dim3((d.naa + 255) / 256, d.naa, d.natm), dim3(256), 0, s, d.naa, L, d.fperm,
-                     T);
-  EXC_CHECK(hipGetLastError());
-  return EXC_OK;
 }

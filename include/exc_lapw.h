@@ -233,7 +233,8 @@ typedef struct exc_kpoint_dev {
                                 /* rounded once to FP64; n from exc_ctx_set_moduli.  Y stage,      */
                                 /* interstitial, lo blocks stay FP64.  With                        */
                                 /* EXC_BATCH_OLP_LEGENDRE (and no 'iora*' h1aa) the Gram form:     */
-                                /* E = A conj(U) (Lambda + sigma)^(1/2) from h_a = U Lambda U^H,   */
+                                /* E = A conj(L) with L L^H = h_a + sigma (sigma from h_a's least  */
+                                /* eigenvalue),                                                    */
                                 /* H_MT = conj(E) E^T - sigma O_APW, one operand to split          */
 #define EXC_BATCH_OLP_LEGENDRE 8 /* needs EXC_BATCH_MATCH: the muffin-tin part of O from the      */
                                  /* radial factors of match by the spherical-harmonic addition   */
