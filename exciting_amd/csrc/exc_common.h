@@ -159,16 +159,19 @@ int exc_launch_olp(const exc_dev &d, int nk, int maxngp, const kdesc *ks, const 
 int exc_launch_bsplit(const exc_dev &d, const kdesc *ks, const mt_item *items, int nitems, int variant, int nblocks,
                       hipStream_t s);
 // modular split of the muffin-tin contraction (k_crt.hip)
-constexpr int kMaxMod = 14;          // moduli available: 241, 233, 229, 221, 205, 197, 193, ...
-constexpr int kCrtLoDigits = 6;      // mixed-radix digits of the low part (their product < 2^53)
-constexpr int kCrtMaxUsed = 12;      // beyond 12 moduli beta > 44: re -+ iota im of the row
-                                     // integers no longer exact in FP64
+constexpr int kMaxMod = 16;          // moduli available: 241, 233, 229, 221, 205, 197, 193, ...
+constexpr int kCrtLoDigits = 6;      // mixed-radix digits of one FP64 part (their product < 2^53)
+constexpr int kCrtMaxUsed = 12;      // moduli a caller may ask for (exc_ctx_set_moduli)
+constexpr int kExactMod = 16;        // moduli of the FP64 path's exact products (beta 57)
 constexpr int kCrtVariants = 11;     // tile / staging variants of the residue GEMM
 struct CrtTab {                      // passed by value to the kernels (kernel-argument segment)
   int n, beta;
   int m[kMaxMod];                    // odd, pairwise coprime, every prime factor 1 mod 4
   int iota[kMaxMod];                 // a square root of -1 modulo m
   double dminv[kMaxMod];
+  float finv[kMaxMod];               // 1 / m
+  // symmetric residues of 2^0, 2^16 | 2^32, 2^48 modulo m, two int16 a word, and of iota times them
+  int wr[kMaxMod][2], wi[kMaxMod][2];
 };
 void exc_crt_tables(int n, CrtTab *t);
 inline int exc_crt_kpad(int ktot) { return (ktot + 63) / 64 * 64; }

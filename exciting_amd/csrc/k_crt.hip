@@ -58,20 +58,27 @@ __device__ __forceinline__ int dres(double x, int m, double minv) { return (int)
 // ---------------------------------------------------------------------------------------
 // scale: the per-row exponents s = beta - e, |X_i| < 2^e, of Yt, and of A when the caller
 // supplies apwalm (with the grouped match, crt_expo_kernel sums A's from the norms the match
-// wrote): one workgroup per (k, 64 rows); wave w sums |x|^2 over its quarter of K, the
-// quarters added in wave order (a fixed order: the exponents do not depend on timing)
+// wrote): one workgroup per (k, 64 rows); each of its 16 waves sums |x|^2 over a part of K, the
+// parts added in wave order (a fixed order: the exponents do not depend on timing).  Bound by
+// reading X; 16 waves since a batch of small k-points has few row blocks (N = 1200, 8
+// k-points: 152 workgroups; 241 us with 4 waves, 86 us with 16; N = 5000, 32 atoms, 8 k-points
+// 1.13 -> 0.87 ms, 5.7 TB/s).
 // ---------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void crt_scale_kernel(const kdesc *__restrict__ ks, int ktot, int beta, int op) {
+constexpr int kScaleWaves = 16;
+
+__global__ __launch_bounds__(64 * kScaleWaves) void crt_scale_kernel(const kdesc *__restrict__ ks, int ktot, int beta,
+                                                                     int op) {
   const kdesc k = ks[blockIdx.z];             // op 0: A (apwalm), 1: Yt, 2: E (in Yt's place) as the left operand
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row = blockIdx.x * 64 + lane;
-  __shared__ double part[4][64];
+  __shared__ double part[kScaleWaves][64];
   if (blockIdx.x * 64 >= k.cnp) return;       // uniform over the workgroup
   const cplx *src = op ? k.yt : k.apwalm;
   const int ld = op ? k.ldy : k.ldg;
-  const int kq = (ktot + 3) / 4, k0 = wave * kq, k1 = min(ktot, k0 + kq);   // op 2 writes xa
+  const int kq = (ktot + kScaleWaves - 1) / kScaleWaves, k0 = wave * kq, k1 = min(ktot, k0 + kq);   // op 2 writes xa
   double acc = 0.0;
   if (row < k.ngp) {
+#pragma unroll 8
     for (int c = k0; c < k1; ++c) {
       const cplx v = src[row + (size_t)c * ld];
       acc = fma(v.re, v.re, acc);
@@ -81,7 +88,9 @@ __global__ __launch_bounds__(256) void crt_scale_kernel(const kdesc *__restrict_
   part[wave][lane] = acc;
   __syncthreads();
   if (wave == 0) {
-    const double s2 = ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+    double s2 = 0.0;
+#pragma unroll
+    for (int w = 0; w < kScaleWaves; ++w) s2 += part[w][lane];
     int e = 0;
     if (s2 > 0.0) frexp(sqrt(s2), &e);       // |X_i| < 2^e
     (op == 1 ? k.xy : k.xa)[row] = row < k.ngp ? beta - e : 0;
@@ -112,28 +121,53 @@ __device__ __forceinline__ unsigned pack4(int a, int b, int c, int d) {
          __builtin_amdgcn_perm((unsigned)d, (unsigned)c, 0x04000c0cu);
 }
 
-// The two residue planes of one modulus for 16 values of k of one row: the maps
-// Re X' + sg iota Im X' and Re X' - sg iota Im X' (sg = -1 for the conjugated left operand A,
-// +1 for the right operand Yt), formed exactly in FP64 from Re X' and the residue of Im X'
-// (|Re X'| + iota (m-1)/2 < 2^45: the quotient by m is then far more accurate than the
-// 1/(2m) margin of its rounding) and reduced to their symmetric residues.
+// the four balanced 16-bit limbs of an integer |x| < 2^58 held in a double, two a word, from the
+// lowest up: each in [-2^15, 2^15), the carries exact (x / 2^16 + 1/2 rounds only where its
+// sum leaves x / 2^16's binade, and then not past an integer)
+__device__ __forceinline__ void limbs(double x, int (&w)[2]) {
+  const double h1 = floor(fma(x, 0x1p-16, 0.5)), l0 = fma(-h1, 0x1p16, x);
+  const double h2 = floor(fma(h1, 0x1p-16, 0.5)), l1 = fma(-h2, 0x1p16, h1);
+  const double h3 = floor(fma(h2, 0x1p-16, 0.5)), l2 = fma(-h3, 0x1p16, h2);
+  w[0] = __builtin_amdgcn_perm((unsigned)(int)l1, (unsigned)(int)l0, 0x05040100u);
+  w[1] = __builtin_amdgcn_perm((unsigned)(int)h3, (unsigned)(int)l2, 0x05040100u);
+}
+
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ int dot2(int a, int b, int c) {
+  return __builtin_amdgcn_sdot2(__builtin_bit_cast(s16x2, a), __builtin_bit_cast(s16x2, b), c, false);
+}
+
+// a residue of |t| < 2^25 modulo m in the low byte (the upper ones are not part of it): t - q m
+// with q = rint(t / m) in the low bits of the float 1.5 2^23 + q, whose other bits are a multiple
+// of 2^22 and drop out modulo 256.  |t - q m| <= m / 2 + 2: the float quotient is within 1/64 of
+// t / m
+__device__ __forceinline__ int lowres(int t, int m, float finv) {
+  return t - __mul24(__float_as_int(fmaf((float)t, finv, 12582912.0f)), m);
+}
+
+// The residue planes of every modulus for 16 values of k of one row: the maps Re X' + sg iota
+// Im X' and Re X' - sg iota Im X' (sg = -1 for the conjugated left operand A, +1 for the right
+// operand Yt).  Modulo m the parts are sums of four limbs times the residues of 2^0 .. 2^48 (for
+// Im X' times iota): |sum| < 4 2^15 120 < 2^24, two v_dot2_i32_i16 each, exact, and their sum and
+// difference are reduced once: 14 32-bit operations per complex value and modulus, where reducing
+// the integers in FP64 took 11 FP64 ones and 2 conversions.
 template <int SG>
-__device__ __forceinline__ void split_planes(const double (&xr)[16], const double (&xi)[16], const CrtTab &t,
+__device__ __forceinline__ void split_planes(const int (&xr)[16][2], const int (&xi)[16][2], const CrtTab &t,
                                              signed char *base, size_t pstride, size_t off) {
 #pragma unroll 1
   for (int l = 0; l < t.n; ++l) {
-    const int m = t.m[l];
-    const double mi = t.dminv[l], io = (double)(SG * t.iota[l]);
+    const int m = t.m[l], a0 = t.wr[l][0], a1 = t.wr[l][1], b0 = t.wi[l][0], b1 = t.wi[l][1];
+    const float fi = t.finv[l];
     unsigned w[2][4];
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       int ru[4], rv[4];
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        const double a = xr[4 * g + b], c = xi[4 * g + b];
-        const double ci = fma(-(double)m, rint(c * mi), c);     // Im X' mod m, exact
-        ru[b] = dres(fma(io, ci, a), m, mi);
-        rv[b] = dres(fma(-io, ci, a), m, mi);
+        const int p = dot2(xr[4 * g + b][0], a0, dot2(xr[4 * g + b][1], a1, 0));
+        const int q = dot2(xi[4 * g + b][0], b0, dot2(xi[4 * g + b][1], b1, 0));
+        ru[b] = lowres(SG > 0 ? p + q : p - q, m, fi);
+        rv[b] = lowres(SG > 0 ? p - q : p + q, m, fi);
       }
       w[0][g] = pack4(ru[0], ru[1], ru[2], ru[3]);
       w[1][g] = pack4(rv[0], rv[1], rv[2], rv[3]);
@@ -156,14 +190,14 @@ __global__ __launch_bounds__(256) void crt_split_kernel(const kdesc *__restrict_
   const cplx *src = (op || gram) ? k.yt : k.apwalm;
   const int ld = (op || gram) ? k.ldy : k.ldg;
   const int s = row < k.ngp ? (op ? k.xy : k.xa)[row] : 0;
-  double xr[16], xi[16];
+  int xr[16][2], xi[16][2];
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     const int c = kc * 16 + q;
     cplx v = {0.0, 0.0};
     if (row < k.ngp && c < ktot) v = src[row + (size_t)c * ld];
-    xr[q] = rint(ldexp(v.re, s));
-    xi[q] = rint(ldexp(v.im, s));
+    limbs(rint(ldexp(v.re, s)), xr[q]);
+    limbs(rint(ldexp(v.im, s)), xi[q]);
   }
   signed char *base = (signed char *)(op ? k.qy : k.qa);
   const size_t pstride = (size_t)kp * k.cnp;            // bytes of one plane
@@ -494,15 +528,18 @@ __global__ __launch_bounds__(64 * WR * WC, 1) void crt_gemm_pipe_kernel(const kd
 }
 
 // ---------------------------------------------------------------------------------------
-// merge: one tile per workgroup (4 waves).  Wave w takes the 32 x 32 blocks w, w + 4, ...
-// of the gemm layout (wave-major as the gemm wrote them, decoded with that variant's wave
-// grid), one lane per gemm lane with its 16 values.
+// merge: one 32 x 32 block of the gemm layout per wave (wave-major as the gemm wrote them, decoded
+// with that variant's wave grid), one lane per gemm lane with its 16 values.  Waves share
+// nothing: the rows' data sit in the wave's own LDS slice, the column's in registers, so there
+// is no barrier and a small batch still fills the chip (with a tile per workgroup and its blocks
+// in turn: 104 us for 5 atoms, N = 260, 8 k-points, 36 here; N = 5000, 32 atoms, 8 k: 2.56 ms, 2.29
+// here).  Bound by Garner's 32-bit arithmetic and by reading the residues and O and writing H.
 // ---------------------------------------------------------------------------------------
 // The moduli and Garner's tables are fixed at compile time for each modulus count (the
 // moduli list is constant; only how many of them is chosen), so every reduction below
 // multiplies by immediates.  Moduli: odd, pairwise coprime, every prime factor 1 mod 4
 // (221 = 13 17, 205 = 5 41), the largest first.
-constexpr int kModList[kMaxMod] = {241, 233, 229, 221, 205, 197, 193, 181, 173, 157, 149, 137, 113, 109};
+constexpr int kModList[kMaxMod] = {241, 233, 229, 221, 205, 197, 193, 181, 173, 157, 149, 137, 113, 109, 101, 97};
 
 constexpr int inv_mod(int a, int m) {   // a^-1 mod m, gcd(a, m) = 1 (extended Euclid)
   int r0 = m, r1 = ((a % m) + m) % m, t0 = 0, t1 = 1;
@@ -528,7 +565,8 @@ struct GarnerTab {
   int w[NM][NM];
   int cre[NM], cim[NM];
   double mk;        // M_6 (or P for fewer moduli): x = x_hi M_6 + x_lo
-  constexpr GarnerTab() : w(), cre(), cim(), mk(1.0) {
+  double mh, ml;    // M_12 = mh + ml
+  constexpr GarnerTab() : w(), cre(), cim(), mk(1.0), mh(0.0), ml(0.0) {
     for (int l = 0; l < NM; ++l) {
       const int m = kModList[l];
       long long ml = 1;
@@ -543,6 +581,12 @@ struct GarnerTab {
       cim[l] = inv_mod(2 * iota_of(m) % m, m) * v % m;
     }
     for (int j = 0; j < (NM < kCrtLoDigits ? NM : kCrtLoDigits); ++j) mk *= kModList[j];
+    if (NM > 2 * kCrtLoDigits) {
+      __int128 m12 = 1;
+      for (int j = 0; j < 2 * kCrtLoDigits; ++j) m12 *= kModList[j];
+      mh = (double)m12;
+      ml = (double)(m12 - (__int128)mh);
+    }
   }
 };
 
@@ -555,7 +599,7 @@ __device__ __forceinline__ int cres(int x) {
   return x - __mul24((int)rintf((float)x * finv), m);
 }
 
-// |s_l c_l| <= 240 240 and |d_j w| <= 120 240: the sum stays below 2^22 for up to 12 moduli
+// |s_l c_l| <= 240 240 and |d_j w| <= 120 240: the sum stays below 2^22 for up to 16 moduli
 template <int NM, int L, bool IM>
 __device__ __forceinline__ void garner_digit(int (&d)[NM], const int (&s)[NM]) {
   constexpr GarnerTab<NM> G{};
@@ -574,154 +618,183 @@ __device__ __forceinline__ double garner(const int (&s)[NM]) {
   constexpr GarnerTab<NM> G{};
   int d[NM];
   garner_digit<NM, 0, IM>(d, s);
-  constexpr int NLO = NM < kCrtLoDigits ? NM : kCrtLoDigits;
+  constexpr int NLO = NM < kCrtLoDigits ? NM : kCrtLoDigits, NMID = NM < 2 * kCrtLoDigits ? NM : 2 * kCrtLoDigits;
   double lo = (double)d[NLO - 1];
 #pragma unroll
   for (int j = NLO - 2; j >= 0; --j) lo = fma(lo, (double)kModList[j], (double)d[j]);
-  double hi = 0.0;
+  double mid = 0.0;
 #pragma unroll
-  for (int j = NM - 1; j >= NLO; --j) hi = fma(hi, (double)kModList[j], (double)d[j]);
-  return fma(hi, G.mk, lo);
+  for (int j = NMID - 1; j >= NLO; --j) mid = fma(mid, (double)kModList[j], (double)d[j]);
+  const double x = fma(mid, G.mk, lo);
+  if constexpr (NM <= NMID) {
+    return x;
+  } else {
+    // beyond 12 moduli a third part x_hi M_12, M_12 = mh + ml to 106 bits: |x| <= M_12 / 2, so the
+    // sum is within two roundings of the exact value
+    double hi = 0.0;
+#pragma unroll
+    for (int j = NM - 1; j >= NMID; --j) hi = fma(hi, (double)kModList[j], (double)d[j]);
+    return fma(hi, G.mh, fma(hi, G.ml, x));
+  }
 }
 
 template <int NM>
 __global__ __launch_bounds__(256) void crt_merge_kernel(const kdesc *__restrict__ ks, const mt_item *__restrict__ items,
-                                                        const signed char *__restrict__ res, int bt, int wr_n, int wc_n,
-                                                        GTab gt, const double *__restrict__ gsig) {
-  const mt_item it = items[blockIdx.x];
+                                                        int nitems, const signed char *__restrict__ res, int bt,
+                                                        int wr_n, int wc_n, GTab gt, const double *__restrict__ gsig) {
+  struct Slice {
+    // Element (row, col) of a block sits in lane (col mod 32) of the gemm layout, so the
+    // conjugate store at (col, row) is coalesced along the lanes; the store at (row, col) goes
+    // through LDS, 16 rows of the block at a time: stored [col][row] with one pad element per
+    // column, read back with 16 lanes along a column (256 contiguous bytes)
+    cplx t[32 * 17];
+    double v[32][3];
+    int g[32][3], ex[32];
+  };
+  __shared__ Slice sl[4];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Slice &sw = sl[wave];
+  const int bpt = (bt / 32) * (bt / 32);                    // blocks of a tile: a multiple of 4
+  const int item = blockIdx.x / (bpt / 4), blk = blockIdx.x % (bpt / 4) * 4 + wave;
+  const mt_item it = items[item];
   const kdesc k = ks[it.k];
   const int ngp = k.ngp;
-  const int row0 = it.ti * bt, col0 = it.tj * bt;
-  __shared__ int gr[kMaxTile][3], gc[kMaxTile][3];
-  __shared__ double vr[kMaxTile][3], vc[kMaxTile][3];
-  __shared__ int er[kMaxTile], ec[kMaxTile];
-  for (int e = threadIdx.x; e < 2 * bt; e += 256) {
-    const bool isr = e < bt;
-    const int q = isr ? e : e - bt;
-    const int idx = (isr ? row0 : col0) + q;
-    int g0 = 0, g1 = 0, g2 = 0, ex = 0;
-    double v0 = 0.0, v1 = 0.0, v2 = 0.0;
-    if (idx < ngp) {
-      const int ig = k.igpig[idx] - 1;
-      g0 = gt.ivg[3 * ig]; g1 = gt.ivg[3 * ig + 1]; g2 = gt.ivg[3 * ig + 2];
-      v0 = k.vgpc[3 * idx]; v1 = k.vgpc[3 * idx + 1]; v2 = k.vgpc[3 * idx + 2];
-      ex = isr ? k.xa[idx] : (it.which ? k.xa[idx] : k.xy[idx]);
-    }
-    int(&g)[kMaxTile][3] = isr ? gr : gc;
-    double(&vv)[kMaxTile][3] = isr ? vr : vc;
-    g[q][0] = g0; g[q][1] = g1; g[q][2] = g2;
-    vv[q][0] = v0; vv[q][1] = v1; vv[q][2] = v2;
-    (isr ? er : ec)[q] = ex;
-  }
-  __syncthreads();
   const int mi_n = bt / wr_n / 32, nj_n = bt / wc_n / 32, per_wave = mi_n * nj_n;
-  const int nblk = (bt / 32) * (bt / 32);
+  const int wv = blk / per_wave, bi = (blk % per_wave) / nj_n, bj = blk % nj_n;
+  const int row0 = it.ti * bt + (wv / wc_n) * (32 * mi_n) + 32 * bi;     // the block's origin
+  const int col0 = it.tj * bt + (wv % wc_n) * (32 * nj_n) + 32 * bj;
+  if (row0 > col0 + 31 || col0 >= ngp) return;              // below the diagonal or past the basis (uniform)
   const size_t ptile = (size_t)bt * bt;                     // residue bytes of one (modulus, product)
-  const signed char *base = res + (size_t)blockIdx.x * NM * 2 * ptile;
+  const signed char *base = res + (size_t)item * NM * 2 * ptile + ((size_t)blk * 64 + lane) * 16;
   cplx *out = it.which == 1 ? k.o : k.h;
   const double sig = it.which == 2 ? *gsig : 0.0;           // Gram form: H_MT = conj(E) E^T - sigma O_APW
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  // Element (row, col) of a 32 x 32 block sits in lane (col mod 32) of the gemm layout, so the
-  // conjugate store at (col, row) is coalesced along the lanes; the store at (row, col) goes
-  // through this wave's LDS slice, 16 rows of the block at a time: stored [col][row] with one
-  // pad element per column, read back with 16 lanes along a column (256 contiguous bytes)
-  __shared__ cplx tb[4][32 * 17];
-  cplx *tw = tb[wave];
-  for (int b4 = 0; b4 < nblk; b4 += 4) {                    // the same trip count in every wave
-    const int blk = b4 + wave;
-    const int wv = blk / per_wave, bi = (blk % per_wave) / nj_n, bj = blk % nj_n;
-    const int wr = wv / wc_n, wc = wv % wc_n;
-    const int rb = wr * (32 * mi_n) + 32 * bi, cb = wc * (32 * nj_n) + 32 * bj;   // block origin in the tile
-    const int cl = cb + (lane & 31);
-    const int col = col0 + cl;
-    uint4 q1[NM], q2[NM];
+  if (lane < 32) {
+    const int idx = row0 + lane;
+    int ig = 0, ex = 0;
+    if (idx < ngp) {
+      ig = k.igpig[idx] - 1;
+      ex = k.xa[idx];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) sw.v[lane][q] = k.vgpc[3 * idx + q];
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) sw.g[lane][q] = gt.ivg[3 * ig + q];
+    sw.ex[lane] = ex;
+  }
+  const int col = col0 + (lane & 31);
+  int gc[3] = {0, 0, 0}, exc = 0;
+  double vc[3] = {0.0, 0.0, 0.0};
+  if (col < ngp) {
+    const int ig = k.igpig[col] - 1;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      gc[q] = gt.ivg[3 * ig + q];
+      vc[q] = k.vgpc[3 * col + q];
+    }
+    exc = it.which ? k.xa[col] : k.xy[col];
+  }
+  auto fence = [] {                                         // orders this wave's LDS stores and loads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  constexpr bool kWhole = NM <= 12;                         // more moduli: half a block's residues at a time (registers)
+  uint4 q1[kWhole ? NM : 1], q2[kWhole ? NM : 1];
+  if constexpr (kWhole) {
 #pragma unroll
     for (int l = 0; l < NM; ++l) {
-      const signed char *b = base + (size_t)l * 2 * ptile + ((size_t)blk * 64 + lane) * 16;
-      q1[l] = *(const uint4 *)b;
-      q2[l] = *(const uint4 *)(b + ptile);
+      q1[l] = *(const uint4 *)(base + (size_t)l * 2 * ptile);
+      q2[l] = *(const uint4 *)(base + (size_t)l * 2 * ptile + ptile);
     }
+  }
+  fence();
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      // Gram form: this half's eight O elements, loaded together ahead of the reconstruction;
-      // read at (col, row), O's conjugate mirror (bit for bit), where the lanes are contiguous
-      cplx om[8];
-      if (it.which == 2) {
+  for (int h = 0; h < 2; ++h) {
+    uint2 p1[NM], p2[NM];
 #pragma unroll
-        for (int vv = 0; vv < 8; ++vv) {
-          const int v = 8 * h + vv;
-          const int row = row0 + rb + 16 * h + 8 * (vv >> 2) + 4 * (lane >> 5) + (v & 3);
-          om[vv] = (col < ngp && row <= col) ? k.o[col + (size_t)row * k.ldh] : cplx{0.0, 0.0};
-        }
+    for (int l = 0; l < NM; ++l) {
+      if constexpr (kWhole) {
+        p1[l] = h ? make_uint2(q1[l].z, q1[l].w) : make_uint2(q1[l].x, q1[l].y);
+        p2[l] = h ? make_uint2(q2[l].z, q2[l].w) : make_uint2(q2[l].x, q2[l].y);
+      } else {
+        p1[l] = *(const uint2 *)(base + (size_t)l * 2 * ptile + 8 * h);
+        p2[l] = *(const uint2 *)(base + (size_t)l * 2 * ptile + ptile + 8 * h);
       }
+    }
+    // Gram form: this half's eight O elements, loaded together ahead of the reconstruction;
+    // read at (col, row), O's conjugate mirror (bit for bit), where the lanes are contiguous
+    cplx om[8];
+    if (it.which == 2) {
 #pragma unroll
       for (int vv = 0; vv < 8; ++vv) {
-        const int v = 8 * h + vv;
-        const int rh = 8 * (vv >> 2) + 4 * (lane >> 5) + (v & 3);   // row within the half
-        const int rl = rb + 16 * h + rh;
-        const int row = row0 + rl;
-        cplx val = {0.0, 0.0};
-        if (col < ngp && row <= col) {
-          // conj(a) b: Re = (U + V)/2, Im = (U - V)/(2 iota) modulo each m
-          const int g = v >> 2, sh = 8 * (v & 3);
-          int sr[NM], si[NM];
-#pragma unroll
-          for (int l = 0; l < NM; ++l) {
-            const unsigned w1 = g == 0 ? q1[l].x : g == 1 ? q1[l].y : g == 2 ? q1[l].z : q1[l].w;
-            const unsigned w2 = g == 0 ? q2[l].x : g == 1 ? q2[l].y : g == 2 ? q2[l].z : q2[l].w;
-            const int u = (signed char)(w1 >> sh), vv = (signed char)(w2 >> sh);
-            sr[l] = u + vv;
-            si[l] = u - vv;
-          }
-          const int sc = -(er[rl] + ec[cl]);
-          double re = ldexp(garner<NM, false>(sr), sc);
-          double im = ldexp(garner<NM, true>(si), sc);
-          const int ig = lookup_g(gt, gr[rl][0] - gc[cl][0], gr[rl][1] - gc[cl][1], gr[rl][2] - gc[cl][2]);
-          if (it.which == 2) {
-            // O_APW = O - its interstitial term, O as the overlap kernel wrote it
-            cplx oa = {om[vv].re, -om[vv].im};
-            if (ig) {
-              const cplx tho = setup_dev::olp_theta(gt, ig, vr[rl], vc[cl]);
-              oa = cplx{oa.re - tho.re, oa.im - tho.im};
-            }
-            re = fma(-sig, oa.re, re);
-            im = fma(-sig, oa.im, im);
-          }
-          if (ig) {
-            const cplx th = gt.cfunig[ig - 1];
-            if (it.which == 1) {
-              re += th.re;
-              im += th.im;
-            } else {
-              const cplx vv2 = gt.veffig[ig - 1];
-              const double t1 = 0.5 * (vr[rl][0] * vc[cl][0] + vr[rl][1] * vc[cl][1] + vr[rl][2] * vc[cl][2]);
-              re += vv2.re + t1 * gt.kinig[ig - 1].re;
-              im += vv2.im + t1 * gt.kinig[ig - 1].im;
-            }
-          }
-          val = cplx{re, im};
-          if (row < col) out[col + (size_t)row * k.ldh] = cplx{re, -im};
-        }
-        tw[(lane & 31) * 17 + rh] = val;
+        const int row = row0 + 16 * h + 8 * (vv >> 2) + 4 * (lane >> 5) + (vv & 3);
+        om[vv] = (col < ngp && row <= col) ? k.o[col + (size_t)row * k.ldh] : cplx{0.0, 0.0};
       }
-      __syncthreads();
-      // 16 rows x 32 columns of this half: lane -> row (lane & 15), columns (lane >> 4) + 4 i
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int cc = (lane >> 4) + 4 * i, r = lane & 15;
-        const int grow = row0 + rb + 16 * h + r, gcol = col0 + cb + cc;
-        if (gcol < ngp && grow <= gcol) out[grow + (size_t)gcol * k.ldh] = tw[cc * 17 + r];
-      }
-      __syncthreads();                                       // the slice is rewritten next
     }
+#pragma unroll
+    for (int vv = 0; vv < 8; ++vv) {
+      const int rh = 8 * (vv >> 2) + 4 * (lane >> 5) + (vv & 3);   // row within the half
+      const int rl = 16 * h + rh, row = row0 + rl;
+      cplx val = {0.0, 0.0};
+      if (col < ngp && row <= col) {
+        // conj(a) b: Re = (U + V)/2, Im = (U - V)/(2 iota) modulo each m
+        const int sh = 8 * (vv & 3);
+        int sr[NM], si[NM];
+#pragma unroll
+        for (int l = 0; l < NM; ++l) {
+          const unsigned w1 = vv < 4 ? p1[l].x : p1[l].y, w2 = vv < 4 ? p2[l].x : p2[l].y;
+          const int u = (signed char)(w1 >> sh), v = (signed char)(w2 >> sh);
+          sr[l] = u + v;
+          si[l] = u - v;
+        }
+        const int sc = -(sw.ex[rl] + exc);
+        double re = ldexp(garner<NM, false>(sr), sc);
+        double im = ldexp(garner<NM, true>(si), sc);
+        const int ig = lookup_g(gt, sw.g[rl][0] - gc[0], sw.g[rl][1] - gc[1], sw.g[rl][2] - gc[2]);
+        if (it.which == 2) {
+          // O_APW = O - its interstitial term, O as the overlap kernel wrote it
+          cplx oa = {om[vv].re, -om[vv].im};
+          if (ig) {
+            const cplx tho = setup_dev::olp_theta(gt, ig, sw.v[rl], vc);
+            oa = cplx{oa.re - tho.re, oa.im - tho.im};
+          }
+          re = fma(-sig, oa.re, re);
+          im = fma(-sig, oa.im, im);
+        }
+        if (ig) {
+          const cplx th = gt.cfunig[ig - 1];
+          if (it.which == 1) {
+            re += th.re;
+            im += th.im;
+          } else {
+            const cplx vv2 = gt.veffig[ig - 1];
+            const double t1 = 0.5 * (sw.v[rl][0] * vc[0] + sw.v[rl][1] * vc[1] + sw.v[rl][2] * vc[2]);
+            re += vv2.re + t1 * gt.kinig[ig - 1].re;
+            im += vv2.im + t1 * gt.kinig[ig - 1].im;
+          }
+        }
+        val = cplx{re, im};
+        if (row < col) out[col + (size_t)row * k.ldh] = cplx{re, -im};
+      }
+      sw.t[(lane & 31) * 17 + rh] = val;
+    }
+    fence();
+    // 16 rows x 32 columns of this half: lane -> row (lane & 15), columns (lane >> 4) + 4 i
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int cc = (lane >> 4) + 4 * i, r = lane & 15;
+      const int grow = row0 + 16 * h + r, gcol = col0 + cc;
+      if (gcol < ngp && grow <= gcol) out[grow + (size_t)gcol * k.ldh] = sw.t[cc * 17 + r];
+    }
+    fence();                                                // the slice is rewritten next
   }
 }
 
 template <int NM>
 int launch_merge_t(const exc_dev &d, const kdesc *ks, const mt_item *items, int nitems, const CrtTab &t,
                    const signed char *res, int bt, int wr, int wc, const double *gsig, hipStream_t s) {
-  hipLaunchKernelGGL((crt_merge_kernel<NM>), dim3(nitems), dim3(256), 0, s, ks, items, res, bt, wr, wc,
-                     setup_dev::make_gtab(d), gsig);
+  hipLaunchKernelGGL((crt_merge_kernel<NM>), dim3(nitems * (bt * bt / 4096)), dim3(256), 0, s, ks, items, nitems, res, bt,
+                     wr, wc, setup_dev::make_gtab(d), gsig);
   EXC_CHECK(hipGetLastError());
   return EXC_OK;
 }
@@ -758,6 +831,20 @@ void exc_crt_tables(int n, CrtTab *t) {
     t->m[l] = kModList[l];
     t->iota[l] = iota_of(kModList[l]);
     t->dminv[l] = 1.0 / kModList[l];
+    t->finv[l] = 1.0f / (float)kModList[l];
+    const int m = kModList[l];
+    long long w = 1;
+    int sr[4], si[4];
+    for (int q = 0; q < 4; ++q) {
+      const int a = (int)w, b = (int)(w * t->iota[l] % m);
+      sr[q] = a > m / 2 ? a - m : a;
+      si[q] = b > m / 2 ? b - m : b;
+      w = w * 65536 % m;
+    }
+    for (int q = 0; q < 2; ++q) {
+      t->wr[l][q] = (int)(((unsigned)sr[2 * q + 1] << 16) | ((unsigned)sr[2 * q] & 0xffffu));
+      t->wi[l][q] = (int)(((unsigned)si[2 * q + 1] << 16) | ((unsigned)si[2 * q] & 0xffffu));
+    }
     lp += log2((double)kModList[l]);
   }
   // beta: the largest b with 2^(2b + 2) <= P, from log2 P with a margin against its rounding
@@ -771,7 +858,7 @@ int exc_launch_crt_prep(const exc_dev &d, int nk, int maxnp, const kdesc *ks, co
   if (nk <= 0 || maxnp <= 0) return EXC_OK;
   const int ktot = d.natm * d.naa, kp = exc_crt_kpad(ktot);
   if (gram) {
-    hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(256), 0, s, ks, ktot, t.beta, 2);
+    hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(64 * kScaleWaves), 0, s, ks, ktot, t.beta, 2);
     EXC_CHECK(hipGetLastError());
     hipLaunchKernelGGL(crt_split_kernel, dim3(maxnp / 64, kp / 64, nk), dim3(256), 0, s, ks, ktot, kp, t, 1);
     EXC_CHECK(hipGetLastError());
@@ -781,10 +868,10 @@ int exc_launch_crt_prep(const exc_dev &d, int nk, int maxnp, const kdesc *ks, co
     hipLaunchKernelGGL(crt_expo_kernel, dim3((maxnp + 255) / 256, 1, nk), dim3(256), 0, s, ks, d.natm, t.beta);
     EXC_CHECK(hipGetLastError());
   } else {
-    hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(256), 0, s, ks, ktot, t.beta, 0);
+    hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(64 * kScaleWaves), 0, s, ks, ktot, t.beta, 0);
     EXC_CHECK(hipGetLastError());
   }
-  hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(256), 0, s, ks, ktot, t.beta, 1);
+  hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(64 * kScaleWaves), 0, s, ks, ktot, t.beta, 1);
   EXC_CHECK(hipGetLastError());
   hipLaunchKernelGGL(crt_split_kernel, dim3(maxnp / 64, kp / 64, 2 * nk), dim3(256), 0, s, ks, ktot, kp, t, 0);
   EXC_CHECK(hipGetLastError());
@@ -839,6 +926,7 @@ int exc_launch_crt_merge(const exc_dev &d, const kdesc *ks, const mt_item *items
     case 10: return launch_merge_t<10>(d, ks, items, nitems, t, res, bt, wr, wc, gsig, s);
     case 11: return launch_merge_t<11>(d, ks, items, nitems, t, res, bt, wr, wc, gsig, s);
     case 12: return launch_merge_t<12>(d, ks, items, nitems, t, res, bt, wr, wc, gsig, s);
+    case kExactMod: return launch_merge_t<kExactMod>(d, ks, items, nitems, t, res, bt, wr, wc, gsig, s);
     default: return EXC_ERR_ARG;
   }
 }
