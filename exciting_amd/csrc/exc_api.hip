@@ -631,9 +631,52 @@ int y_narrow(const exc_ctx *c, long tiles, int wide) {
   return 4 * tiles <= c->ncu ? kYWave1 : tiles <= 2 * c->ncu ? kYWave2 : tiles <= 5 * c->ncu ? kYDirect : wide;
 }
 
+// Whether an FP64 batch's muffin-tin products conj(A) Yt^T run as exact integer products (k_crt.hip:
+// 16 moduli, operands as 57-bit integers of their row's scale, so that the only roundings are
+// the operands' and the result's: against 80-bit sums the error is an eighth to a third of the
+// FP64 MFMA tiles') instead of on FP64 MFMA.  Per k-point the MFMA tiles take 5.5e-8 K N^2 us, the
+// exact products 2.1e-8 K N^2 (residue GEMM) + 2.4e-5 K N (planes of both operands) + 2.2e-5 N^2
+// (reconstruction), K = natm naa: even at 700 / N + 650 / K = 1, with a margin for the tails of
+// smaller grids.  Measured for the whole grouped setup, graph replays (us; MFMA, exact; the left
+// side): K = 1936, N = 1200, 16 k-points 4052, 4257 (0.92); 2420, 1600, 8 k 3909, 3784 (0.71); 5808, 1200, 2
+// k 1731, 1564 (0.70); 2904, 1900, 8 k 6284, 5739 (0.59); 3872, 2500, 8 k 13738, 10961 (0.45); 7744, 5000,
+// 4 k 46263, 27646 (0.22).
+bool exact_pays(const exc_ctx *c, int maxn) {
+  return maxn > 0 && 700.0 / maxn + 650.0 / ((double)c->d.natm * c->d.naa) <= 0.7;
+}
+
+constexpr size_t kExactPlanes = (size_t)24 << 30;   // residue planes of the k-points in the workspace at a time
+
 long tri_tiles(int ngp, int t) {
   const long n = (ngp + t - 1) / t;
   return n * (n + 1) / 2;
+}
+
+// rows of a k-point's residue planes, and the planes' bytes for one operand (2 maps per modulus)
+int crt_rows(int ngp) { return (ngp + 255) / 256 * 256; }
+size_t crt_plane_bytes(int ngp, int nmod, int kp) { return (size_t)2 * nmod * kp * crt_rows(ngp); }
+
+// Whether the exact products' workspace (planes of one group of k-points, their residues) is
+// there or fits well into the free device memory; if not the batch runs on FP64 MFMA
+int exact_fits(exc_ctx *c, int nk, const exc_kpoint_dev *ks, bool olp, int cv, int nmod, int kp, bool *fits) {
+  int bt = 0, wr = 0, wc = 0;
+  *fits = false;
+  if (exc_crt_shape(cv, &bt, &wr, &wc)) return EXC_OK;
+  size_t q = 0, r = 0, qmax = 0, rmax = 0;
+  for (int k = 0; k < nk; ++k) {
+    const size_t b = 2 * crt_plane_bytes(ks[k].ngp, nmod, kp);
+    if (q && q + b > kExactPlanes) q = r = 0;
+    q += b;
+    r += (size_t)tri_tiles(ks[k].ngp, bt) * (olp ? 1 : 2) * nmod * 2 * bt * bt;
+    qmax = std::max(qmax, q);
+    rmax = std::max(rmax, r);
+  }
+  size_t need = 0, fr = 0, total = 0;
+  if (qmax > c->crt_q_bytes) need += qmax;
+  if (rmax > c->crt_res_bytes) need += rmax;
+  if (need) EXC_CHECK(hipMemGetInfo(&fr, &total));
+  *fits = !need || need < fr - fr / 4;
+  return EXC_OK;
 }
 
 // H (h given), O (o given) or both of one k-point from device arrays
@@ -835,17 +878,17 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
                  EXC_BATCH_SPLIT_CRT)))
     return EXC_ERR_ARG;
   const bool split = flags & EXC_BATCH_SPLIT_BF16;
-  const bool crt = flags & EXC_BATCH_SPLIT_CRT;
-  if (split && crt) return EXC_ERR_ARG;
+  const bool icrt = flags & EXC_BATCH_SPLIT_CRT;
+  if (split && icrt) return EXC_ERR_ARG;
   // exact int32 sums of K residue products: K 128^2 < 2^31
-  if (crt && c->d.natm * c->d.naa > 131000) return EXC_ERR_UNSUPPORTED;
+  if (icrt && c->d.natm * c->d.naa > 131000) return EXC_ERR_UNSUPPORTED;
   // the addition-theorem overlap needs the radial factors that only the grouped match writes
   const bool olp = flags & EXC_BATCH_OLP_LEGENDRE;
   if (olp && !(flags & EXC_BATCH_MATCH)) return EXC_ERR_ARG;
   if (split && c->d.naa > kSplitKB) return EXC_ERR_UNSUPPORTED;
   // 'iora*' overlap terms: the APW-APW factor I + h1aa in the addition-theorem form only; the
   // split products' O tiles take none of the terms
-  if (((c->d.iora & 1) || ((split || crt) && c->d.iora)) && !olp) return EXC_ERR_UNSUPPORTED;
+  if (((c->d.iora & 1) || ((split || icrt) && c->d.iora)) && !olp) return EXC_ERR_UNSUPPORTED;
   if (nk == 0) return EXC_OK;
   int rc = use_device(c);
   if (rc) return rc;
@@ -870,6 +913,9 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   // residue GEMM: the register-pipelined 256 x 256 form from N = 2048, 128 x 128 tiles below
   int maxn = 0;
   for (int k = 0; k < nk; ++k) maxn = std::max(maxn, ks[k].ngp);
+  // the FP64 path by exact integer products (its O tiles take no 'iora*' terms)
+  bool exact = !split && !icrt && c->bmt_variant < 0 && c->d.natm * c->d.naa <= 131000 && !(c->d.iora && !olp) &&
+               exact_pays(c, maxn);
   const int cv = c->crt_variant >= 0 ? c->crt_variant : (maxn >= 2048 ? 8 : 4);
   const int ov = c->olp_variant >= 0 ? c->olp_variant : 3;   // rows along lanes, column factors as scalars, pipelined
   int fv = c->fork_variant;
@@ -877,37 +923,45 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   // matrix (no 'iora*' h1aa); built in by default unless the shift sigma exceeds half of
   // h_a's largest |eigenvalue| (the form's rounding grows with sigma)
   bool gram = false;
-  if (crt && olp && !(c->d.iora & 1) && c->crt_form != 0) {
+  if (icrt && olp && !(c->d.iora & 1) && c->crt_form != 0) {
     if ((rc = gram_build(c))) return rc;
     gram = std::isfinite(c->gram_sigma) && (c->crt_form == 1 || c->gram_sigma <= 0.5 * c->gram_lmax);
   }
   // graph shape: one chain (faster for the FP64 path on workloads 1-4: the overlap kernel only
   // competes with the MT kernel), the overlap and lo on a side branch for the Gram form, whose
-  // residue GEMM leaves the vector units idle (+1% at workload 3; the merge waits for the branch)
-  if (fv < 0) fv = gram ? 0 : 1;
+  // residue GEMM leaves the vector units idle (+1% at workload 3; the merge waits for the branch),
+  // and for the exact products (13738 MFMA us of above: 10961 as one chain, 10829 with the branch)
+  if (fv < 0) fv = gram || exact ? 0 : 1;
   const cplx *gram_t = gram ? c->gram_table : nullptr;
   const double *gram_s = gram ? c->gram_sig_dev : nullptr;
   // moduli: the caller's count, else 10 with the Gram form (its rounding error is far below
   // the (A, Yt) form's: 5.7e-10 Ha at 10 moduli against 2.6e-9 at 11 on workload 3) and 11
-  const int nmod = c->crt_nmod > 0 ? c->crt_nmod : (gram ? 10 : 11);
+  const int nmod = exact ? kExactMod : c->crt_nmod > 0 ? c->crt_nmod : (gram ? 10 : 11);
   CrtTab ct;
-  if (crt) {
-    exc_crt_tables(nmod, &ct);
+  if (icrt || exact) exc_crt_tables(nmod, &ct);
+  if (icrt) {
     c->crt_last_form = gram ? 1 : 0;
     c->crt_last_nmod = nmod;
   }
-  constexpr int kCrtPlanes = 2;                             // residue planes per operand and modulus
   const int kp = exc_crt_kpad(c->d.natm * c->d.naa);
   // batch signature: descriptors, flags and variants
   // the Gram form's E stage on its triangular table: narrow column tiles skip more of it
   // (64 x 64 three-product tiles, 5.7 against 6.7 ms at workload 3; the dense Y stage keeps
   // 64 x 128, 8.8 against 9.1 ms)
   const int ye = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, 4);
-  int tail[9] = {nk, flags, bv, yv, crt ? cv : -1, (crt ? nmod : -1) + 100 * ov, fv, gram, ye};
+  int tail[9] = {nk, flags, bv, yv, icrt || exact ? cv : -1, (icrt || exact ? nmod : -1) + 100 * ov, fv, gram, ye};
   std::vector<char> sig(sizeof(exc_kpoint_dev) * nk + sizeof(tail));
   memcpy(sig.data(), ks, sizeof(exc_kpoint_dev) * nk);
   memcpy(sig.data() + sizeof(exc_kpoint_dev) * nk, tail, sizeof(tail));
   const bool same = (sig == c->batch_sig);
+  if (exact) {
+    if (same) {
+      exact = c->batch_exact;
+    } else if ((rc = exact_fits(c, nk, ks, olp, cv, ct.n, kp, &exact))) {
+      return rc;
+    }
+  }
+  const bool crt = icrt || exact;
   if (same && (flags & EXC_BATCH_GRAPH) && c->graph_exec) {
     StageTimer t(c, EXC_STAGE_GRAPH);
     EXC_CHECK(hipGraphLaunch(c->graph_exec, c->stream));
@@ -955,10 +1009,21 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
     // squared row norms of A per atom (cnp each), when the grouped match runs here
     const size_t nparts = do_match ? (size_t)c->d.natm : 0;
     size_t ptot2 = 0;
+    c->crt_groups.clear();
+    c->batch_exact = exact;
     if (crt) {
+      size_t q = 0;
       for (int k = 0; k < nk; ++k) {
-        const size_t cnp = (size_t)(ks[k].ngp + 255) / 256 * 256;
-        qtot += (size_t)(gram ? 1 : 2) * kCrtPlanes * ct.n * kp * cnp;   // the Gram form splits E only
+        const size_t cnp = crt_rows(ks[k].ngp);
+        const size_t b = (gram ? 1 : 2) * crt_plane_bytes(ks[k].ngp, ct.n, kp);   // the Gram form splits E only
+        // the exact products' many planes: the k-points in groups that share the workspace
+        if (k == 0 || (exact && q && q + b > kExactPlanes)) {
+          c->crt_groups.push_back({k, 0, 0, 0, 0, 0, 0});
+          q = 0;
+        }
+        c->crt_groups.back().nk += 1;
+        q += b;
+        qtot = std::max(qtot, q);
         xtot += 2 * cnp;
         ptot2 += nparts * cnp;
       }
@@ -968,11 +1033,11 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
     }
     std::vector<mt_item> citems;
     std::vector<int2> cwork;
-    size_t qoff = 0, xoff = 0, poff2 = 0;
-    int maxcnp = 0;
+    size_t qoff = 0, xoff = 0, poff2 = 0, rmax = 0;
+    size_t grp = 0;                                          // the group of k-point k
     std::vector<kdesc> kd(nk);
     std::vector<mt_item> items, oitems;
-    const int T = split ? exc_bsplit_tile(bv) : exc_bmt_tile(bv);
+    const int T = split ? exc_bsplit_tile(bv) : exact ? 64 : exc_bmt_tile(bv);
     const int TO = exc_olp_tile();
     size_t yoff = 0, poff = 0, eoff = 0, roff = 0, rtoff = 0;
     int maxngp = 0;
@@ -1019,17 +1084,25 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
         // planes [modulus][plane][K/16][cnp][16] of A then of Yt; tiles (k, ti <= tj, H | O)
         // in 4 x 4 blocks of tiles, and the (tile, modulus, product) work modulus- and
         // product-major within the k-point, the tiles in that block order
-        const int cnp = (q.ngp + 255) / 256 * 256;
+        if (k == c->crt_groups[grp].k0 + c->crt_groups[grp].nk) ++grp;
+        exc_ctx::CrtGroup &g = c->crt_groups[grp];
+        if (k == g.k0) {
+          qoff = 0;
+          g.item0 = (int)citems.size();
+          g.work0 = (int)cwork.size();
+        }
+        const int cnp = crt_rows(q.ngp);
+        const size_t pb = crt_plane_bytes(q.ngp, ct.n, kp);
         e.cnp = cnp;
         e.qa = (char *)c->crt_q + qoff;
-        e.qy = gram ? nullptr : (char *)c->crt_q + qoff + (size_t)kCrtPlanes * ct.n * kp * cnp;
-        qoff += (size_t)(gram ? 1 : 2) * kCrtPlanes * ct.n * kp * cnp;
+        e.qy = gram ? nullptr : (char *)c->crt_q + qoff + pb;
+        qoff += (gram ? 1 : 2) * pb;
         e.xa = c->crt_x + xoff;
         e.xy = c->crt_x + xoff + cnp;
         e.pa2 = (do_match && !gram) ? c->crt_parts + poff2 : nullptr;
         poff2 += nparts * cnp;
         xoff += 2 * (size_t)cnp;
-        maxcnp = cnp > maxcnp ? cnp : maxcnp;
+        g.maxcnp = std::max(g.maxcnp, cnp);
         const int nt = (q.ngp + cbt - 1) / cbt, first = (int)citems.size(), S = 4;
         for (int which = 0; which < (olp ? 1 : 2); ++which)
           for (int bj = 0; bj < nt; bj += S)
@@ -1039,7 +1112,10 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
                   citems.push_back({k, ti, tj, gram ? 2 : which});
         for (int l = 0; l < ct.n; ++l)
           for (int p = 0; p < 2; ++p)
-            for (int i = first; i < (int)citems.size(); ++i) cwork.push_back(make_int2(i, 4 * l + p));
+            for (int i = first; i < (int)citems.size(); ++i) cwork.push_back(make_int2(i - g.item0, 4 * l + p));
+        g.nitem = (int)citems.size() - g.item0;
+        g.nwork = (int)cwork.size() - g.work0;
+        rmax = std::max(rmax, (size_t)g.nitem * ct.n * 2 * cbt * cbt);
       }
       maxngp = q.ngp > maxngp ? q.ngp : maxngp;
       const int nt = (q.ngp + T - 1) / T;
@@ -1067,12 +1143,8 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
         EXC_CHECK(hipMemcpy(c->d_oitems, oitems.data(), sizeof(mt_item) * oitems.size(), hipMemcpyHostToDevice));
     }
     c->batch_noitems = (int)oitems.size();
-    c->batch_ncitems = (int)citems.size();
-    c->batch_ncwork = (int)cwork.size();
-    c->batch_maxcnp = maxcnp;
     if (crt) {
-      const size_t rbytes = (size_t)citems.size() * ct.n * 2 * cbt * cbt;
-      if ((rc = grow((void **)&c->crt_res, &c->crt_res_bytes, rbytes ? rbytes : 1))) return rc;
+      if ((rc = grow((void **)&c->crt_res, &c->crt_res_bytes, rmax ? rmax : 1))) return rc;
       if ((rc = grow((void **)&c->d_citems, &c->citems_cap, sizeof(mt_item) * (citems.empty() ? 1 : citems.size()))))
         return rc;
       if ((rc = grow((void **)&c->d_cwork, &c->cwork_cap, sizeof(int2) * (cwork.empty() ? 1 : cwork.size()))))
@@ -1148,21 +1220,28 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
     if (crt) {
       // the residue GEMM and the merge write only H's (and without the addition theorem O's)
       // APW-APW tiles: no conflict with the side branch
-      {
-        StageTimer t(c, capture ? -1 : EXC_STAGE_CRTPREP);
-        if ((r = exc_launch_crt_prep(c->d, nk, c->batch_maxcnp, c->d_ks, ct, do_match, gram, c->stream))) return r;
-      }
-      {
-        StageTimer t(c, capture ? -1 : EXC_STAGE_CRTGEMM);
-        if ((r = exc_launch_crt_gemm(c->d, c->d_ks, c->d_citems, c->d_cwork, c->batch_ncwork, ct, c->crt_res, cv,
-                                     c->stream)))
+      for (const exc_ctx::CrtGroup &g : c->crt_groups) {
+        {
+          StageTimer t(c, capture ? -1 : EXC_STAGE_CRTPREP);
+          if ((r = exc_launch_crt_prep(c->d, g.nk, g.maxcnp, c->d_ks + g.k0, ct, do_match, gram, exact, c->stream)))
+            return r;
+        }
+        {
+          StageTimer t(c, capture ? -1 : EXC_STAGE_CRTGEMM);
+          if ((r = exc_launch_crt_gemm(c->d, c->d_ks, c->d_citems + g.item0, c->d_cwork + g.work0, g.nwork, ct,
+                                       c->crt_res, cv, c->stream)))
+            return r;
+        }
+        if (gram && fork && hipStreamWaitEvent(c->stream, c->ev_join, 0) != hipSuccess) return EXC_ERR_HIP;
+        StageTimer t(c, capture ? -1 : EXC_STAGE_CRTMERGE);
+        if ((r = exc_launch_crt_merge(c->d, c->d_ks, c->d_citems + g.item0, g.nitem, ct, c->crt_res, cv, gram_s,
+                                      c->stream)))
           return r;
       }
-      if (gram && fork && hipStreamWaitEvent(c->stream, c->ev_join, 0) != hipSuccess) return EXC_ERR_HIP;
-      StageTimer t(c, capture ? -1 : EXC_STAGE_CRTMERGE);
-      if ((r = exc_launch_crt_merge(c->d, c->d_ks, c->d_citems, c->batch_ncitems, ct, c->crt_res, cv, gram_s,
-                                    c->stream)))
-        return r;
+      if (exact) {
+        StageTimer t(c, capture ? -1 : EXC_STAGE_BMT);
+        if ((r = exc_launch_bmt_fix(c->d, c->d_ks, c->d_items, c->batch_nitems, c->stream))) return r;
+      }
     } else if (split) {
       {
         StageTimer t(c, capture ? -1 : EXC_STAGE_SPLIT);

@@ -176,8 +176,11 @@ struct CrtTab {                      // passed by value to the kernels (kernel-a
 void exc_crt_tables(int n, CrtTab *t);
 inline int exc_crt_kpad(int ktot) { return (ktot + 63) / 64 * 64; }
 int exc_crt_shape(int variant, int *bt, int *wr, int *wc);   // tile edge and wave grid of a GEMM variant
+constexpr int kBadRow = -(1 << 29);   // row exponent of a row the exact products do not take (not finite, out of range)
 int exc_launch_crt_prep(const exc_dev &d, int nk, int maxnp, const kdesc *ks, const CrtTab &t, bool a_parts,
-                        bool gram, hipStream_t s);
+                        bool gram, bool exact, hipStream_t s);
+// the FP64 MFMA tiles of the items that hold a kBadRow row (none as a rule)
+int exc_launch_bmt_fix(const exc_dev &d, const kdesc *ks, const mt_item *items, int nitems, hipStream_t s);
 int exc_launch_crt_gemm(const exc_dev &d, const kdesc *ks, const mt_item *items, const int2 *work, int nwork,
                         const CrtTab &t, signed char *res, int variant, hipStream_t s);
 int exc_launch_crt_merge(const exc_dev &d, const kdesc *ks, const mt_item *items, int nitems, const CrtTab &t,

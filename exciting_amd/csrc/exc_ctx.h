@@ -102,7 +102,12 @@ struct exc_ctx {
   size_t citems_cap;
   int2 *d_cwork;
   size_t cwork_cap;
-  int batch_ncitems, batch_ncwork, batch_maxcnp;
+  // k-points whose residue planes are in the workspace at a time (ranges of the k, item and work lists)
+  struct CrtGroup {
+    int k0, nk, item0, nitem, work0, nwork, maxcnp;
+  };
+  std::vector<CrtGroup> crt_groups;
+  bool batch_exact;           // the FP64 batch's muffin-tin products run as exact integer products
   std::vector<char> batch_sig;   // the batch the descriptors / graph were built for
   int batch_nitems, batch_nblocks, batch_maxngp, batch_nk;
   hipGraph_t graph;

@@ -100,6 +100,31 @@ int launch_bmt_dma_grid_t(const exc_dev &d, const kdesc *ks, const mt_item *item
   return EXC_OK;
 }
 
+// After the exact products: the 64 x 64 FP64 tiles of the items with a row they did not take (its
+// exponents carry kBadRow), eight items per workgroup; without such a row this only reads the
+// exponents
+constexpr int kFixItems = 8;
+__global__ __launch_bounds__(512) void bmt_fix_kernel(const kdesc *__restrict__ ks, const mt_item *__restrict__ items,
+                                                      int nitems, int ktot, GTab gt, const int *__restrict__ kperm) {
+  using T = MtTileDMA<64, 16, 2, 2, 4, true>;
+  using St = typename T::Stage;
+  __shared__ typename T::Tables tb;
+  EXC_DMA_STAGES(St, 2)
+  const int end = min(nitems, ((int)blockIdx.x + 1) * kFixItems);
+  for (int it = blockIdx.x * kFixItems; it < end; ++it) {
+    const mt_item w = items[it];
+    const kdesc k = ks[w.k];
+    bool bad = false;
+    if (threadIdx.x < 128) {
+      const int idx = 64 * (threadIdx.x < 64 ? w.ti : w.tj) + (threadIdx.x & 63);
+      bad = idx < k.ngp && (k.xa[idx] == kBadRow || k.xy[idx] == kBadRow);
+    }
+    if (!__syncthreads_or(bad)) continue;
+    T::run(tb, EXC_DMA_STAGE_ARGS(St), k.ngp, ktot, k.apwalm, k.ldg, k.yt, k.ldy, k.igpig, k.vgpc, gt, k.h, k.o,
+           k.ldh, kperm, w.ti, w.tj, w.which);
+  }
+}
+
 // narrow tiles (mt_wave.h)
 template <int TB>
 __global__ __launch_bounds__(256) void bystage_wave_kernel(const kdesc *__restrict__ ks, int natm, int naa,
@@ -243,6 +268,14 @@ int exc_launch_bmt(const exc_dev &d, const kdesc *ks, const mt_item *items, int 
     case kMtWave2: return launch_bmt_wave_t<2>(d, ks, items, nitems, s);
     default: return EXC_ERR_ARG;
   }
+}
+
+int exc_launch_bmt_fix(const exc_dev &d, const kdesc *ks, const mt_item *items, int nitems, hipStream_t s) {
+  if (nitems <= 0) return EXC_OK;
+  hipLaunchKernelGGL(bmt_fix_kernel, dim3((nitems + kFixItems - 1) / kFixItems), dim3(512), 0, s, ks, items, nitems,
+                     d.natm * d.naa, make_gtab(d), d.kperm);
+  EXC_CHECK(hipGetLastError());
+  return EXC_OK;
 }
 
 int exc_launch_blo(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hipStream_t s) {

@@ -1,7 +1,11 @@
 // Modular split of the muffin-tin contraction on gfx950 (EXC_BATCH_SPLIT_CRT).
 //
 // H_MT = conj(A) Yt^T (and O_MT = conj(A) A^T) from exact integer products instead of FP64
-// MFMA, the other terms of the setup staying FP64:
+// MFMA, the other terms of the setup staying FP64.  The plain FP64 path takes the same route at
+// large sizes with 16 moduli (beta = 57, exc_setup_batched_dev's exact_pays): every element down
+// to 2^-4 of its row's 2-norm then enters with all its 53 bits, and rows the integers cannot
+// represent (not finite, norms outside 1e-125 .. 1e145) are marked and their tiles left to
+// FP64 MFMA (bmt_fix_kernel):
 //
 //  scale : per row i of an operand X (N x K complex, K = natm naa) the exponent e_i with
 //          |X_i|_2 < 2^e_i and s_i = beta - e_i, beta the largest with 2^(2 beta + 2) <= P,
@@ -67,25 +71,31 @@ __device__ __forceinline__ int dres(double x, int m, double minv) { return (int)
 constexpr int kScaleWaves = 16;
 
 __global__ __launch_bounds__(64 * kScaleWaves) void crt_scale_kernel(const kdesc *__restrict__ ks, int ktot, int beta,
-                                                                     int op) {
+                                                                     int op, int exact) {
   const kdesc k = ks[blockIdx.z];             // op 0: A (apwalm), 1: Yt, 2: E (in Yt's place) as the left operand
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row = blockIdx.x * 64 + lane;
   __shared__ double part[kScaleWaves][64];
+  __shared__ int some[64];                    // the row has a nonzero value
   if (blockIdx.x * 64 >= k.cnp) return;       // uniform over the workgroup
+  if (wave == 0) some[lane] = 0;
   const cplx *src = op ? k.yt : k.apwalm;
   const int ld = op ? k.ldy : k.ldg;
   const int kq = (ktot + kScaleWaves - 1) / kScaleWaves, k0 = wave * kq, k1 = min(ktot, k0 + kq);   // op 2 writes xa
   double acc = 0.0;
+  bool nz = false;
   if (row < k.ngp) {
 #pragma unroll 8
     for (int c = k0; c < k1; ++c) {
       const cplx v = src[row + (size_t)c * ld];
       acc = fma(v.re, v.re, acc);
       acc = fma(v.im, v.im, acc);
+      nz = nz || v.re != 0.0 || v.im != 0.0;
     }
   }
   part[wave][lane] = acc;
+  __syncthreads();
+  if (nz) some[lane] = 1;
   __syncthreads();
   if (wave == 0) {
     double s2 = 0.0;
@@ -93,13 +103,16 @@ __global__ __launch_bounds__(64 * kScaleWaves) void crt_scale_kernel(const kdesc
     for (int w = 0; w < kScaleWaves; ++w) s2 += part[w][lane];
     int e = 0;
     if (s2 > 0.0) frexp(sqrt(s2), &e);       // |X_i| < 2^e
-    (op == 1 ? k.xy : k.xa)[row] = row < k.ngp ? beta - e : 0;
+    int x = beta - e;
+    // not finite, or so large or small that the squares' sum is not the norm's
+    if (exact && (!(s2 < 1e290) || (s2 < 1e-250 && some[lane]))) x = kBadRow;
+    (op == 1 ? k.xy : k.xa)[row] = row < k.ngp ? x : 0;
   }
 }
 
 // A's exponents from the squared norms per (atom, row) that the grouped match wrote (in
 // closed form), summed in atom order: no pass over A.  One thread per row.
-__global__ __launch_bounds__(256) void crt_expo_kernel(const kdesc *__restrict__ ks, int natm, int beta) {
+__global__ __launch_bounds__(256) void crt_expo_kernel(const kdesc *__restrict__ ks, int natm, int beta, int exact) {
   const kdesc k = ks[blockIdx.z];
   const int row = blockIdx.x * 256 + threadIdx.x;
   if (row >= k.cnp) return;
@@ -108,7 +121,8 @@ __global__ __launch_bounds__(256) void crt_expo_kernel(const kdesc *__restrict__
     for (int a = 0; a < natm; ++a) s2 += k.pa2[(size_t)a * k.cnp + row];
   int e = 0;
   if (s2 > 0.0) frexp(sqrt(s2), &e);
-  k.xa[row] = row < k.ngp ? beta - e : 0;
+  const int x = exact && !(s2 < 1e290 && s2 > 1e-250) ? kBadRow : beta - e;
+  k.xa[row] = row < k.ngp ? x : 0;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -852,26 +866,28 @@ void exc_crt_tables(int n, CrtTab *t) {
 }
 
 // a_parts: the grouped match wrote A's squared norms per atom (else A takes a pass of its
-// own, as Yt always does); gram: E in Yt's buffer is the only operand
+// own, as Yt always does); gram: E in Yt's buffer is the only operand; exact: rows the integers
+// cannot hold are marked (kBadRow)
 int exc_launch_crt_prep(const exc_dev &d, int nk, int maxnp, const kdesc *ks, const CrtTab &t, bool a_parts,
-                        bool gram, hipStream_t s) {
+                        bool gram, bool exact, hipStream_t s) {
   if (nk <= 0 || maxnp <= 0) return EXC_OK;
+  const int ex = exact;
   const int ktot = d.natm * d.naa, kp = exc_crt_kpad(ktot);
   if (gram) {
-    hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(64 * kScaleWaves), 0, s, ks, ktot, t.beta, 2);
+    hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(64 * kScaleWaves), 0, s, ks, ktot, t.beta, 2, ex);
     EXC_CHECK(hipGetLastError());
     hipLaunchKernelGGL(crt_split_kernel, dim3(maxnp / 64, kp / 64, nk), dim3(256), 0, s, ks, ktot, kp, t, 1);
     EXC_CHECK(hipGetLastError());
     return EXC_OK;
   }
   if (a_parts) {
-    hipLaunchKernelGGL(crt_expo_kernel, dim3((maxnp + 255) / 256, 1, nk), dim3(256), 0, s, ks, d.natm, t.beta);
+    hipLaunchKernelGGL(crt_expo_kernel, dim3((maxnp + 255) / 256, 1, nk), dim3(256), 0, s, ks, d.natm, t.beta, ex);
     EXC_CHECK(hipGetLastError());
   } else {
-    hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(64 * kScaleWaves), 0, s, ks, ktot, t.beta, 0);
+    hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(64 * kScaleWaves), 0, s, ks, ktot, t.beta, 0, ex);
     EXC_CHECK(hipGetLastError());
   }
-  hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(64 * kScaleWaves), 0, s, ks, ktot, t.beta, 1);
+  hipLaunchKernelGGL(crt_scale_kernel, dim3(maxnp / 64, 1, nk), dim3(64 * kScaleWaves), 0, s, ks, ktot, t.beta, 1, ex);
   EXC_CHECK(hipGetLastError());
   hipLaunchKernelGGL(crt_split_kernel, dim3(maxnp / 64, kp / 64, 2 * nk), dim3(256), 0, s, ks, ktot, kp, t, 0);
   EXC_CHECK(hipGetLastError());
