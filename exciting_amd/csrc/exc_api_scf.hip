@@ -215,19 +215,19 @@ int exc_rhovalk_dev(exc_ctx *c, int lradstep, const double *zbshtvr, const doubl
   const size_t o_c = al(sizeof(cplx) * (size_t)ldw * nst);   // W, then evecfv evecsv, then the kernels' work
   const size_t o_k = o_c + (evecsv ? al(sizeof(cplx) * (size_t)nmat * nst) : 0);
   if ((rc = grow(&c->rvw, &c->rvw_bytes, o_k + exc_rhovalk_work_bytes(d, lmaxvr, c->dims.nlomax, nst)))) return rc;
-  exc_ctx::EigWorker &W = c->ew[0];
-  W.s = c->stream;
-  if (!W.blas && rocblas_create_handle(&W.blas) != rocblas_status_success) {
-    W.blas = nullptr;
-    return EXC_ERR_HIP;
-  }
-  if (rocblas_set_stream(W.blas, W.s) != rocblas_status_success) return EXC_ERR_HIP;
   const HmlLayout H = hml_layout(c, lmaxvr, nrmtmax);
   const char *b = (const char *)c->hml;
   const int *di = (const int *)(b + H.o_i);
-  const rocblas_double_complex one = {1.0, 0.0}, zero = {0.0, 0.0};
   StageTimer t(c, EXC_STAGE_SCF);
   if (evecsv) {   // the states evecfv evecsv (wavefmt is linear in the coefficients)
+    exc_ctx::EigWorker &W = c->ew[0];
+    W.s = c->stream;
+    if (!W.blas && rocblas_create_handle(&W.blas) != rocblas_status_success) {
+      W.blas = nullptr;
+      return EXC_ERR_HIP;
+    }
+    if (rocblas_set_stream(W.blas, W.s) != rocblas_status_success) return EXC_ERR_HIP;
+    const rocblas_double_complex one = {1.0, 0.0}, zero = {0.0, 0.0};
     cplx *c2 = (cplx *)((char *)c->rvw + o_c);
     if (rocblas_zgemm(W.blas, rocblas_operation_none, rocblas_operation_none, nmat, nst, nst, &one,
                       (const rocblas_double_complex *)evecfv, ldv, (const rocblas_double_complex *)evecsv, nst,
@@ -237,16 +237,14 @@ int exc_rhovalk_dev(exc_ctx *c, int lradstep, const double *zbshtvr, const doubl
     ldv = nmat;
   }
   // W = A^T C (the zdotu of wavefmt.f90:95 for every (atom, io, lm <= lmaxvr) and state at
-  // once): per atom the first apwordmax lmmaxvr columns of its apwalm block, one strided batch
-  // over the atoms; row a naa + io + apwordmax lm of W (leading dimension natm naa)
+  // once): per atom the first apwordmax lmmaxvr columns of its apwalm block; row
+  // a naa + io + apwordmax lm of W (leading dimension natm naa)
   if (ngp > 0) {
     const int mrows = d.apwordmax * (lmaxvr + 1) * (lmaxvr + 1);
-    if (rocblas_zgemm_strided_batched(W.blas, rocblas_operation_transpose, rocblas_operation_none, mrows, nst, ngp,
-                                      &one, (const rocblas_double_complex *)apwalm, ngkmax,
-                                      (rocblas_stride)ngkmax * d.naa, (const rocblas_double_complex *)evecfv, ldv, 0,
-                                      &zero, (rocblas_double_complex *)c->rvw, ldw, (rocblas_stride)d.naa,
-                                      d.natm) != rocblas_status_success)
-      return EXC_ERR_HIP;
+    if ((rc = exc_launch_xty(d.natm, ngp, (const cplx *)evecfv, ldv, nst, 0, (const cplx *)apwalm, ngkmax, mrows,
+                             (size_t)ngkmax * d.naa, (cplx *)c->rvw, ldw, d.naa, false, c->ncu,
+                             c->stream)))
+      return rc;
   } else {
     EXC_CHECK(hipMemsetAsync(c->rvw, 0, sizeof(cplx) * (size_t)ldw * nst, c->stream));
   }
@@ -449,7 +447,7 @@ int exc_gensfacgp(exc_ctx *c, int ngp, const double *vgpc, int ld, double *sfacg
 }
 
 namespace {
-constexpr int kRhoirChunk = 64;   // states per batched FFT of genrhoir
+constexpr int kRhoirChunk = 64;   // most states per batched FFT of genrhoir
 
 // rhoir += the interstitial density of the nst states of each of nk k-points (device arrays)
 int rhoir_run(exc_ctx *c, int nk, const int *ngp, const int *const *igpig, int nst, const int *ldv,
@@ -457,7 +455,9 @@ int rhoir_run(exc_ctx *c, int nk, const int *ngp, const int *const *igpig, int n
   int rc;
   if ((rc = scf_prepare(c))) return rc;
   const exc_dev &d = c->d;
-  const int N = c->dims.ngrtot, B = std::min(nst, kRhoirChunk);
+  const int N = c->dims.ngrtot;
+  // states per transform: nearly equal chunks (200 states: 4 of 50, not 3 of 64 and one of 64 for 8)
+  const int nch = (nst + kRhoirChunk - 1) / kRhoirChunk, B = (nst + nch - 1) / nch;
   if ((rc = grow((void **)&c->zb, &c->zb_bytes, sizeof(cplx) * (size_t)B * N))) return rc;
   if (c->fftb_n != B) {
     if (c->fftb_n > 0) hipfftDestroy(c->fftb);

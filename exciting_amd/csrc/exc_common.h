@@ -142,7 +142,8 @@ int exc_launch_vjp(const exc_dev &d, int ngp, int nst, const cplx *apwalm, int l
                    const double *wo, cplx *work, double *dedtau, double *dedv, int ncu, int yv, hipStream_t s);
 // out[b os + i si + j] = sum_k X(k, i) Y(k, j) (k_atc.hip)
 int exc_launch_xty(int nb, int n, const cplx *X, int ldx, int ni, size_t xs, const cplx *Y, int ldy, int nj, size_t ys,
-                   cplx *out, size_t si, size_t os, int ncu, hipStream_t s);
+                   cplx *out, size_t si, size_t os, bool three, int ncu,
+                   hipStream_t s);
 // split-BF16 muffin-tin stage
 constexpr int kSplitKB = 256;       // APW functions per atom block, padded (naa <= 256)
 constexpr int kSplitPlanes = 6;     // 3 slices x (re, im)

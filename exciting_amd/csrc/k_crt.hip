@@ -53,7 +53,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void;
 
-constexpr int kMaxTile = 256;    // largest tile edge of the gemm and merge kernels; rows padded to it
 
 // symmetric residue of an exact integer held in a double, |x| < 2^52, modulo an odd m
 // (|x/m| is never within 1/(2m) of a half-integer, far above the rounding of x/m)

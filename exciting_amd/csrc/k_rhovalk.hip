@@ -11,20 +11,24 @@
 //   z(itp, ir, j) = sum_f u_f(ir) P(itp, f, j)
 //   rfmt(itp, ir) = sum_j t_j |z|^2 = sum_{f <= f'} u_f(ir) u_f'(ir) R(itp, f, f'),
 //   R = (2 - delta_ff') Re sum_j t_j P(itp, f, j) conj(P(itp, f', j)),   t_j = w occ_j,
-// with t_j = 0 for |w occ_j| <= epsocc.  Three kernels: rv_p (per state and atom: the
-// coefficients in LDS, P for every (itp, f)), rv_q (per point and atom: R over the states in
-// chunks staged through LDS), rv_r (per 8 mesh points and atom: rfmt from R and u, then
-// rfshtvr).  Flops per k-point 8 lmmaxvr (2 lmaxvr + 1) nf nst + 4 lmmaxvr nf^2 nst per atom
-// and 2 lmmaxvr nf^2 + 2 lmmaxvr^2 per atom and mesh point, nf = apwordmax (lmaxvr + 1) +
+// with t_j = 0 for |w occ_j| <= epsocc.  Three kernels: rv_p (P), rv_q (R), rv_r (rfmt from R
+// and u, then rfshtvr).  Flops per k-point 8 lmmaxvr (2 lmaxvr + 1) nf nst + 4 lmmaxvr nf^2 nst
+// per atom and 2 lmmaxvr nf^2 + 2 lmmaxvr^2 per atom and mesh point, nf = apwordmax (lmaxvr + 1) +
 // nlomax, instead of 8 lmmaxvr^2 per atom, mesh point and state.
+//
+// All three sums run on the FP64 matrix cores: they are a few GFLOP in many short products, so
+// latency bounds them, and a 16 x 16 tile per wave with its operands straight from L2 (P is
+// written and read with the states contiguous) leaves few loads in a row.  8 atoms, lmaxvr 8, 200
+// states, 500 mesh points: rv_p 39 -> 16 us, rv_q 40 -> 16, rv_r 78 -> 24 (a thread per
+// element with LDS operands before).
 #include "exc_common.h"
 
 namespace {
 
 constexpr int kRvThreads = 256;
-constexpr int kRvChunk = 32;     // states per LDS stage of rv_q
-constexpr int kRvPts = 8;        // mesh points per workgroup of rv_r
-constexpr int kRvMaxM = 17;      // 2 lmaxvr + 1, lmaxvr <= 8
+constexpr int kRvMaxF = 31;      // radial functions of an atom
+constexpr int kRvMaxV = 81;      // lmmaxvr, lmaxvr <= 8
+constexpr int kRvSteps = 5;      // groups of 4 of the 2 l + 1 <= 17 orders m
 
 struct RvArgs {
   int lmv, lmaxvr, lradstep, nrmtmax, nlomax, lmaxapw, ao, naa, ldw, ngp, ldv, nst, nf, npair;
@@ -36,7 +40,7 @@ struct RvArgs {
   double wk, eps;
   const cplx *zb;                    // zbshtvr(itp, lm), lmv x lmv column-major
   const double *rf;                  // rfshtvr(lm, itp), lmv x lmv column-major
-  cplx *p;                           // P[((a lmv + itp) nst + j) nf + f]
+  cplx *p;                           // P[((a lmv + itp) nf + f) nst + j]
   double *r;                         // R[(a npair + pair) lmv + itp], pairs f <= f' row by row
   double *rhomt;                     // (lmv, nrmtmax, natm)
 };
@@ -51,121 +55,241 @@ __device__ __forceinline__ int rv_fun_l(const RvArgs &p, int is, int f) {
   return l <= p.lmaxvr ? l : -1;
 }
 
+__device__ __forceinline__ d4_t rv_mfma(double a, double b, d4_t c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// P for 16 points x 16 states of one atom: the radial functions of one l are a product of
+// zbshtvr's 2 l + 1 columns with the coefficients; the waves share the l (a nearly equal number
+// of orders m each) and the local orbitals
 __global__ __launch_bounds__(kRvThreads) void rv_p_kernel(exc_dev d, RvArgs p) {
-  __shared__ cplx ca[4 * 81];            // W(a, io, lm; j) at io + ao lm (ao <= 4, lmv <= 81)
-  __shared__ cplx cl[8 * kRvMaxM];       // lo coefficients (ilo, m + l), nlomax <= 8
-  const int j = blockIdx.x, a = blockIdx.y, t = threadIdx.x;
+  const int j0 = 16 * blockIdx.x, i0 = 16 * blockIdx.y, a = blockIdx.z;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int is = d.spidx[a], lmv = p.lmv, nfa = p.ao * (p.lmaxvr + 1);
-  for (int e = t; e < p.ao * lmv; e += kRvThreads) ca[e] = p.w[(size_t)p.ldw * j + (size_t)a * p.naa + e];
-  if (t == 0) {   // the atom's lo rows: (ilo, m), m fastest (genidxlo order)
-    const int lo0 = p.ngp + d.dm_lo[2 * a];
-    int off = 0;
-    for (int ilo = 0; ilo < p.nlorb[is]; ++ilo) {
-      const int l = p.lorbl[ilo + p.nlomax * is];
-      if (l <= p.lmaxvr)
-        for (int mm = 0; mm < 2 * l + 1; ++mm) cl[ilo * kRvMaxM + mm] = p.evec[lo0 + off + mm + (size_t)p.ldv * j];
-      off += 2 * l + 1;
+  const int itp = min(i0 + li, lmv - 1), jc = min(j0 + li, p.nst - 1);
+  // functions f0, f0 + 1 (the second if two) of angular momentum l, coefficient of order m at
+  // c[m cs], the second's next to it
+  auto put = [&](int f, const d4_t &re, const d4_t &im) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = i0 + 4 * v + lg;
+      if (i < lmv && j0 + li < p.nst)
+        p.p[(((size_t)a * lmv + i) * p.nf + f) * p.nst + j0 + li] = cplx{re[v], im[v]};
     }
+  };
+  auto fun = [&](int f0, bool two, int l, const cplx *c, int cs) {
+    const int nm = 2 * l + 1;
+    const cplx *zb = p.zb + itp + (size_t)lmv * (l * l);
+    cplx z[kRvSteps], x[kRvSteps], y[kRvSteps];
+#pragma unroll
+    for (int g = 0; g < kRvSteps; ++g)
+      if (4 * g < nm) {
+        const int m = min(4 * g + lg, nm - 1);
+        z[g] = zb[(size_t)lmv * m];
+        x[g] = c[(size_t)cs * m];
+        y[g] = c[(size_t)cs * m + (two ? 1 : 0)];
+      }
+    d4_t xr = {0.0, 0.0, 0.0, 0.0}, xi = xr, yr = xr, yi = xr;
+#pragma unroll
+    for (int g = 0; g < kRvSteps; ++g)
+      if (4 * g < nm) {
+        if (4 * g + lg >= nm) z[g] = x[g] = y[g] = cplx{0.0, 0.0};   // repeated orders
+        xr = rv_mfma(z[g].re, x[g].re, xr);
+        xi = rv_mfma(z[g].re, x[g].im, xi);
+        xr = rv_mfma(-z[g].im, x[g].im, xr);
+        xi = rv_mfma(z[g].im, x[g].re, xi);
+        if (two) {
+          yr = rv_mfma(z[g].re, y[g].re, yr);
+          yi = rv_mfma(z[g].re, y[g].im, yi);
+          yr = rv_mfma(-z[g].im, y[g].im, yr);
+          yi = rv_mfma(z[g].im, y[g].re, yi);
+        }
+      }
+    put(f0, xr, xi);
+    if (two) put(f0 + 1, yr, yi);
+  };
+  const cplx *w = p.w + (size_t)p.ldw * jc + (size_t)a * p.naa;
+  for (int t = 0; t <= p.lmaxvr; ++t) {
+    if (((t & 7) < 4 ? (t & 7) : 7 - (t & 7)) != wave) continue;
+    const int l = p.lmaxvr - t;
+    for (int io = 0; io < p.ao; io += 2) fun(p.ao * l + io, io + 1 < p.ao, l, w + io + p.ao * (l * l), p.ao);
   }
-  __syncthreads();
-  for (int e = t; e < lmv * p.nf; e += kRvThreads) {
-    const int itp = e / p.nf, f = e - itp * p.nf;
+  // the atom's lo rows: (ilo, m), m fastest (genidxlo order)
+  const cplx *lo = p.evec + (size_t)p.ldv * jc + p.ngp + d.dm_lo[2 * a];
+  int off = 0;
+  for (int f = nfa; f < p.nf; ++f) {
     const int l = rv_fun_l(p, is, f);
-    cplx v = {0.0, 0.0};
-    if (l >= 0) {
-      for (int mm = 0; mm < 2 * l + 1; ++mm) {
-        const cplx b = p.zb[itp + (size_t)lmv * (l * l + mm)];
-        const cplx c = f < nfa ? ca[(f % p.ao) + p.ao * (l * l + mm)] : cl[(f - nfa) * kRvMaxM + mm];
-        v.re += b.re * c.re - b.im * c.im;
-        v.im += b.re * c.im + b.im * c.re;
+    if ((f - nfa) % 4 == wave) {
+      if (l >= 0) {
+        fun(f, false, l, lo + off, 1);
+      } else {
+        const d4_t zero = {0.0, 0.0, 0.0, 0.0};
+        put(f, zero, zero);
       }
     }
-    p.p[(((size_t)a * lmv + itp) * p.nst + j) * p.nf + f] = v;
+    if (f - nfa < p.nlorb[is]) off += 2 * p.lorbl[f - nfa + p.nlomax * is] + 1;
   }
 }
 
-__global__ __launch_bounds__(kRvThreads) void rv_q_kernel(exc_dev d, RvArgs p) {
-  extern __shared__ cplx ps[];   // kRvChunk x nf, then kRvChunk weights
-  const int itp = blockIdx.x, a = blockIdx.y, t = threadIdx.x, nf = p.nf;
-  double *tw = (double *)(ps + kRvChunk * nf);
-  // this thread's pairs f <= f' (at most 2 per thread: npair <= 2 kRvThreads)
-  int f1[2] = {-1, -1}, g1[2] = {0, 0};
-  for (int k = 0; k < 2; ++k) {
-    int q = t + k * kRvThreads;
-    if (q >= p.npair) break;
-    int f = 0;
-    while (q >= nf - f) {
-      q -= nf - f;
-      ++f;
+// R of one point and atom: the pairs of functions as up to three 16 x 16 tiles (f <= f'), the
+// real and imaginary parts of 4 states a k-step each, the states split over the waves
+template <int TF>
+__global__ __launch_bounds__(kRvThreads) void rv_q_kernel(RvArgs p) {
+  constexpr int NT = TF * (TF + 1) / 2, U = 4;
+  __shared__ double red[NT * 4][4][64];
+  const int itp = blockIdx.x, a = blockIdx.y, nf = p.nf;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const cplx *pa = p.p + ((size_t)a * p.lmv + itp) * nf * p.nst;
+  const int ng = (p.nst + 3) / 4;
+  double sum[NT][4] = {};
+  for (int g0 = wave; g0 < ng; g0 += 4 * U) {
+    cplx x[U][TF];
+    double oc[U];
+    d4_t acc[NT];                                      // of these 16 states: short sums, as chunks round less
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = d4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = min(4 * (g0 + 4 * u) + lg, p.nst - 1);
+      oc[u] = p.occ[j];
+#pragma unroll
+      for (int t = 0; t < TF; ++t) x[u][t] = pa[(size_t)min(16 * t + li, nf - 1) * p.nst + j];
     }
-    f1[k] = f;
-    g1[k] = f + q;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = 4 * (g0 + 4 * u) + lg < p.nst;
+      const double t1 = p.wk * oc[u], tw = in && fabs(t1) > p.eps ? t1 : 0.0;   // rhovalk.f90:101-102
+#pragma unroll
+      for (int t = 0; t < TF; ++t)
+        if (!in) x[u][t] = cplx{0.0, 0.0};
+#pragma unroll
+      for (int t = 0, k = 0; t < TF; ++t)
+#pragma unroll
+        for (int q = t; q < TF; ++q, ++k) {
+          acc[k] = rv_mfma(tw * x[u][t].re, x[u][q].re, acc[k]);
+          acc[k] = rv_mfma(tw * x[u][t].im, x[u][q].im, acc[k]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NT; ++k)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sum[k][v] += acc[k][v];
   }
-  double acc[2] = {0.0, 0.0};
-  const cplx *pa = p.p + ((size_t)a * p.lmv + itp) * p.nst * nf;
-  for (int j0 = 0; j0 < p.nst; j0 += kRvChunk) {
-    const int nj = min(kRvChunk, p.nst - j0);
-    for (int e = t; e < nj * nf; e += kRvThreads) ps[e] = pa[(size_t)j0 * nf + e];
-    if (t < nj) {
-      const double t1 = p.wk * p.occ[j0 + t];
-      tw[t] = fabs(t1) > p.eps ? t1 : 0.0;   // rhovalk.f90:101-102
-    }
-    __syncthreads();
-    for (int k = 0; k < 2; ++k) {
-      if (f1[k] < 0) continue;
-      double s = 0.0;
-      for (int jj = 0; jj < nj; ++jj) {
-        const cplx x = ps[jj * nf + f1[k]], y = ps[jj * nf + g1[k]];
-        s += tw[jj] * (x.re * y.re + x.im * y.im);
-      }
-      acc[k] += s;
-    }
-    __syncthreads();
-  }
-  for (int k = 0; k < 2; ++k) {
-    if (f1[k] < 0) continue;
-    const int q = t + k * kRvThreads;
-    p.r[((size_t)a * p.npair + q) * p.lmv + itp] = (f1[k] == g1[k] ? 1.0 : 2.0) * acc[k];
+#pragma unroll
+  for (int k = 0; k < NT; ++k)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[4 * k + v][wave][lane] = sum[k][v];
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < NT; ++m) {
+    const int e = wave * NT + m, k = e >> 2;   // tiles in the order (0, 0), (0, 1), (1, 1)
+    const int f = 16 * (k == 2 ? 1 : 0) + 4 * (e & 3) + lg, g = 16 * (k > 0 ? 1 : 0) + li;
+    if (f > g || g >= nf) continue;
+    const double s = (red[e][0][lane] + red[e][1][lane]) + (red[e][2][lane] + red[e][3][lane]);
+    const int q = f * nf - f * (f - 1) / 2 + g - f;
+    p.r[((size_t)a * p.npair + q) * p.lmv + itp] = (f == g ? 1.0 : 2.0) * s;
   }
 }
 
-__global__ __launch_bounds__(128) void rv_r_kernel(exc_dev d, RvArgs p) {
-  extern __shared__ double us[];   // u[kRvPts][nf], then rfmt[kRvPts][lmv]
-  const int a = blockIdx.y, t = threadIdx.x, nf = p.nf, lmv = p.lmv;
+// 16 mesh points of one atom: rfmt = (u_f u_f') R over the pairs, then rfmt rfshtvr^T; a wave takes
+// every fourth tile of 16 harmonics
+__global__ __launch_bounds__(kRvThreads) void rv_r_kernel(exc_dev d, RvArgs p) {
+  constexpr int NV = (kRvMaxV + 15) / 16, NW = (NV + 3) / 4, U = 4;
+  __shared__ double us[kRvMaxF][17];
+  __shared__ unsigned char pf[kRvMaxF * (kRvMaxF + 1) / 2], pg[kRvMaxF * (kRvMaxF + 1) / 2];
+  __shared__ double rfm[kRvMaxV][17];
+  const int a = blockIdx.y, nf = p.nf, lmv = p.lmv;
   const int is = d.spidx[a], nr = p.nrmt[is];
-  const int irc0 = blockIdx.x * kRvPts;
+  const int irc0 = blockIdx.x * 16;
   if (irc0 * p.lradstep >= nr) return;   // uniform over the workgroup
-  double *rfm = us + kRvPts * nf;
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nfa = p.ao * (p.lmaxvr + 1);
-  for (int e = t; e < kRvPts * nf; e += 128) {
-    const int r = e / nf, f = e - r * nf, ir = (irc0 + r) * p.lradstep;
+  for (int e = threadIdx.x; e < 16 * nf; e += kRvThreads) {
+    const int f = e >> 4, r = e & 15, ir = (irc0 + r) * p.lradstep;
     double u = 0.0;
     if (ir < nr && rv_fun_l(p, is, f) >= 0)
       u = f < nfa ? p.apwfr[ir + (size_t)p.nrmtmax * 2 * ((f % p.ao) + (size_t)p.ao * (f / p.ao + (size_t)(p.lmaxapw + 1) * a))]
                   : p.lofr[ir + (size_t)p.nrmtmax * 2 * ((f - nfa) + (size_t)p.nlomax * a)];
-    us[e] = u;
+    us[f][r] = u;
+  }
+  for (int e = threadIdx.x; e < nf * nf; e += kRvThreads) {
+    const int f = e / nf, g = e - f * nf;
+    if (f > g) continue;
+    const int q = f * nf - f * (f - 1) / 2 + g - f;
+    pf[q] = (unsigned char)f;
+    pg[q] = (unsigned char)g;
   }
   __syncthreads();
-  if (t < lmv) {
-    double s[kRvPts];
-    for (int r = 0; r < kRvPts; ++r) s[r] = 0.0;
-    const double *ra = p.r + (size_t)a * p.npair * lmv + t;
-    int q = 0;
-    for (int f = 0; f < nf; ++f)
-      for (int g = f; g < nf; ++g, ++q) {
-        const double rv = ra[(size_t)q * lmv];
-        for (int r = 0; r < kRvPts; ++r) s[r] += rv * us[r * nf + f] * us[r * nf + g];
+  const int nv = (lmv + 15) / 16;
+  int vc[NW];   // this lane's column in each tile of this wave
+#pragma unroll
+  for (int w = 0; w < NW; ++w) vc[w] = min(16 * (wave + 4 * w) + li, lmv - 1);
+  const d4_t zero = {0.0, 0.0, 0.0, 0.0};
+  d4_t sum[NW], acc[NW];   // the sum and that of 16 of its terms (chunks round less)
+#pragma unroll
+  for (int w = 0; w < NW; ++w) sum[w] = zero;
+  if (wave < nv) {
+    const double *ra = p.r + (size_t)a * p.npair * lmv;
+    for (int q0 = 0; q0 < p.npair; q0 += 4 * U) {
+      double b[U][NW];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = min(q0 + 4 * u + lg, p.npair - 1);
+#pragma unroll
+        for (int w = 0; w < NW; ++w) b[u][w] = ra[(size_t)q * lmv + vc[w]];
       }
-    for (int r = 0; r < kRvPts; ++r) rfm[r * lmv + t] = s[r];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = min(q0 + 4 * u + lg, p.npair - 1);
+        const bool in = q0 + 4 * u + lg < p.npair;
+        const double x = in ? us[pf[q]][li] * us[pg[q]][li] : 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) acc[w] = rv_mfma(x, in ? b[u][w] : 0.0, u == 0 ? zero : acc[w]);
+      }
+#pragma unroll
+      for (int w = 0; w < NW; ++w) sum[w] += acc[w];
+    }
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+      if (16 * (wave + 4 * w) + li < lmv)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) rfm[16 * (wave + 4 * w) + li][4 * v + lg] = sum[w][v];
   }
   __syncthreads();
-  if (t < lmv) {   // rhomt(:, ir, a) += rfshtvr rfmt(:, ir)   (rhovalk.f90:183-207)
-    for (int r = 0; r < kRvPts; ++r) {
-      const int ir = (irc0 + r) * p.lradstep;
-      if (ir >= nr) break;
-      double v = 0.0;
-      for (int q = 0; q < lmv; ++q) v += p.rf[t + (size_t)lmv * q] * rfm[r * lmv + q];
-      p.rhomt[t + (size_t)lmv * (ir + (size_t)p.nrmtmax * a)] += v;
+  if (wave >= nv) return;
+  // rhomt(:, ir, a) += rfshtvr rfmt(:, ir)   (rhovalk.f90:183-207)
+#pragma unroll
+  for (int w = 0; w < NW; ++w) sum[w] = zero;
+  for (int q0 = 0; q0 < lmv; q0 += 4 * U) {
+    double b[U][NW];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = min(q0 + 4 * u + lg, lmv - 1);
+#pragma unroll
+      for (int w = 0; w < NW; ++w) b[u][w] = p.rf[vc[w] + (size_t)lmv * q];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = min(q0 + 4 * u + lg, lmv - 1);
+      const bool in = q0 + 4 * u + lg < lmv;
+      const double x = in ? rfm[q][li] : 0.0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) acc[w] = rv_mfma(x, in ? b[u][w] : 0.0, u == 0 ? zero : acc[w]);
+    }
+#pragma unroll
+    for (int w = 0; w < NW; ++w) sum[w] += acc[w];
+  }
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const int lm = 16 * (wave + 4 * w) + li;
+    if (lm >= lmv) continue;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int ir = (irc0 + 4 * v + lg) * p.lradstep;
+      if (ir < nr) p.rhomt[lm + (size_t)lmv * (ir + (size_t)p.nrmtmax * a)] += sum[w][v];
     }
   }
 }
@@ -189,7 +313,7 @@ int exc_launch_rhovalk(const exc_dev &d, int lmaxvr, int lradstep, int nrmtmax, 
   RvArgs p;
   p.nf = d.apwordmax * (lmaxvr + 1) + nl;
   p.npair = p.nf * (p.nf + 1) / 2;
-  if (lmaxvr > 8 || d.apwordmax > 4 || nl > 8 || p.npair > 2 * kRvThreads || lradstep < 1 || d.natm > 65535 ||
+  if (lmaxvr > 8 || d.apwordmax > 4 || nl > 8 || p.nf > kRvMaxF || lradstep < 1 || d.natm > 65535 ||
       nst > 65535)
     return EXC_ERR_ARG;
   p.lmv = lmv;
@@ -219,14 +343,15 @@ int exc_launch_rhovalk(const exc_dev &d, int lmaxvr, int lradstep, int nrmtmax, 
   p.p = (cplx *)work;
   p.r = (double *)((char *)work + ((sizeof(cplx) * d.natm * (size_t)lmv * nst * p.nf + 255) & ~(size_t)255));
   p.rhomt = rhomt;
-  hipLaunchKernelGGL(rv_p_kernel, dim3(nst, d.natm), dim3(kRvThreads), 0, s, d, p);
+  hipLaunchKernelGGL(rv_p_kernel, dim3((nst + 15) / 16, (lmv + 15) / 16, d.natm), dim3(kRvThreads), 0, s, d, p);
   EXC_CHECK(hipGetLastError());
-  const size_t lq = sizeof(cplx) * kRvChunk * p.nf + sizeof(double) * kRvChunk;
-  hipLaunchKernelGGL(rv_q_kernel, dim3(lmv, d.natm), dim3(kRvThreads), lq, s, d, p);
+  if (p.nf <= 16)
+    hipLaunchKernelGGL(rv_q_kernel<1>, dim3(lmv, d.natm), dim3(kRvThreads), 0, s, p);
+  else
+    hipLaunchKernelGGL(rv_q_kernel<2>, dim3(lmv, d.natm), dim3(kRvThreads), 0, s, p);
   EXC_CHECK(hipGetLastError());
   const int nrc = (nrmtmax + lradstep - 1) / lradstep;
-  const size_t lr = sizeof(double) * kRvPts * ((size_t)p.nf + lmv);
-  hipLaunchKernelGGL(rv_r_kernel, dim3((nrc + kRvPts - 1) / kRvPts, d.natm), dim3(128), lr, s, d, p);
+  hipLaunchKernelGGL(rv_r_kernel, dim3((nrc + 15) / 16, d.natm), dim3(kRvThreads), 0, s, d, p);
   EXC_CHECK(hipGetLastError());
   return EXC_OK;
 }

@@ -391,7 +391,7 @@ int exc_launch_vjp(const exc_dev &d, int ngp, int nst, const cplx *apwalm, int l
   int *key = (int *)(rep + d.ngvec), *perm = key + ngp;
   const GTab gt = setup_dev::make_gtab(d);
   int rc;
-  if ((rc = exc_launch_xty(1, ngp, apwalm, ldg, ktot, 0, evec, ldc, nst, 0, u, nst, 0, ncu, s))) return rc;
+  if ((rc = exc_launch_xty(1, ngp, apwalm, ldg, ktot, 0, evec, ldc, nst, 0, u, nst, 0, true, ncu, s))) return rc;
   if ((rc = exc_launch_ystage(d, nst, u, nst, hu, nst, yv, s))) return rc;
   hipLaunchKernelGGL(vjp_z_kernel, dim3((nst + 63) / 64, (d.naa + 3) / 4, d.natm), dim3(256), 0, s, ngp, nst, d.naa,
                      d.maxnlo, d.nlomax, d.apwordmax, d.dm_lo, d.lod, d.loa, d.oalo, evec, ldc, wh, wo, u, hu);
