@@ -917,7 +917,7 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   bool exact = !split && !icrt && c->bmt_variant < 0 && c->d.natm * c->d.naa <= 131000 && !(c->d.iora && !olp) &&
                exact_pays(c, maxn);
   const int cv = c->crt_variant >= 0 ? c->crt_variant : (maxn >= 2048 ? 8 : 4);
-  const int ov = c->olp_variant >= 0 ? c->olp_variant : 3;   // rows along lanes, column factors as scalars, pipelined
+  const int ov = c->olp_variant >= 0 ? c->olp_variant : kOlpBcast;   // rows along lanes, columns by DPP broadcast
   int fv = c->fork_variant;
   // the modular split's Gram form: needs O_APW from the addition theorem, equal to A's Gram
   // matrix (no 'iora*' h1aa); built in by default unless the shift sigma exceeds half of

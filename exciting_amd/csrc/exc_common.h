@@ -129,6 +129,8 @@ constexpr int kBmtVariants = 4;      // grouped MT
 // 32 wide with the sum split over the waves, and 64 wide without (Y stage); they sum in another
 // order than the variants counted above
 constexpr int kYWave1 = 16, kYWave2 = 17, kYDirect = 18, kMtWave1 = 16, kMtWave2 = 17;
+// the overlap kernel the default takes (not one of the numbered variants)
+constexpr int kOlpBcast = 16;
 // Grouped launches over nk k-points described by ks (device memory); maxngp bounds the grids.
 int exc_launch_bmatch(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hipStream_t s);
 int exc_launch_bystage(const exc_dev &d, int nk, int maxngp, const kdesc *ks, int variant, hipStream_t s);

@@ -16,8 +16,9 @@
 // thread (rows tr + 16 i, columns tc + (64 / CJ) j; variant 0: CJ = 2, 512 threads; variant
 // 1: CJ = 4, 256 threads, half the LDS reads per FMA); per atom the rows' and columns' radial
 // factors and structure factors are brought to LDS by DMA, the next atom's while the current
-// one is evaluated (two stages).  Variant 2 (the default, below) keeps the atom loop out of
-// LDS.  Epilogue as the MFMA tile: + Theta(G_i - G_j), store (i, j) and conj at (j, i).
+// one is evaluated (two stages).  Variant 2 (below) keeps the atom loop out of
+// LDS, and so does the default, after it.  Epilogue as the MFMA tile: + Theta(G_i - G_j), store (i, j) and
+// conj at (j, i).
 #include "setup_dev.h"
 #include "mt_dma.h"
 
@@ -564,6 +565,192 @@ void launch_pipe(const exc_dev &d, const kdesc *ks, const mt_item *items, int ni
                      make_gtab(d));
 }
 
+// ---------------------------------------------------------------------------------------
+// The default: variant 3's sums with no scalar loads.  Variant 3 takes the columns' factors of
+// every step as 32 scalars a wave, each used once, so they miss the scalar cache, and one step
+// ahead is as far as they fit: its FP64 units work half of the time (N = 5000, 32 atoms, 8
+// k-points: 7.0 ms for 3.9 ms of multiply-adds).  Here a wave takes 64 rows x 16 columns and the
+// columns' factors are loaded like the rows', one column a lane of each row of 16 lanes, four
+// steps ahead in order; the multiply-add takes lane e's value itself (DPP row_newbcast):
+//   b = bt b2;  b += x b1;  b += r_0 c_0[lane e];  b += r_1 c_1[lane e].
+// Two waves per SIMD (4 waves a workgroup, two workgroups per CU); the interstitial indices of all
+// of a lane's elements are looked up together, before the atom loop.  Bound by the FP64 units, the
+// broadcasting multiply-adds at about half rate: 6.0 ms there; N = 2500, 16 atoms, 8 k-points 1.0 -> 0.86;
+// N = 260, 5 atoms, 8 k-points 31 -> 21 us.
+// ---------------------------------------------------------------------------------------
+// b[A..D] += ca[lane A..D of the row] ra + cb[...] rb.  The s_nop covers the two wait states between
+// a vector instruction that may have written ca or cb and a DPP read of them.
+#define OLP_MAC4(A, B, C, D)                                                       \
+  asm("s_nop 1\n\t"                                                                \
+      "v_fmac_f64_dpp %0, %4, %6 row_newbcast:" #A " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %1, %4, %6 row_newbcast:" #B " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %2, %4, %6 row_newbcast:" #C " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %3, %4, %6 row_newbcast:" #D " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %0, %5, %7 row_newbcast:" #A " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %1, %5, %7 row_newbcast:" #B " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %2, %5, %7 row_newbcast:" #C " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %3, %5, %7 row_newbcast:" #D " row_mask:0xf bank_mask:0xf"     \
+      : "+&v"(t[A]), "+&v"(t[B]), "+&v"(t[C]), "+&v"(t[D])                         \
+      : "v"(ca), "v"(cb), "v"(ra), "v"(rb))
+__device__ __forceinline__ void olp_mac(double (&t)[16], double ca, double cb, double ra, double rb) {
+  OLP_MAC4(0, 1, 2, 3);
+  OLP_MAC4(4, 5, 6, 7);
+  OLP_MAC4(8, 9, 10, 11);
+  OLP_MAC4(12, 13, 14, 15);
+}
+#undef OLP_MAC4
+// (re, im)[A] += conj(u + i v) (ca + i cb)[lane A], u + i v = S(G) b
+#define OLP_PHASE(A)                                                               \
+  asm("s_nop 1\n\t"                                                                \
+      "v_fmac_f64_dpp %0, %2, %4 row_newbcast:" #A " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %1, %3, %4 row_newbcast:" #A " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %0, %3, %5 row_newbcast:" #A " row_mask:0xf bank_mask:0xf\n\t" \
+      "v_fmac_f64_dpp %1, %2, -%5 row_newbcast:" #A " row_mask:0xf bank_mask:0xf"    \
+      : "+&v"(re[A]), "+&v"(im[A])                                                 \
+      : "v"(ca), "v"(cb), "v"(ra * b[A]), "v"(rb * b[A]))
+__device__ __forceinline__ void olp_phase(double (&re)[16], double (&im)[16], const double (&b)[16], double ca,
+                                          double cb, double ra, double rb) {
+  OLP_PHASE(0); OLP_PHASE(1); OLP_PHASE(2); OLP_PHASE(3); OLP_PHASE(4); OLP_PHASE(5); OLP_PHASE(6); OLP_PHASE(7);
+  OLP_PHASE(8); OLP_PHASE(9); OLP_PHASE(10); OLP_PHASE(11); OLP_PHASE(12); OLP_PHASE(13); OLP_PHASE(14); OLP_PHASE(15);
+}
+#undef OLP_PHASE
+
+template <int NL>
+__global__ __launch_bounds__(256, 2) void olp_bcast_kernel(const kdesc *__restrict__ ks,
+                                                           const mt_item *__restrict__ items, int nitems, int natm,
+                                                           GTab gt) {
+  // columns per wave; steps per atom, and with the idle ones that keep a step's registers the same
+  // for every atom; steps loaded ahead
+  constexpr int E = 16, D = 4, NS = NL + 1, NSP = (NS + D - 1) / D * D;
+  __shared__ double uc[kOT][3];
+  __shared__ int gc[kOT][3];
+  __shared__ cplx tr[4][E * 65];
+  const int chunk = (nitems + 7) / 8, qb = blockIdx.x / 8;
+  const int item = (blockIdx.x % 8) * chunk + qb;
+  if (qb >= chunk || item >= nitems) return;
+  const mt_item w = items[item];
+  const kdesc k = ks[w.k];
+  const int ngp = k.ngp, row0 = w.ti * kOT, col0 = w.tj * kOT;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = row0 + lane, rowc = min(row, ngp - 1);
+  const int cw = col0 + E * wave;
+  const int ld = rft_ld(ngp);
+  const size_t sb = (size_t)ld * 16;                    // bytes per slot of rft
+  const unsigned rofs = (unsigned)row * 16, cofs = (unsigned)(cw + (lane & 15)) * 16;
+  gdv2 rr[D], cc[D];
+  auto issue = [&](int q, const unsigned char *at, int s) {
+    rr[q] = *(gdv2_ptr)(at + s * sb + rofs);
+    cc[q] = *(gdv2_ptr)(at + s * sb + cofs);
+  };
+  const unsigned char *base = (const unsigned char *)k.rft;
+#pragma unroll
+  for (int s = 0; s < D; ++s)
+    if (s < NS) issue(s, base, s);
+  if (threadIdx.x < kOT) {
+    const int q = threadIdx.x, idx = col0 + q;
+    double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+    int g0 = 0, g1 = 0, g2 = 0;
+    if (idx < ngp) {
+      double st, ct, sp, cp;
+      sincos(k.tpgpc[2 * idx], &st, &ct);
+      sincos(k.tpgpc[2 * idx + 1], &sp, &cp);
+      u0 = st * cp; u1 = st * sp; u2 = ct;
+      const int ig = k.igpig[idx] - 1;
+      g0 = gt.ivg[3 * ig]; g1 = gt.ivg[3 * ig + 1]; g2 = gt.ivg[3 * ig + 2];
+    }
+    uc[q][0] = u0; uc[q][1] = u1; uc[q][2] = u2;
+    gc[q][0] = g0; gc[q][1] = g1; gc[q][2] = g2;
+  }
+  double ur0, ur1, ur2;
+  int gr0, gr1, gr2;
+  {
+    double st, ct, sp, cp;
+    sincos(k.tpgpc[2 * rowc], &st, &ct);
+    sincos(k.tpgpc[2 * rowc + 1], &sp, &cp);
+    ur0 = st * cp; ur1 = st * sp; ur2 = ct;
+    const int ig = k.igpig[rowc] - 1;
+    gr0 = gt.ivg[3 * ig]; gr1 = gt.ivg[3 * ig + 1]; gr2 = gt.ivg[3 * ig + 2];
+  }
+  __syncthreads();
+  double x[E], are[E], aim[E];
+  int ig[E];                                            // index of G_i - G_j; 0: none, -1: not stored
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int q = E * wave + e, c = col0 + q;
+    x[e] = ur0 * uc[q][0] + ur1 * uc[q][1] + ur2 * uc[q][2];
+    are[e] = aim[e] = 0.0;
+    // lookup_g's index without its branches: the loads of all columns go out together
+    const int d0 = gr0 - gc[q][0] - gt.lo0, d1 = gr1 - gc[q][1] - gt.lo1, d2 = gr2 - gc[q][2] - gt.lo2;
+    const bool in = (unsigned)d0 < (unsigned)gt.n0 && (unsigned)d1 < (unsigned)gt.n1 && (unsigned)d2 < (unsigned)gt.n2;
+    const int v = gt.ivgig[in ? d0 + gt.n0 * (d1 + gt.n1 * d2) : 0];
+    ig[e] = in && v > 0 && v <= gt.ngvec ? v : 0;
+    if (!(c < ngp && row <= c)) ig[e] = -1;
+  }
+  double bt[NL];
+#pragma unroll
+  for (int l = 0; l < NL; ++l) bt[l] = kScaled.beta[l];
+#pragma unroll 1
+  for (int at = 0; at < natm; ++at) {
+    const unsigned char *next = at + 1 < natm ? base + NS * sb : base;   // (the last atom's again: unused)
+    double b1[E], b2[E];
+#pragma unroll
+    for (int s = 0; s < NSP; ++s) {
+      if (s < NL) {
+        double t[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          if (s == 0) t[e] = 0.0;
+          else if (s == 1) t[e] = x[e] * b1[e];
+          else t[e] = fma(x[e], b1[e], bt[NL - 1 - s] * b2[e]);
+        }
+        olp_mac(t, cc[s % D].x, cc[s % D].y, rr[s % D].x, rr[s % D].y);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          b2[e] = b1[e];
+          b1[e] = t[e];
+        }
+      } else if (s == NL) {                             // conj(S(G)) S(G') sum_l P_l c_l
+        olp_phase(are, aim, b1, cc[s % D].x, cc[s % D].y, rr[s % D].x, rr[s % D].y);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + D < NSP ? s + D < NS : s + D - NSP < NS) issue(s % D, s + D < NSP ? base : next, s + D < NSP ? s + D : s + D - NSP);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    base = next;
+  }
+  // + Theta(G_i - G_j); store (i, j) and conj at (j, i) through this wave's LDS slice, as variant 2
+  cplx *tw = tr[wave];
+  unsigned miss = 0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int c = cw + e;
+    const bool has = ig[e] > 0;
+    const cplx th = olp_theta(gt, has ? ig[e] : 1, k.vgpc + 3 * rowc, k.vgpc + 3 * min(c, ngp - 1));
+    are[e] += has ? th.re : 0.0;
+    aim[e] += has ? th.im : 0.0;
+    miss += ig[e] == 0;
+    if (ig[e] >= 0) k.o[row + (size_t)c * k.ldh] = cplx{are[e], aim[e]};
+    tw[e * 65 + lane] = cplx{are[e], -aim[e]};
+  }
+  if (miss && gt.miss) atomicAdd(gt.miss, miss);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int e = lane & 15, r = (lane >> 4) + 4 * i;
+    const int gr = row0 + r, c = cw + e;
+    if (c < ngp && gr < c) k.o[c + (size_t)gr * k.ldh] = tw[e * 65 + r];
+  }
+}
+
+template <int NL>
+void launch_bcast(const exc_dev &d, const kdesc *ks, const mt_item *items, int nitems, hipStream_t s) {
+  hipLaunchKernelGGL(olp_bcast_kernel<NL>, dim3((nitems + 7) / 8 * 8), dim3(256), 0, s, ks, items, nitems, d.natm,
+                     make_gtab(d));
+}
+
 }  // namespace
 
 int exc_olp_tile() { return kOT; }
@@ -618,6 +805,26 @@ int exc_launch_olp(const exc_dev &d, int nk, int maxngp, const kdesc *ks, const 
         case 11: launch_pipe<11>(d, ks, items, nitems, s); break;
         case 12: launch_pipe<12>(d, ks, items, nitems, s); break;
         case 13: launch_pipe<13>(d, ks, items, nitems, s); break;
+        default: return EXC_ERR_UNSUPPORTED;
+      }
+      break;
+    case kOlpBcast:
+      hipLaunchKernelGGL(olp_rft_kernel, dim3((maxngp + kOT - 1 + 255) / 256, d.natm, nk), dim3(256), 0, s, ks,
+                         d.lmaxmat + 1);
+      EXC_CHECK(hipGetLastError());
+      switch (d.lmaxmat + 1) {
+        case 2: launch_bcast<2>(d, ks, items, nitems, s); break;
+        case 3: launch_bcast<3>(d, ks, items, nitems, s); break;
+        case 4: launch_bcast<4>(d, ks, items, nitems, s); break;
+        case 5: launch_bcast<5>(d, ks, items, nitems, s); break;
+        case 6: launch_bcast<6>(d, ks, items, nitems, s); break;
+        case 7: launch_bcast<7>(d, ks, items, nitems, s); break;
+        case 8: launch_bcast<8>(d, ks, items, nitems, s); break;
+        case 9: launch_bcast<9>(d, ks, items, nitems, s); break;
+        case 10: launch_bcast<10>(d, ks, items, nitems, s); break;
+        case 11: launch_bcast<11>(d, ks, items, nitems, s); break;
+        case 12: launch_bcast<12>(d, ks, items, nitems, s); break;
+        case 13: launch_bcast<13>(d, ks, items, nitems, s); break;
         default: return EXC_ERR_UNSUPPORTED;
       }
       break;
