@@ -635,14 +635,15 @@ int y_narrow(const exc_ctx *c, long tiles, int wide) {
 // 16 moduli, operands as 57-bit integers of their row's scale, so that the only roundings are
 // the operands' and the result's: against 80-bit sums the error is an eighth to a third of the
 // FP64 MFMA tiles') instead of on FP64 MFMA.  Per k-point the MFMA tiles take 5.5e-8 K N^2 us, the
-// exact products 2.1e-8 K N^2 (residue GEMM) + 2.4e-5 K N (planes of both operands) + 2.2e-5 N^2
-// (reconstruction), K = natm naa: even at 700 / N + 650 / K = 1, with a margin for the tails of
+// exact products 2.1e-8 K N^2 (residue GEMM) + 2.4e-5 K N (planes of both operands) + 1.3e-5 N^2
+// (reconstruction), K = natm naa: even near 700 / N + 650 / K = 1, with a margin for the tails of
 // smaller grids.  Measured for the whole grouped setup, graph replays (us; MFMA, exact; the left
-// side): K = 1936, N = 1200, 16 k-points 4052, 4257 (0.92); 2420, 1600, 8 k 3909, 3784 (0.71); 5808, 1200, 2
-// k 1731, 1564 (0.70); 2904, 1900, 8 k 6284, 5739 (0.59); 3872, 2500, 8 k 13738, 10961 (0.45); 7744, 5000,
-// 4 k 46263, 27646 (0.22).
+// side): K = 1452, N = 1000, 16 k-points 2274, 2440 (1.15); 1936, 1200, 16 k 4149, 4015-4159 (0.92);
+// 7744, 900, 2 k 1618, 1460 (0.86); 2904, 1200, 4 k 1633, 1542 (0.81); 1452, 2000, 8 k 3794, 3271 (0.80);
+// 1936, 1600, 16 k 6519, 6033 (0.77); 2420, 1600, 8 k 4036, 3632 (0.71); 5808, 1200, 2 k 1725, 1501 (0.70); 2904,
+// 1900, 8 k 6596, 5478 (0.59); 3872, 2500, 8 k 13738, 10400 (0.45); 7744, 5000, 4 k 46263, 26800 (0.22).
 bool exact_pays(const exc_ctx *c, int maxn) {
-  return maxn > 0 && 700.0 / maxn + 650.0 / ((double)c->d.natm * c->d.naa) <= 0.7;
+  return maxn > 0 && 700.0 / maxn + 650.0 / ((double)c->d.natm * c->d.naa) <= 0.88;
 }
 
 constexpr size_t kExactPlanes = (size_t)24 << 30;   // residue planes of the k-points in the workspace at a time

@@ -545,8 +545,9 @@ __global__ __launch_bounds__(64 * WR * WC, 1) void crt_gemm_pipe_kernel(const kd
 // with that variant's wave grid), one lane per gemm lane with its 16 values.  Waves share
 // nothing: the rows' data sit in the wave's own LDS slice, the column's in registers, so there
 // is no barrier and a small batch still fills the chip (with a tile per workgroup and its blocks
-// in turn: 104 us for 5 atoms, N = 260, 8 k-points, 36 here; N = 5000, 32 atoms, 8 k: 2.56 ms, 2.29
-// here).  Bound by Garner's 32-bit arithmetic and by reading the residues and O and writing H.
+// in turn: 104 us for 5 atoms, N = 260, 8 k-points, 36 here; N = 5000, 32 atoms, 8 k: 2.56 ms, 2.26
+// here; with 16 moduli, N = 2500, 16 atoms, 8 k: 1.19 ms with a multiply-add per pair of
+// digits, 0.71).  Bound by Garner's 32-bit arithmetic and by reading the residues and O and writing H.
 // ---------------------------------------------------------------------------------------
 // The moduli and Garner's tables are fixed at compile time for each modulus count (the
 // moduli list is constant; only how many of them is chosen), so every reduction below
@@ -575,7 +576,7 @@ constexpr int iota_of(int m) {          // the smallest square root of -1 modulo
 // c_l = (2^-1 or (2 iota_l)^-1) M_l^-1 mod m_l and w[l][j] = (M_j mod m_l) M_l^-1 mod m_l.
 template <int NM>
 struct GarnerTab {
-  int w[NM][NM];
+  int w[NM][(NM + 3) / 4];   // -w_lj symmetric modulo m_l, a byte each, four j a word (0 for j >= l)
   int cre[NM], cim[NM];
   double mk;        // M_6 (or P for fewer moduli): x = x_hi M_6 + x_lo
   double mh, ml;    // M_12 = mh + ml
@@ -589,7 +590,11 @@ struct GarnerTab {
         ml = ml * kModList[j] % m;
       }
       const int v = inv_mod((int)ml, m);
-      for (int j = 0; j < l; ++j) w[l][j] = mj[j] * v % m;
+      for (int j = 0; j < l; ++j) {
+        int x = m - mj[j] * v % m;
+        if (x > m / 2) x -= m;
+        w[l][j / 4] |= (int)((unsigned)(x & 0xff) << (8 * (j % 4)));
+      }
       cre[l] = inv_mod(2, m) * v % m;
       cim[l] = inv_mod(2 * iota_of(m) % m, m) * v % m;
     }
@@ -612,15 +617,22 @@ __device__ __forceinline__ int cres(int x) {
   return x - __mul24((int)rintf((float)x * finv), m);
 }
 
-// |s_l c_l| <= 240 240 and |d_j w| <= 120 240: the sum stays below 2^22 for up to 16 moduli
+// |s_l c_l| <= 240 240 and |d_j w| <= 120 120: the sum stays below 2^22 for up to 16 moduli.  The
+// digits are packed four a word as they come, so that a dot product of bytes takes four of them (a
+// multiply-add each was half of the merge's instructions, and more code than the instruction cache holds).
 template <int NM, int L, bool IM>
-__device__ __forceinline__ void garner_digit(int (&d)[NM], const int (&s)[NM]) {
+__device__ __forceinline__ void garner_digit(int (&d)[NM], int (&dp)[(NM + 3) / 4], const int (&s)[NM]) {
   constexpr GarnerTab<NM> G{};
   int acc = __mul24(s[L], IM ? G.cim[L] : G.cre[L]);
 #pragma unroll
-  for (int j = 0; j < L; ++j) acc -= __mul24(d[j], G.w[L][j]);
+  for (int j = 0; j < (L + 3) / 4; ++j) acc = __builtin_amdgcn_sdot4(dp[j], G.w[L][j], acc, false);
   d[L] = cres<L>(acc);
-  if constexpr (L + 1 < NM) garner_digit<NM, L + 1, IM>(d, s);
+  if constexpr (L + 1 < NM) {
+    // byte L % 4 of word L / 4
+    if constexpr (L % 4 == 0) dp[L / 4] = d[L] & 0xff;
+    else dp[L / 4] = __builtin_amdgcn_perm((unsigned)d[L], (unsigned)dp[L / 4], L % 4 == 1 ? 0x0c0c0400u : L % 4 == 2 ? 0x0c040100u : 0x04020100u);
+    garner_digit<NM, L + 1, IM>(d, dp, s);
+  }
 }
 
 // Re' (IM false) or Im' in [-(P-1)/2, (P-1)/2] from s_l = U + V (or U - V) modulo each m_l:
@@ -629,8 +641,8 @@ __device__ __forceinline__ void garner_digit(int (&d)[NM], const int (&s)[NM]) {
 template <int NM, bool IM>
 __device__ __forceinline__ double garner(const int (&s)[NM]) {
   constexpr GarnerTab<NM> G{};
-  int d[NM];
-  garner_digit<NM, 0, IM>(d, s);
+  int d[NM], dp[(NM + 3) / 4];
+  garner_digit<NM, 0, IM>(d, dp, s);
   constexpr int NLO = NM < kCrtLoDigits ? NM : kCrtLoDigits, NMID = NM < 2 * kCrtLoDigits ? NM : 2 * kCrtLoDigits;
   double lo = (double)d[NLO - 1];
 #pragma unroll
@@ -720,6 +732,7 @@ __global__ __launch_bounds__(256) void crt_merge_kernel(const kdesc *__restrict_
       q2[l] = *(const uint4 *)(base + (size_t)l * 2 * ptile + ptile);
     }
   }
+  unsigned miss = 0;
   fence();
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -734,6 +747,19 @@ __global__ __launch_bounds__(256) void crt_merge_kernel(const kdesc *__restrict_
         p2[l] = *(const uint2 *)(base + (size_t)l * 2 * ptile + ptile + 8 * h);
       }
     }
+    // the interstitial indices of this half's 8 elements (lookup_g without its branches: the loads
+    // go out together), -1 where nothing is stored
+    int ig[8];
+#pragma unroll
+    for (int vv = 0; vv < 8; ++vv) {
+      const int rl = 16 * h + 8 * (vv >> 2) + 4 * (lane >> 5) + (vv & 3), row = row0 + rl;
+      const int d0 = sw.g[rl][0] - gc[0] - gt.lo0, d1 = sw.g[rl][1] - gc[1] - gt.lo1, d2 = sw.g[rl][2] - gc[2] - gt.lo2;
+      const bool in = (unsigned)d0 < (unsigned)gt.n0 && (unsigned)d1 < (unsigned)gt.n1 && (unsigned)d2 < (unsigned)gt.n2;
+      const int v = gt.ivgig[in ? d0 + gt.n0 * (d1 + gt.n1 * d2) : 0];
+      ig[vv] = in && v > 0 && v <= gt.ngvec ? v : 0;
+      if (!(col < ngp && row <= col)) ig[vv] = -1;
+      miss += ig[vv] == 0;
+    }
     // Gram form: this half's eight O elements, loaded together ahead of the reconstruction;
     // read at (col, row), O's conjugate mirror (bit for bit), where the lanes are contiguous
     cplx om[8];
@@ -741,7 +767,7 @@ __global__ __launch_bounds__(256) void crt_merge_kernel(const kdesc *__restrict_
 #pragma unroll
       for (int vv = 0; vv < 8; ++vv) {
         const int row = row0 + 16 * h + 8 * (vv >> 2) + 4 * (lane >> 5) + (vv & 3);
-        om[vv] = (col < ngp && row <= col) ? k.o[col + (size_t)row * k.ldh] : cplx{0.0, 0.0};
+        om[vv] = ig[vv] >= 0 ? k.o[col + (size_t)row * k.ldh] : cplx{0.0, 0.0};
       }
     }
 #pragma unroll
@@ -749,7 +775,7 @@ __global__ __launch_bounds__(256) void crt_merge_kernel(const kdesc *__restrict_
       const int rh = 8 * (vv >> 2) + 4 * (lane >> 5) + (vv & 3);   // row within the half
       const int rl = 16 * h + rh, row = row0 + rl;
       cplx val = {0.0, 0.0};
-      if (col < ngp && row <= col) {
+      {
         // conj(a) b: Re = (U + V)/2, Im = (U - V)/(2 iota) modulo each m
         const int sh = 8 * (vv & 3);
         int sr[NM], si[NM];
@@ -763,31 +789,28 @@ __global__ __launch_bounds__(256) void crt_merge_kernel(const kdesc *__restrict_
         const int sc = -(sw.ex[rl] + exc);
         double re = ldexp(garner<NM, false>(sr), sc);
         double im = ldexp(garner<NM, true>(si), sc);
-        const int ig = lookup_g(gt, sw.g[rl][0] - gc[0], sw.g[rl][1] - gc[1], sw.g[rl][2] - gc[2]);
+        const bool has = ig[vv] > 0;
+        const int g = max(ig[vv], 1);
         if (it.which == 2) {
           // O_APW = O - its interstitial term, O as the overlap kernel wrote it
           cplx oa = {om[vv].re, -om[vv].im};
-          if (ig) {
-            const cplx tho = setup_dev::olp_theta(gt, ig, sw.v[rl], vc);
-            oa = cplx{oa.re - tho.re, oa.im - tho.im};
-          }
+          const cplx tho = setup_dev::olp_theta(gt, g, sw.v[rl], vc);
+          oa = cplx{oa.re - (has ? tho.re : 0.0), oa.im - (has ? tho.im : 0.0)};
           re = fma(-sig, oa.re, re);
           im = fma(-sig, oa.im, im);
         }
-        if (ig) {
-          const cplx th = gt.cfunig[ig - 1];
-          if (it.which == 1) {
-            re += th.re;
-            im += th.im;
-          } else {
-            const cplx vv2 = gt.veffig[ig - 1];
-            const double t1 = 0.5 * (sw.v[rl][0] * vc[0] + sw.v[rl][1] * vc[1] + sw.v[rl][2] * vc[2]);
-            re += vv2.re + t1 * gt.kinig[ig - 1].re;
-            im += vv2.im + t1 * gt.kinig[ig - 1].im;
-          }
+        if (it.which == 1) {
+          const cplx th = gt.cfunig[g - 1];
+          re += has ? th.re : 0.0;
+          im += has ? th.im : 0.0;
+        } else {
+          const cplx vv2 = gt.veffig[g - 1], kin = gt.kinig[g - 1];
+          const double t1 = 0.5 * (sw.v[rl][0] * vc[0] + sw.v[rl][1] * vc[1] + sw.v[rl][2] * vc[2]);
+          re += has ? vv2.re + t1 * kin.re : 0.0;
+          im += has ? vv2.im + t1 * kin.im : 0.0;
         }
         val = cplx{re, im};
-        if (row < col) out[col + (size_t)row * k.ldh] = cplx{re, -im};
+        if (row < col && col < ngp) out[col + (size_t)row * k.ldh] = cplx{re, -im};
       }
       sw.t[(lane & 31) * 17 + rh] = val;
     }
@@ -801,6 +824,7 @@ __global__ __launch_bounds__(256) void crt_merge_kernel(const kdesc *__restrict_
     }
     fence();                                                // the slice is rewritten next
   }
+  if (miss && gt.miss) atomicAdd(gt.miss, miss);
 }
 
 template <int NM>
