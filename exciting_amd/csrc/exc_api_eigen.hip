@@ -185,10 +185,10 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   const size_t o_e = o_d + al(8 * (size_t)n * nb);
   const size_t o_tau = o_e + al(8 * (size_t)n * nb), o_i = o_tau + al(16 * (size_t)n * nb);
   const size_t o_kd = o_i + al(12 * (size_t)nb);
-  // variant 6: V (n x kBT), G and T (kBT x kBT), W1 and W2 (kBT x nev) per k-point
+  // variant 6: V (n x kBT), W1 and W2 (kBT x nev) per k-point, G and T (kBT x kBT) of every block
+  const size_t bt = blocked ? al(16 * (size_t)kBT * kBT * nb * ((n - 1 + kBT - 1) / kBT)) : 0;
   const size_t o_v = o_kd + al(sizeof(eig_kdesc) * nb), o_g = o_v + (blocked ? al(16 * (size_t)n * kBT * nb) : 0);
-  const size_t o_t = o_g + (blocked ? al(16 * (size_t)kBT * kBT * nb) : 0);
-  const size_t o_w1 = o_t + (blocked ? al(16 * (size_t)kBT * kBT * nb) : 0);
+  const size_t o_t = o_g + bt, o_w1 = o_t + bt;
   const size_t o_w2 = o_w1 + (blocked ? al(16 * (size_t)kBT * nev * nb) : 0);
   const size_t o_wv = o_w2 + (blocked ? al(16 * (size_t)kBT * nev * nb) : 0);
   // variant 7: eigenvalues, block and split indices, failure flags (n each) and 4 ints per k-point
@@ -196,7 +196,8 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   const size_t o_is = o_ib + (bisect ? al(4 * (size_t)n * nb) : 0);
   const size_t o_if = o_is + (bisect ? al(4 * (size_t)n * nb) : 0);
   const size_t o_si = o_if + (bisect ? al(4 * (size_t)n * nb) : 0);
-  const size_t total = o_si + (bisect ? al(16 * (size_t)nb) : 0);
+  const size_t o_tr = o_si + (bisect ? al(16 * (size_t)nb) : 0);
+  const size_t total = o_tr + (bisect ? 0 : al(exc_trd_work_bytes(n, nb)));
   int rc;
   if ((rc = grow(&c->eg, &c->eg_bytes, total))) return rc;
   char *base = (char *)c->eg;
@@ -230,7 +231,7 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   std::vector<int> hi(3 * (size_t)nb, 0);
   // every handle's workspace sized for its calls (the largest order n) before anything is queued
   {
-    auto *V = (rocblas_double_complex *)(base + o_v), *G = (rocblas_double_complex *)(base + o_g);
+    auto *V = (rocblas_double_complex *)(base + o_v);
     auto *T = (rocblas_double_complex *)(base + o_t), *W1 = (rocblas_double_complex *)(base + o_w1);
     auto *W2 = (rocblas_double_complex *)(base + o_w2);
     const rocblas_double_complex zero = {0.0, 0.0}, mone = {-1.0, 0.0};
@@ -243,11 +244,11 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
            rocsolver_ztrtri_strided_batched(hb, up, nu, n, B, n, sm, info + nb, nb);
            rocblas_ztrmm_strided_batched(hb, rocblas_side_right, up, N, nu, n, n, &one, B, n, sm, A, n, sm, Z, n, sm, nb);
            rocblas_ztrmm_strided_batched(hb, rocblas_side_left, up, CT, nu, n, n, &one, B, n, sm, Z, n, sm, A, n, sm, nb);
-           rocsolver_zhetrd_strided_batched(hb, up, n, A, n, sm, d, n, e, n, (rocblas_double_complex *)tau, n, nb);
+           if (bisect)
+             rocsolver_zhetrd_strided_batched(hb, up, n, A, n, sm, d, n, e, n, (rocblas_double_complex *)tau, n, nb);
            if (blocked) {
-             rocblas_zgemm_strided_batched(hb, CT, N, ib, ib, n, &one, V, n, sv, V, n, sv, &zero, G, ib, st2, nb);
              rocblas_zgemm_strided_batched(hb, CT, N, ib, nev, n, &one, V, n, sv, Z, n, sxx, &zero, W1, ib, sw, nb);
-             rocblas_zgemm_strided_batched(hb, N, N, ib, nev, ib, &one, T, ib, st2, W1, ib, sw, &zero, W2, ib, sw, nb);
+             rocblas_zgemm_strided_batched(hb, N, N, ib, nev, ib, &one, T, kBT, st2, W1, ib, sw, &zero, W2, ib, sw, nb);
              rocblas_zgemm_strided_batched(hb, N, N, n, nev, ib, &mone, V, n, sv, W2, ib, sw, &one, Z, n, sxx, nb);
              rocblas_ztrmm_strided_batched(hb, rocblas_side_left, up, N, nu, n, nev, &one, B, n, sm, Z, n, sxx, A, n, sxx,
                                            nb);
@@ -294,9 +295,21 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   if (st == rocblas_status_success)   // H = U^-H Z
     st = rocblas_ztrmm_strided_batched(hb, rocblas_side_left, up, rocblas_operation_conjugate_transpose, nu, n, n,
                                        &one, B, n, sm, Z, n, sm, A, n, sm, nb);
-  if (st == rocblas_status_success)   // C = Q T Q^H
+  if (st != rocblas_status_success) return fail("trtri / trmm strided_batched status", (int)st, n);
+  // C = Q T Q^H: k_trd.hip reads both triangles, the lower one made the upper's conjugate.  Variant 7
+  // keeps the library's reduction: dstebz picks the lowest nev by a count over the whole of T and then
+  // works on T split at its smallest e, and on another T of the same matrix (equal to rounding) it has
+  // left out a repeated lowest eigenvalue.
+  if (bisect) {
     st = rocsolver_zhetrd_strided_batched(hb, up, n, A, n, sm, d, n, e, n, (rocblas_double_complex *)tau, n, nb);
-  if (st != rocblas_status_success) return fail("trtri / trmm / zhetrd strided_batched status", (int)st, n);
+    if (st != rocblas_status_success) return fail("zhetrd strided_batched status", (int)st, n);
+  } else {
+    for (int b = 0; b < nb; ++b)
+      if ((rc = exc_launch_eig_hermfill(ph + (size_t)b * mat, n, n, c->stream))) return rc;
+    if ((rc = exc_launch_trd(n, nb, ph, d, e, tau, base + o_tr, c->stream))) return rc;
+  }
+  auto block_t = [&](int i0) { return (cplx *)(base + o_t) + (size_t)(i0 / kBT) * kBT * kBT * nb; };
+  if (blocked && (rc = exc_launch_eig_tblock(dkd, ph, tau, nb, n, (cplx *)(base + o_g), block_t(0), c->stream))) return rc;
   // variant 6: the eigenvectors of T of k-point b in X = pz + b n nev (rows past nmat_k zero)
   const size_t sx = (size_t)n * nev;
   if (blocked) EXC_CHECK(hipMemsetAsync(pz, 0, sizeof(cplx) * sx * nb, c->stream));
@@ -356,22 +369,19 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   if (err) return err;
   if (blocked) {
     // X := Q X = H(n-2) ... H(0) X, block [i0, i0 + ib) of reflectors at a time, block 0 first
-    auto *V = (rocblas_double_complex *)(base + o_v), *G = (rocblas_double_complex *)(base + o_g);
-    auto *T = (rocblas_double_complex *)(base + o_t), *W1 = (rocblas_double_complex *)(base + o_w1);
+    auto *V = (rocblas_double_complex *)(base + o_v), *W1 = (rocblas_double_complex *)(base + o_w1);
     auto *W2 = (rocblas_double_complex *)(base + o_w2);
     const rocblas_double_complex zero = {0.0, 0.0}, mone = {-1.0, 0.0};
     const auto N = rocblas_operation_none, CT = rocblas_operation_conjugate_transpose;
     const rocblas_stride sv = (rocblas_stride)n * kBT, st2 = (rocblas_stride)kBT * kBT;
     const rocblas_stride sw = (rocblas_stride)kBT * nev, sxx = (rocblas_stride)sx;
     for (int i0 = 0; i0 < n - 1 && st == rocblas_status_success; i0 += kBT) {
-      const int ib = std::min(kBT, n - 1 - i0), mb = i0 + ib;   // rows 0 .. mb-1 of the block's vectors
+      const int ib = std::min(kBT, n - 1 - i0), mb = i0 + ib;
+      auto *T = (rocblas_double_complex *)block_t(i0);
       if ((rc = exc_launch_eig_vblock(ph, nb, n, i0, ib, sv, (cplx *)V, c->stream))) return rc;
-      st = rocblas_zgemm_strided_batched(hb, CT, N, ib, ib, mb, &one, V, n, sv, V, n, sv, &zero, G, ib, st2, nb);
-      if (st != rocblas_status_success) break;
-      if ((rc = exc_launch_eig_tblock(dkd, (const cplx *)G, tau, nb, n, i0, ib, st2, (cplx *)T, c->stream))) return rc;
       st = rocblas_zgemm_strided_batched(hb, CT, N, ib, nev, mb, &one, V, n, sv, Z, n, sxx, &zero, W1, ib, sw, nb);
       if (st == rocblas_status_success)
-        st = rocblas_zgemm_strided_batched(hb, N, N, ib, nev, ib, &one, T, ib, st2, W1, ib, sw, &zero, W2, ib, sw, nb);
+        st = rocblas_zgemm_strided_batched(hb, N, N, ib, nev, ib, &one, T, kBT, st2, W1, ib, sw, &zero, W2, ib, sw, nb);
       if (st == rocblas_status_success)
         st = rocblas_zgemm_strided_batched(hb, N, N, mb, nev, ib, &mone, V, n, sv, W2, ib, sw, &one, Z, n, sxx, nb);
     }

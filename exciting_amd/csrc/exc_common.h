@@ -201,10 +201,13 @@ int exc_launch_eig_hermfill(cplx *h, int n, int ldh, hipStream_t s);
 int exc_launch_eig_pad(const eig_kdesc *ks, int nb, int n, cplx *ph, cplx *po, double sigma, hipStream_t s);
 int exc_launch_eig_r2c(const double *zr, int m, int ncols, int ldr, cplx *zc, int ldc, hipStream_t s);
 int exc_launch_eig_vblock(const cplx *A, int nb, int n, int i0, int ib, size_t sv, cplx *V, hipStream_t s);
-int exc_launch_eig_tblock(const eig_kdesc *ks, const cplx *G, const cplx *tau, int nb, int n, int i0, int ib,
-                          size_t sgt, cplx *T, hipStream_t s);
+int exc_launch_eig_tblock(const eig_kdesc *ks, const cplx *A, const cplx *tau, int nb, int n, cplx *G, cplx *T,
+                          hipStream_t s);
 int exc_launch_eig_sort_r2c(const double *zr, int m, int nev, int ldr, const int *nfound, const double *w, cplx *x,
                             int ldx, double *eval, hipStream_t s);
+// tridiagonal reduction of a batch (k_trd.hip)
+size_t exc_trd_work_bytes(int n, int nb);
+int exc_launch_trd(int n, int nb, cplx *a, double *d, double *e, cplx *tau, void *work, hipStream_t s);
 int exc_launch_eig_copyout(const eig_kdesc *ks, int nb, int n, int nev, const cplx *x, hipStream_t s);
 // direct-route muffin-tin density (k_rhovalk.hip)
 size_t exc_rhovalk_work_bytes(const exc_dev &d, int lmaxvr, int nlomax, int nst);

@@ -110,47 +110,97 @@ __global__ __launch_bounds__(256) void eig_vblock_kernel(const cplx *A, int n, i
   V[(size_t)k * sv + r + (size_t)n * c] = v;
 }
 
-// T (ib x ib, lower triangular) of the block reflector H(i0+ib-1) ... H(i0) = I - V T V^H from
-// G = V^H V and tau (zlarft, direct 'B', storev 'C'): for i = ib-1 down to 0,
-// T(i, i) = tau_i, T(i+1:, i) = -tau_i T(i+1:, i+1:) G(i+1:, i).  The reflectors of k-point k
-// beyond its own order (i >= nmat_k - 1: the pad columns and the coupling column, zero
-// vectors) are left out (tau taken as 0).  One workgroup of kTB threads per k-point; thread
-// r owns row r of T.
+// G = V^H V (lower triangle) of every block of kTB reflectors of every k-point, V as above straight from A:
+// a 16 x 16 tile per workgroup, the rows split over its 4 waves (FP64 MFMA, operands from L2).  All blocks in one
+// launch: as a product per block, 64 x 64 results leave the chip idle for 20 of them in turn.
 constexpr int kTB = 64;
-__global__ __launch_bounds__(kTB) void eig_tblock_kernel(const eig_kdesc *ks, const cplx *G, const cplx *tau, int n,
-                                                         int i0, int ib, size_t sgt, cplx *T) {
-  const int k = blockIdx.x, r = threadIdx.x;
-  const int last = ks[k].n - 1;   // reflectors i0 + i < last are the k-point's
-  const cplx *g = G + (size_t)k * sgt;   // G and T of k-point k: leading dimension ib, at k * sgt
-  cplx *t = T + (size_t)k * sgt;
-  __shared__ double tre[kTB][kTB], tim[kTB][kTB];   // T(r, q) at [q][r]: row r is thread r's
-  __shared__ cplx tmp[kTB];
-  for (int q = 0; q < kTB; ++q) tre[q][r] = tim[q][r] = 0.0;
-  for (int i = ib - 1; i >= 0; --i) {
-    const cplx ti = i0 + i < last ? tau[(size_t)k * n + i0 + i] : czero();
-    if (r > i && r < ib) {   // tmp(r) = -tau_i G(r, i)
-      const cplx p = cmul(ti, g[r + ib * i]);
-      tmp[r] = {-p.re, -p.im};
-    }
-    __syncthreads();
-    if (r > i && r < ib) {   // T(r, i) = sum_{q = i+1}^{r} T(r, q) tmp(q)
-      double are = 0.0, aim = 0.0;
-      for (int q = i + 1; q <= r; ++q) {
-        const double xr = tre[q][r], xi = tim[q][r], yr = tmp[q].re, yi = tmp[q].im;
-        are += xr * yr - xi * yi;
-        aim += xr * yi + xi * yr;
-      }
-      tre[i][r] = are;
-      tim[i][r] = aim;
-    }
-    if (r == i) {
-      tre[i][i] = ti.re;
-      tim[i][i] = ti.im;
-    }
-    __syncthreads();
+__global__ __launch_bounds__(256) void eig_vhv_kernel(const cplx *A, int n, cplx *G) {
+  const int tile = blockIdx.x, nblk = gridDim.y, blk = blockIdx.y, k = blockIdx.z;
+  int ti = 0, tj = tile;                                   // ti >= tj, row by row
+  while (tj > ti) tj -= ++ti;
+  const int i0 = blk * kTB, ib = min(kTB, n - 1 - i0), mb = i0 + ib;
+  if (16 * ti >= ib) return;
+  __shared__ cplx red[4][4][64];
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int fi = i0 + min(16 * ti + li, ib - 1), fj = i0 + min(16 * tj + li, ib - 1);   // reflectors
+  const cplx *pi = A + (size_t)k * n * n + (size_t)n * (fi + 1), *pj = A + (size_t)k * n * n + (size_t)n * (fj + 1);
+  d4_t re = {0.0, 0.0, 0.0, 0.0}, im = re;
+#pragma unroll 4
+  for (int r0 = 4 * wave; r0 < mb; r0 += 16) {
+    const int r = r0 + lg, rc = min(r, mb - 1);
+    cplx x = pi[rc], y = pj[rc];
+    x = r < fi ? x : cplx{r == fi ? 1.0 : 0.0, 0.0};
+    y = r < fj ? y : cplx{r == fj ? 1.0 : 0.0, 0.0};
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.re, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.im, im, 0, 0, 0);
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.im, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(-x.im, y.re, im, 0, 0, 0);
   }
-  if (r < ib)
-    for (int q = 0; q < ib; ++q) t[r + (size_t)ib * q] = {tre[q][r], tim[q][r]};
+#pragma unroll
+  for (int v = 0; v < 4; ++v) red[v][wave][lane] = cplx{re[v], im[v]};
+  __syncthreads();
+  cplx s = {0.0, 0.0};
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    s.re += red[wave][w][lane].re;
+    s.im += red[wave][w][lane].im;
+  }
+  const int i = 16 * ti + 4 * wave + lg, j = 16 * tj + li;
+  if (i < ib && j < ib) G[((size_t)k * nblk + blk) * kTB * kTB + i + kTB * j] = s;
+}
+
+// T (ib x ib, lower triangular) of the block reflector H(i0+ib-1) ... H(i0) = I - V T V^H from
+// G = V^H V and tau (zlarft, direct 'B', storev 'C').  T^-1 has the diagonal 1 / tau_r and the lower
+// triangle of G, so column i of T is a forward substitution of its own:
+//   T(i, i) = tau_i,  T(r, i) = -tau_r sum_{i <= q < r} G(r, q) T(q, i).
+// The reflectors of k-point k beyond its own order (i >= nmat_k - 1: the pad columns and the
+// coupling column, zero vectors) are left out (tau taken as 0).  One workgroup per block and k-point: lane
+// i holds column i, its rows dealt to the 4 waves' registers, G in LDS.  A chain of ib sums either
+// way: 158 us a block by zlarft's order on one wave, 58 here, and all blocks in one launch.
+__global__ __launch_bounds__(4 * kTB) void eig_tblock_kernel(const eig_kdesc *ks, const cplx *G, const cplx *tau, int n,
+                                                             cplx *T) {
+  const int nblk = gridDim.x, blk = blockIdx.x, k = blockIdx.y, i = threadIdx.x & (kTB - 1);
+  const int i0 = blk * kTB, ib = min(kTB, n - 1 - i0);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kTB);
+  const int last = ks[k].n - 1;   // reflectors i0 + i < last are the k-point's
+  const cplx *g = G + ((size_t)k * nblk + blk) * kTB * kTB;
+  cplx *t = T + ((size_t)blk * gridDim.y + k) * kTB * kTB;   // a block's T of all k-points together
+  __shared__ cplx sg[kTB][kTB];          // G(r, q) at [q][r]
+  __shared__ cplx red[2][4][kTB], st[kTB];
+  for (int e = threadIdx.x; e < kTB * ib; e += 4 * kTB) sg[e / kTB][e % kTB] = g[e];
+  if (threadIdx.x < kTB) st[i] = i < ib && i0 + i < last ? tau[(size_t)k * n + i0 + i] : czero();
+  __syncthreads();
+  cplx col[kTB / 4];                     // T(4 j + wave, i)
+#pragma unroll
+  for (int j = 0; j < kTB / 4; ++j) col[j] = czero();
+#pragma unroll 1
+  for (int r = 0; r < ib; ++r) {
+    cplx s = {0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < kTB / 4; ++j)
+      if (4 * j + wave < r) {
+        const cplx p = cmul(sg[4 * j + wave][r], col[j]);
+        s.re += p.re;
+        s.im += p.im;
+      }
+    red[r & 1][wave][i] = s;
+    __syncthreads();
+    if ((r & 3) != wave) continue;
+    const cplx tr = st[r];
+    cplx v = {0.0, 0.0};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      v.re += red[r & 1][w][i].re;
+      v.im += red[r & 1][w][i].im;
+    }
+    v = cmul(tr, v);
+    v = i < r ? cplx{-v.re, -v.im} : i == r ? tr : czero();
+#pragma unroll
+    for (int j = 0; j < kTB / 4; ++j)
+      if (4 * j + wave == r) col[j] = v;
+    if (i < ib) t[r + kTB * i] = v;
+  }
 }
 
 // Eigenpairs of a tridiagonal matrix from bisection and inverse iteration (dstebz with eorder
@@ -229,11 +279,15 @@ int exc_launch_eig_vblock(const cplx *A, int nb, int n, int i0, int ib, size_t s
   return EXC_OK;
 }
 
-int exc_launch_eig_tblock(const eig_kdesc *ks, const cplx *G, const cplx *tau, int nb, int n, int i0, int ib,
-                          size_t sgt, cplx *T, hipStream_t s) {
-  if (nb <= 0 || ib <= 0) return EXC_OK;
-  if (ib > kTB || i0 + ib > n || sgt < (size_t)ib * ib) return EXC_ERR_ARG;
-  hipLaunchKernelGGL(eig_tblock_kernel, dim3(nb), dim3(kTB), 0, s, ks, G, tau, n, i0, ib, sgt, T);
+// T of every block of kTB reflectors: block b of k-point k at (b nb + k) kTB^2, leading dimension kTB; G: as much
+int exc_launch_eig_tblock(const eig_kdesc *ks, const cplx *A, const cplx *tau, int nb, int n, cplx *G, cplx *T,
+                          hipStream_t s) {
+  if (nb <= 0 || n < 2) return EXC_OK;
+  const int nblk = (n - 1 + kTB - 1) / kTB, t = kTB / 16;
+  if (nblk > 65535 || nb > 65535) return EXC_ERR_ARG;
+  hipLaunchKernelGGL(eig_vhv_kernel, dim3(t * (t + 1) / 2, nblk, nb), dim3(256), 0, s, A, n, G);
+  EXC_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(eig_tblock_kernel, dim3(nblk, nb), dim3(4 * kTB), 0, s, ks, G, tau, n, T);
   EXC_CHECK(hipGetLastError());
   return EXC_OK;
 }
