@@ -6,12 +6,13 @@
 // One workgroup of 8 or 16 waves per atom: the matrices (242 x 242 at lmax 10) are far too small to
 // spread over the chip, and a library solve of the whole batch spends its time on the ~1000
 // launches of its column steps and on eigenvectors nobody needs (8 atoms, naa 242: about 8 ms; here
-// 2.2 ms for the extremes and 0.37 for the factor).  Bound by one CU's path to L2 and by the chain of barriers.
+// 1.8 ms for the extremes and 0.37 for the factor).  Bound by one CU's path to L2 and by the chain of barriers.
 //  * gram_extremes_kernel: Householder tridiagonalization, then the smallest and the largest
-//    eigenvalue by Sturm counts of 128 points each at a time.  The rank-2 update of step j - 1
-//    is applied in the same pass over the trailing matrix that forms step j's matrix-vector
-//    product: one read and one write of it per step, both triangles, so that every access runs
-//    along columns and no sum crosses lanes.
+//    eigenvalue by Sturm counts of 128 points each at a time.  A step reads the trailing matrix once for
+//    its matrix-vector product, both triangles, so that every access runs along columns and no sum
+//    crosses lanes; the rank-2 updates wait in LDS, corrected for in the products, and are applied 8 at a
+//    time on the matrix cores (1.82 ms; 2.24 with each step's update applied in the next one's
+//    pass, a read and a write of the matrix a step).
 //  * gram_chol_kernel: left-looking by panels of 16 columns.
 #include "wave_sum.h"
 
@@ -41,15 +42,16 @@ __device__ __forceinline__ int sturm(int n, const double *d, const double *e2, d
 
 // R: 64-row chunks of n.  h: the upper triangles are read; m: n x n scratch per atom; ext[2 a]:
 // the smallest and largest eigenvalue of atom a (NaN where h is not finite)
-template <int R, int kGT = R <= 4 ? 1024 : 512>       // (the larger orders need the registers)
+template <int R, int kGT = R <= 4 ? 1024 : 512, int NB = R <= 4 ? 8 : 6>       // (the larger orders need the registers and LDS)
 __global__ __launch_bounds__(kGT) void gram_extremes_kernel(int n, const cplx *__restrict__ h, cplx *__restrict__ m,
                                                             double *__restrict__ ext) {
   constexpr int kGW = kGT / 64;
-  __shared__ cplx vp[64 * R], wp[64 * R], vn[64 * R];   // v, w of the last step, v of this one
+  __shared__ cplx pv[NB][64 * R], pw[NB][64 * R];       // v, w of the panel: the matrix lacks their updates
+  __shared__ cplx vn[64 * R];                           // v of this step
   __shared__ cplx red[kGW][64 * R];
-  __shared__ cplx col[64 * R];                          // the next column, short of the last step's update
+  __shared__ cplx col[64 * R];                          // the next column, short of the panel's updates
   __shared__ double d[64 * R], e2[64 * R], buf[2][kGW];
-  __shared__ cplx s_alpha;
+  __shared__ cplx s_alpha, sab[2 * NB];                 // w_q^H v, then v_q^H v
   __shared__ int cnt[2][2];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const cplx *H = h + (size_t)n * n * blockIdx.x;
@@ -61,16 +63,19 @@ __global__ __launch_bounds__(kGT) void gram_extremes_kernel(int n, const cplx *_
       M[i + (size_t)n * k] = x;
       if (k == 0) col[i] = x;
     }
-  for (int i = tid; i < 64 * R; i += kGT) vp[i] = wp[i] = cplx{0.0, 0.0};
   __syncthreads();
+  int p = 0;                                            // steps since the last update of the matrix
   for (int j = 0; j < n - 1; ++j) {
-    // column j with the last step's update, and its Householder vector (thread i: row i)
+    // column j with the panel's updates, and its Householder vector (thread i: row i)
     cplx x = {0.0, 0.0};
     if (tid >= j && tid < n) {
       x = col[tid];
-      const cplx v = vp[tid], w = wp[tid], vj = vp[j], wj = wp[j];
-      x.re -= v.re * wj.re + v.im * wj.im + w.re * vj.re + w.im * vj.im;
-      x.im -= v.im * wj.re - v.re * wj.im + w.im * vj.re - w.re * vj.im;
+#pragma unroll 2
+      for (int q = 0; q < p; ++q) {
+        const cplx v = pv[q][tid], w = pw[q][tid], vj = pv[q][j], wj = pw[q][j];
+        x.re -= v.re * wj.re + v.im * wj.im + w.re * vj.re + w.im * vj.im;
+        x.im -= v.im * wj.re - v.re * wj.im + w.im * vj.re - w.re * vj.im;
+      }
     }
     if (wave < R) {                                     // the waves that hold rows
       if (tid == j) d[j] = x.re;
@@ -79,46 +84,55 @@ __global__ __launch_bounds__(kGT) void gram_extremes_kernel(int n, const cplx *_
       if (lane == 0) buf[0][wave] = t;
     }
     __syncthreads();
-    double xn2 = 0.0;
+    cplx tau = {0.0, 0.0};
+    if (wave < R) {                                     // (the others would only take turns at the FP64 units)
+      double xn2 = 0.0;
 #pragma unroll
-    for (int w = 0; w < R; ++w) xn2 += buf[0][w];
-    const cplx al = s_alpha;
-    cplx tau = {0.0, 0.0}, sc = {0.0, 0.0};
-    double beta = al.re;
-    if (xn2 != 0.0 || al.im != 0.0) {
-      beta = -copysign(sqrt(al.re * al.re + al.im * al.im + xn2), al.re);
-      const double bi = 1.0 / beta;
-      tau = cplx{(beta - al.re) * bi, -al.im * bi};
-      const double dr = al.re - beta, di = al.im, q = 1.0 / (dr * dr + di * di);
-      sc = cplx{dr * q, -di * q};
+      for (int w = 0; w < R; ++w) xn2 += buf[0][w];
+      const cplx al = s_alpha;
+      cplx sc = {0.0, 0.0};
+      double beta = al.re;
+      if (xn2 != 0.0 || al.im != 0.0) {
+        beta = -copysign(sqrt(al.re * al.re + al.im * al.im + xn2), al.re);
+        const double bi = 1.0 / beta;
+        tau = cplx{(beta - al.re) * bi, -al.im * bi};
+        const double dr = al.re - beta, di = al.im, q = 1.0 / (dr * dr + di * di);
+        sc = cplx{dr * q, -di * q};
+      }
+      if (tid == 0) e2[j] = beta * beta;
+      vn[tid] = tid == j + 1 ? cplx{1.0, 0.0} : (tid > j + 1 && tid < n) ? cmul(x, sc) : cplx{0.0, 0.0};
     }
-    if (tid == 0) e2[j] = beta * beta;
-    if (tid < 64 * R) vn[tid] = tid == j + 1 ? cplx{1.0, 0.0} : (tid > j + 1 && tid < n) ? cmul(x, sc) : cplx{0.0, 0.0};
     __syncthreads();
-    // trailing matrix: last step's update, and this wave's columns' share of A v
-    cplx acc[R], va[R], wa[R];
+    // this wave's columns' share of A v
+    cplx acc[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      acc[r] = cplx{0.0, 0.0};
-      va[r] = vp[lane + 64 * r];
-      wa[r] = wp[lane + 64 * r];
-    }
-#pragma unroll 2
+    for (int r = 0; r < R; ++r) acc[r] = cplx{0.0, 0.0};
+#pragma unroll 4
     for (int k = j + 1 + wave; k < n; k += kGW) {
-      const cplx vk = vp[k], wk = wp[k], v = vn[k];
-      cplx *cl = M + (size_t)n * k;
+      const cplx v = vn[k];
+      const cplx *cl = M + (size_t)n * k;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int i = lane + 64 * r;
         if (64 * r + 63 <= j || i >= n) continue;       // rows above the trailing matrix: whole chunks skipped
-        cplx a = cl[i];
-        a.re = fma(-va[r].re, wk.re, fma(-va[r].im, wk.im, fma(-wa[r].re, vk.re, fma(-wa[r].im, vk.im, a.re))));
-        a.im = fma(-va[r].im, wk.re, fma(va[r].re, wk.im, fma(-wa[r].im, vk.re, fma(wa[r].re, vk.im, a.im))));
-        cl[i] = a;
+        const cplx a = cl[i];
         if (k == j + 1) col[i] = a;                     // wave 0's first column: the next step's
         acc[r].re = fma(a.re, v.re, fma(-a.im, v.im, acc[r].re));
         acc[r].im = fma(a.re, v.im, fma(a.im, v.re, acc[r].im));
       }
+    }
+    // the panel's products with v, one a wave
+    for (int t = wave; t < 2 * p; t += kGW) {
+      const cplx *b = t < p ? pw[t] : pv[t - p];
+      cplx s = {0.0, 0.0};
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const cplx y = b[lane + 64 * r], v = vn[lane + 64 * r];
+        s.re += y.re * v.re + y.im * v.im;
+        s.im += y.re * v.im - y.im * v.re;
+      }
+      s = cplx{wave_sum(s.re), wave_sum(s.im)};
+      if (lane == 0) sab[t] = s;
     }
     double vav = 0.0;                                   // this wave's share of v^H A v (real)
 #pragma unroll
@@ -130,31 +144,79 @@ __global__ __launch_bounds__(kGT) void gram_extremes_kernel(int n, const cplx *_
     vav = wave_sum(vav);
     if (lane == 0) buf[1][wave] = vav;
     __syncthreads();
-    // p = tau A v, w = p - 1/2 tau (p^H v) v with p^H v = conj(tau) v^H A v
+    // z = A v less the panel's updates of A, w = tau z - 1/2 |tau|^2 (v^H z) v
     if (tid < 64 * R) {
-      cplx p = {0.0, 0.0}, v = {0.0, 0.0};
+      cplx w = {0.0, 0.0}, v = {0.0, 0.0};
       if (tid > j && tid < n) {
         v = vn[tid];
+        cplx z = {0.0, 0.0};
+        double s = 0.0;
 #pragma unroll
-        for (int w = 0; w < kGW; ++w) {
-          p.re += red[w][tid].re;
-          p.im += red[w][tid].im;
+        for (int q = 0; q < kGW; ++q) {
+          z.re += red[q][tid].re;
+          z.im += red[q][tid].im;
+          s += buf[1][q];
         }
-        p = cmul(tau, p);
+#pragma unroll 2
+        for (int q = 0; q < p; ++q) {
+          const cplx a = sab[q], b = sab[p + q], x = pv[q][tid], y = pw[q][tid];
+          z.re -= x.re * a.re - x.im * a.im + y.re * b.re - y.im * b.im;
+          z.im -= x.re * a.im + x.im * a.re + y.re * b.im + y.im * b.re;
+          s -= 2.0 * (a.re * b.re + a.im * b.im);
+        }
+        const double hk = -0.5 * (tau.re * tau.re + tau.im * tau.im) * s;
+        w = cmul(tau, z);
+        w = cplx{fma(hk, v.re, w.re), fma(hk, v.im, w.im)};
       }
-      double s = 0.0;
+      pv[p][tid] = v;
+      pw[p][tid] = w;
+    }
+    __syncthreads();
+    if (++p < NB) continue;
+    // A -= V W^H + W V^H below and right of (j, j): the 16 x 16 tiles on and below the diagonal dealt to
+    // the waves, their conjugates stored above it
+    p = 0;
+    const int li = lane & 15, lg = lane >> 4, t0 = (j + 1) / 16, nt = (n + 15) / 16 - t0;
+    for (int tile = wave; tile < nt * (nt + 1) / 2; tile += kGW) {
+      int ti = (int)((sqrtf(8.0f * tile + 1.0f) - 1.0f) * 0.5f);   // ti >= tk, row by row
+      ti += (ti + 1) * (ti + 2) / 2 <= tile;
+      ti -= ti * (ti + 1) / 2 > tile;
+      const int tk = tile - ti * (ti + 1) / 2, k0 = 16 * (t0 + tk), i = 16 * (t0 + ti) + li;
+      cplx a[4];
 #pragma unroll
-      for (int w = 0; w < kGW; ++w) s += buf[1][w];
-      const double hk = -0.5 * (tau.re * tau.re + tau.im * tau.im) * s;
-      vp[tid] = v;
-      wp[tid] = cplx{fma(hk, v.re, p.re), fma(hk, v.im, p.im)};
+      for (int v = 0; v < 4; ++v) a[v] = M[min(i, n - 1) + (size_t)n * min(k0 + 4 * v + lg, n - 1)];
+      d4_t re = {0.0, 0.0, 0.0, 0.0}, im = re;
+#pragma unroll
+      for (int q0 = 0; q0 < NB; q0 += 4) {
+        const int q = min(q0 + lg, NB - 1);
+        const bool in = q0 + lg < NB;
+        auto mac = [&](cplx y, cplx x) {                // + x conj(y)
+          if (!in) x = y = cplx{0.0, 0.0};
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(y.re, x.re, re, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(y.re, x.im, im, 0, 0, 0);
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(y.im, x.im, re, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(-y.im, x.re, im, 0, 0, 0);
+        };
+        mac(pw[q][k0 + li], pv[q][i]);
+        mac(pv[q][k0 + li], pw[q][i]);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int k = k0 + 4 * v + lg;
+        if (i <= j || k <= j || i >= n || k >= n) continue;
+        const cplx x = {a[v].re - re[v], a[v].im - im[v]};
+        M[i + (size_t)n * k] = x;
+        if (k == j + 1) col[i] = x;
+        if (ti > tk) M[k + (size_t)n * i] = cplx{x.re, -x.im};
+      }
     }
     __syncthreads();
   }
   const int j = n - 1;
   if (tid == 0) {
-    const cplx v = vp[j], w = wp[j];
-    d[j] = col[j].re - 2.0 * (v.re * w.re + v.im * w.im);
+    double x = col[j].re;
+    for (int q = 0; q < p; ++q) x -= 2.0 * (pv[q][j].re * pw[q][j].re + pv[q][j].im * pw[q][j].im);
+    d[j] = x;
   }
   __syncthreads();
   // bounds (Gershgorin), and whether all is finite; 4 waves from here on
