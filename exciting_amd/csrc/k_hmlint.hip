@@ -6,8 +6,7 @@
 // the cubic spline of the product integrated interval by interval (fderiv.f90:64-72).  That
 // functional is linear in the sampled values, so it is a fixed weight vector per mesh,
 //     int f = sum_r wt_r f_r,
-// computed once on the host by the same spline recurrences (spline.f90:46-96) applied to the
-// unit vectors.  On the device:
+// computed on the host by the spline's recurrences (spline.f90:46-96) transposed.  On the device:
 //  * hml_radial_kernel, one workgroup per (atom, q): for q < lmmaxvr the potential integrals
 //    P_q(a, b) = sum_r wt_r r^2 V_q(r) u_a u_b (mt_pot.f90:142-212), q = lmmaxvr the kinetic
 //    ones K(a, b) = sum_r wt_r (1/2 u_a' u_b' r^2 + 1/2 l(l+1) u_a u_b) for l_a = l_b
@@ -67,10 +66,14 @@ __device__ __forceinline__ const double *radial_u(const HmlArgs &A, int atom, in
   return A.lofr + (size_t)A.nrmtmax * 2 * (ilo + (size_t)A.nlomax * atom);
 }
 
+// 16 x 16 tiles of the pairs (a, b) on the matrix cores, r split over the waves: 8 atoms, 26 functions, 500
+// points, lmaxvr 6 230 -> 54 us (a thread per pair, each walking the mesh before)
+static_assert(kHT == 256, "four waves");
 __global__ __launch_bounds__(kHT) void hml_radial_kernel(HmlArgs A) {
   const int q = blockIdx.x, atom = blockIdx.y;
   const int is = A.spidx[atom], nr = A.nrmt[is];
   extern __shared__ double sw[];   // [nr] weights of this block's integrand
+  __shared__ double red[2][4][4][64];
   const double *wt = A.wt + (size_t)A.nrmtmax * is, *x = A.spr + (size_t)A.nrmtmax * is;
   for (int r = threadIdx.x; r < nr; r += kHT) {
     const double r2 = x[r] * x[r];
@@ -82,25 +85,80 @@ __global__ __launch_bounds__(kHT) void hml_radial_kernel(HmlArgs A) {
   }
   __syncthreads();
   double *out = A.rad + ((size_t)atom * (A.lmv + 2) + q) * A.nf * A.nf;
-  for (int p = threadIdx.x; p < A.nf * A.nf; p += kHT) {
-    const int a = p / A.nf, b = p % A.nf;
-    int la = 0, lb = 0;
-    const double *ua = radial_u(A, atom, a, &la), *ub = radial_u(A, atom, b, &lb);
-    double s = 0.0;
-    if (ua && ub && (q != A.lmv || la == lb)) {
-      if (q == A.lmv) {
-        const double ang = 0.5 * la * (la + 1);
-        const double *dua = ua + A.nrmtmax, *dub = ub + A.nrmtmax;
-        for (int r = 0; r < nr; ++r) {
-          const double r2 = x[r] * x[r];
-          s = fma(sw[r], fma(0.5 * r2, dua[r] * dub[r], ang * (ua[r] * ub[r])), s);
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int per = (nr + 15) / 16 * 4, rb = wave * per, re = min(nr, rb + per);
+  // blocks of 32 x 32 pairs, I <= J: (2 I + i, 2 J + j) tiles of 16 functions, the one below the
+  // diagonal of a diagonal block left out
+  const int nblk = (A.nf + 31) / 32;
+  for (int I = 0; I < nblk; ++I)
+    for (int J = I; J < nblk; ++J) {
+      const bool diag = I == J;
+      const double *u[4];                                // functions 32 I + 16 t + li, then 32 J + ..., where there are
+      bool has[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        int l;
+        const int f = 32 * (t < 2 ? I : J) + 16 * (t & 1) + li;
+        u[t] = f < A.nf ? radial_u(A, atom, f, &l) : nullptr;
+        has[t] = u[t];
+        if (!has[t]) u[t] = A.apwfr;
+      }
+      // sums over this wave's r of weight u_a u_b, ofs 0: the functions, nrmtmax: their derivatives
+      // with 1/2 r^2
+      d4_t acc[2][4];
+      auto product = [&](d4_t *s, int ofs) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s[k] = d4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 8
+        for (int r0 = rb; r0 < re; r0 += 4) {
+          const int r = min(r0 + lg, nr - 1);
+          const bool in = r0 + lg < re;
+          double w = sw[r], y[4];
+          if (ofs) w *= 0.5 * (x[r] * x[r]);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) y[t] = t < 2 || !diag ? u[t][r + ofs] : y[t - 2];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) y[t] = in && has[t] ? y[t] : 0.0;
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              if (i <= j || !diag)
+                s[2 * i + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? w * y[i] : 0.0, y[2 + j], s[2 * i + j], 0, 0, 0);
         }
-      } else {
-        for (int r = 0; r < nr; ++r) s = fma(sw[r], ua[r] * ub[r], s);
+      };
+      product(acc[0], 0);
+      if (q == A.lmv) product(acc[1], A.nrmtmax);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        __syncthreads();                                 // the last tile's sums are read
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          red[0][v][wave][lane] = acc[0][k][v];
+          if (q == A.lmv) red[1][v][wave][lane] = acc[1][k][v];
+        }
+        __syncthreads();
+        // element 4 wave + lg of the rows, li of the columns; the lower triangle is the upper's mirror
+        const int a = 32 * I + 16 * (k >> 1) + 4 * wave + lg, b = 32 * J + 16 * (k & 1) + li;
+        if (a <= b && b < A.nf) {
+          double f = 0.0;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) f += red[0][wave][w][lane];
+          if (q == A.lmv) {
+            double g = 0.0;
+            int la = 0, lb = 0;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) g += red[1][wave][w][lane];
+            radial_u(A, atom, a, &la);
+            radial_u(A, atom, b, &lb);
+            f = la == lb ? fma(0.5 * la * (la + 1), f, g) : 0.0;
+          }
+          out[a * A.nf + b] = f;
+          out[b * A.nf + a] = f;
+        }
       }
     }
-    out[a * A.nf + b] = s;
-  }
 }
 
 // the Gaunt sum + kinetic term of one element; a1, a3 radial function indices
@@ -314,55 +372,51 @@ cplx gaunt_yry(int l1, int l2, int l3, int m1, int m2, int m3) {
 
 }  // namespace
 
-// Integration weights of fderiv(-1) on the mesh x (n >= 4 points): the spline recurrences run
-// on all n unit vectors at once (column j of the right-hand side is e_j).
+// Integration weights of fderiv(-1) on the mesh x (n >= 4 points): the integral of the spline is
+//   sum_i dx_i (f_i + f_{i+1}) / 2 - dx_i^3 / 12 (c2_i + c2_{i+1}),
+// linear in f, so its weights are the transposed recurrences of spline.f90 run backwards from the
+// coefficients of the c2: O(n).  (Run forwards on the n unit vectors, O(n^2), they took 0.5 ms of the
+// host for each species of 500 points, before anything of an SCF iteration could be launched.)
 void exc_hml_spline_weights(int n, const double *x, double *wt) {
-  std::vector<double> w(n), c1((size_t)n * n, 0.0), c3((size_t)n * n, 0.0), c2s(n);
-  auto F = [&](int i, int j) { return i == j ? 1.0 : 0.0; };
-  for (int i = 0; i < n - 1; ++i) {
-    w[i] = 1.0 / (x[i + 1] - x[i]);
-    for (int j = 0; j < n; ++j) c1[(size_t)i * n + j] = w[i] * (F(i + 1, j) - F(i, j));
-  }
-  c2s[0] = 1.0;
-  for (int j = 0; j < n; ++j) c3[j] = (c1[n + j] - c1[j]) / (x[2] - x[0]);
-  double t1 = (x[1] - x[0]) * w[1], t2 = t1 * c2s[0], t3 = 1.0 / (2.0 * (t1 + 1.0));
-  c2s[1] = t3;
-  std::vector<double> t4(n);
-  for (int j = 0; j < n; ++j) {
-    t4[j] = 3.0 * (c1[n + j] - c1[j]) * w[1] - t2 * c3[j];
-    c3[n + j] = t4[j];
-  }
+  std::vector<double> w(n - 1), c2s(n), t2(n), g(n, 0.0), c1(n - 1, 0.0);
+  for (int i = 0; i < n - 1; ++i) w[i] = 1.0 / (x[i + 1] - x[i]);
+  // the elimination's factors: r_i = 3 (c1_i - c1_{i-1}) w_i - t2_i r_{i-1}, c2_i = c2s_i s_i,
+  // s_i = r_i - c2s_{i+1} s_{i+1} (1 <= i < n - 1), s_0 = r_0, s_{n-1} = r_{n-1}
+  c2s[0] = c2s[n - 1] = 1.0;
+  double t1 = (x[1] - x[0]) * w[1];
+  t2[1] = t1;
+  c2s[1] = 1.0 / (2.0 * (t1 + 1.0));
   for (int i = 2; i < n - 1; ++i) {
     t1 = (x[i] - x[i - 1]) * w[i];
-    t2 = t1 * t3;
-    t3 = 1.0 / (2.0 * t1 + 2.0 - t2);
-    c2s[i] = t3;
-    for (int j = 0; j < n; ++j) {
-      t4[j] = 3.0 * (c1[(size_t)i * n + j] - c1[(size_t)(i - 1) * n + j]) * w[i] - t2 * t4[j];
-      c3[(size_t)i * n + j] = t4[j];
-    }
+    t2[i] = t1 * c2s[i - 1];
+    c2s[i] = 1.0 / (2.0 * t1 + 2.0 - t2[i]);
   }
-  c2s[n - 1] = 1.0;
-  std::vector<double> tb(n);
-  for (int j = 0; j < n; ++j) {
-    tb[j] = (c1[(size_t)(n - 2) * n + j] - c1[(size_t)(n - 3) * n + j]) / (x[n - 1] - x[n - 3]);
-    c3[(size_t)(n - 1) * n + j] = tb[j];
-  }
-  for (int i = n - 2; i >= 1; --i)
-    for (int j = 0; j < n; ++j) {
-      tb[j] = c3[(size_t)i * n + j] - tb[j] * c2s[i + 1];
-      c3[(size_t)i * n + j] = tb[j];
-    }
-  // c2 = c2s * c3; then c3, c1 of each interval, and the integral
-  for (int j = 0; j < n; ++j) wt[j] = 0.0;
+  // derivatives of the integral: by the c2 (times c2s: by the s), then by the r
   for (int i = 0; i < n - 1; ++i) {
-    const double dx = x[i + 1] - x[i];
-    for (int j = 0; j < n; ++j) {
-      const double c2i = c2s[i] * c3[(size_t)i * n + j], c2n = c2s[i + 1] * c3[(size_t)(i + 1) * n + j];
-      const double c3i = 0.3333333333333333333 * (c2n - c2i) * w[i];
-      const double c1i = c1[(size_t)i * n + j] - (c2i + c3i * dx) * dx;
-      wt[j] += (((0.25 * c3i * dx + 0.3333333333333333333 * c2i) * dx + 0.5 * c1i) * dx + F(i, j)) * dx;
-    }
+    const double dx = x[i + 1] - x[i], d = -dx * dx * dx / 12.0;
+    g[i] += d;
+    g[i + 1] += d;
+  }
+  for (int i = 0; i < n; ++i) g[i] *= c2s[i];
+  for (int i = 1; i < n - 1; ++i) g[i + 1] -= c2s[i + 1] * g[i];
+  // by the c1 (first differences of f times w)
+  const double ge = g[n - 1] / (x[n - 1] - x[n - 3]);
+  c1[n - 2] += ge;
+  c1[n - 3] -= ge;
+  for (int i = n - 2; i >= 1; --i) {
+    const double d = 3.0 * w[i] * g[i];
+    c1[i] += d;
+    c1[i - 1] -= d;
+    g[i - 1] -= t2[i] * g[i];
+  }
+  const double gb = g[0] / (x[2] - x[0]);
+  c1[1] += gb;
+  c1[0] -= gb;
+  for (int i = 0; i < n; ++i) wt[i] = 0.0;
+  for (int i = 0; i < n - 1; ++i) {
+    const double half = 0.5 * (x[i + 1] - x[i]), d = w[i] * c1[i];
+    wt[i] += half - d;
+    wt[i + 1] += half + d;
   }
 }
 
