@@ -220,7 +220,7 @@ int exc_ctx_set_variant(exc_ctx *c, int stage, int variant) {
   if (!c) return EXC_ERR_ARG;
   switch (stage) {
     case EXC_STAGE_YSTAGE:
-      if (variant < -1 || (variant >= kYstageVariants && (variant < kYWave1 || variant > kYDirect))) return EXC_ERR_ARG;
+      if (variant < -1 || (variant >= kYstageVariants && (variant < kYWave1 || variant > kYWave2))) return EXC_ERR_ARG;
       c->y_variant = variant;
       return EXC_OK;
     case EXC_STAGE_MT:
@@ -622,13 +622,14 @@ int mt_narrow(const exc_ctx *c, long tiles, int wide) {
   return 2 * tiles <= c->ncu ? kMtWave1 : 2 * tiles <= 5 * c->ncu ? kMtWave2 : wide;
 }
 
-// The Y stage by its 64 x 128 tiles: 16-wide up to a quarter of the CUs, 32-wide up to two per CU,
-// the 64-wide ones without LDS up to five per CU.  Measured (us; wide, 16-, 32-, 64-wide direct): 8
-// tiles (2 atoms, N = 97) 46, 8, 12, 26; 64 (8 k) 48, 22, 19, 27; 200 (5 atoms, N = 260, 4 k) 50, 51, 36, 47;
-// 400 (8 k) 83, 93, 63, 66; 560 (5 atoms, N = 400, 8 k) 178, 225, 150, 147; 1216 (8 atoms, N = 1200, 4 k)
-// 304, 564, 308, 275; 4864 (16 k) 1054, -, 1188, 1049; 10240 (16 atoms, N = 2500, 8 k) 2101, -, 2488, 2221.
+// The Y stage by its 64 x 128 tiles: 16-wide up to a quarter of the CUs, 32-wide up to 1.4 per CU,
+// beyond that 64 x 64 with BK 8 (variant 4: more workgroups a CU than the 64 x 128 tiles, and less
+// padding at naa = 162), per-k above five per CU `wide`.  Measured (us; 64 x 64, 16-, 32-wide): 8 tiles (2 atoms,
+// N = 97) 46, 8, 12; 64 (8 k) 48, 22, 19; 200 (5 atoms, N = 260, 4 k) 45, 51, 37; 400 (8 k) 63, 93, 64; 880 (N =
+// 700, 8 k) 117, -, 130; (64 x 64, 64 x 128): 1216 (8 atoms, N = 1200, 4 k) 263, 285; 4864 (16 k) 977, 1014;
+// 10240 (16 atoms, N = 2500, 8 k) 2204, 2218; 20224 (32 atoms, N = 5000, 4 k) 4070, 4138.
 int y_narrow(const exc_ctx *c, long tiles, int wide) {
-  return 4 * tiles <= c->ncu ? kYWave1 : tiles <= 2 * c->ncu ? kYWave2 : tiles <= 5 * c->ncu ? kYDirect : wide;
+  return 4 * tiles <= c->ncu ? kYWave1 : 10 * tiles <= 14 * c->ncu ? kYWave2 : tiles <= 5 * c->ncu ? 4 : wide;
 }
 
 // Whether an FP64 batch's muffin-tin products conj(A) Yt^T run as exact integer products (k_crt.hip:
@@ -910,7 +911,7 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   }
   const int bv = split ? (c->bsplit_variant >= 0 ? c->bsplit_variant : 3)
                        : (c->bmt_variant >= 0 ? c->bmt_variant : mt_narrow(c, mtiles, 0));
-  const int yv = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, 0);   // 64x128 Y tiles, DMA-staged, 3 products
+  const int yv = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, 4);   // 64x64 Y tiles, DMA-staged, 3 products
   // residue GEMM: the register-pipelined 256 x 256 form from N = 2048, 128 x 128 tiles below
   int maxn = 0;
   for (int k = 0; k < nk; ++k) maxn = std::max(maxn, ks[k].ngp);
@@ -946,11 +947,7 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   }
   const int kp = exc_crt_kpad(c->d.natm * c->d.naa);
   // batch signature: descriptors, flags and variants
-  // the Gram form's E stage on its triangular table: narrow column tiles skip more of it
-  // (64 x 64 three-product tiles, 5.7 against 6.7 ms at workload 3; the dense Y stage keeps
-  // 64 x 128, 8.8 against 9.1 ms)
-  const int ye = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, 4);
-  int tail[9] = {nk, flags, bv, yv, icrt || exact ? cv : -1, (icrt || exact ? nmod : -1) + 100 * ov, fv, gram, ye};
+  int tail[8] = {nk, flags, bv, yv, icrt || exact ? cv : -1, (icrt || exact ? nmod : -1) + 100 * ov, fv, gram};
   std::vector<char> sig(sizeof(exc_kpoint_dev) * nk + sizeof(tail));
   memcpy(sig.data(), ks, sizeof(exc_kpoint_dev) * nk);
   memcpy(sig.data() + sizeof(exc_kpoint_dev) * nk, tail, sizeof(tail));
@@ -1210,7 +1207,7 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
         dy.haa = (cplx *)gram_t;
         dy.ytri = 1;
       }
-      if ((r = exc_launch_bystage(dy, nk, c->batch_maxngp, c->d_ks, gram ? ye : yv, c->stream))) return r;
+      if ((r = exc_launch_bystage(dy, nk, c->batch_maxngp, c->d_ks, yv, c->stream))) return r;
     }
     // the Gram form's merge reads O's APW block: the overlap runs before it
     const bool olp_first = gram && !fork;

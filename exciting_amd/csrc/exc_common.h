@@ -126,9 +126,8 @@ constexpr int kYstageVariants = 5;   // per-k and grouped Y stage (the same shap
 constexpr int kMtVariants = 3;       // per-k MT
 constexpr int kBmtVariants = 4;      // grouped MT
 // the tiles of mt_wave.h (per-k and grouped), chosen by the built-in rules at small sizes: 16 and
-// 32 wide with the sum split over the waves, and 64 wide without (Y stage); they sum in another
-// order than the variants counted above
-constexpr int kYWave1 = 16, kYWave2 = 17, kYDirect = 18, kMtWave1 = 16, kMtWave2 = 17;
+// 32 wide with the sum split over the waves; they sum in another order than the variants counted above
+constexpr int kYWave1 = 16, kYWave2 = 17, kMtWave1 = 16, kMtWave2 = 17;
 // the overlap kernel the default takes (not one of the numbered variants)
 constexpr int kOlpBcast = 16;
 // Grouped launches over nk k-points described by ks (device memory); maxngp bounds the grids.

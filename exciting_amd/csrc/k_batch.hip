@@ -173,25 +173,6 @@ int launch_bmt_wave_t(const exc_dev &d, const kdesc *ks, const mt_item *items, i
   return EXC_OK;
 }
 
-// one 32 x 32 block per wave, operands straight to registers (mt_wave.h)
-__global__ __launch_bounds__(256, 2) void bystage_direct_kernel(const kdesc *__restrict__ ks, int natm, int naa,
-                                                                const cplx *__restrict__ haa,
-                                                                const int *__restrict__ fperm, int tri) {
-  const int ias = blockIdx.z % natm;
-  const kdesc k = ks[blockIdx.z / natm];
-  const int row0 = blockIdx.x * 64, col0 = blockIdx.y * 64;
-  if (row0 >= k.ngp) return;
-  YTileDirect::run(k.ngp, naa, k.apwalm + (size_t)k.ldg * naa * ias, k.ldg, haa + (size_t)naa * naa * ias,
-                   k.yt + (size_t)k.ldy * naa * ias, k.ldy, row0, col0, fperm, tri ? min(col0, naa) : 0);
-}
-
-int launch_bystage_direct(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hipStream_t s) {
-  hipLaunchKernelGGL(bystage_direct_kernel, dim3((maxngp + 63) / 64, (d.naa + 63) / 64, d.natm * nk), dim3(256), 0, s, ks,
-                     d.natm, d.naa, d.haa, d.fperm, d.ytri);
-  EXC_CHECK(hipGetLastError());
-  return EXC_OK;
-}
-
 template <int MAXLO>
 __global__ __launch_bounds__(lo_dev::kThreads) void blo_kernel(
     const kdesc *__restrict__ ks, int naa, int maxnlo, int nlomax, int apwordmax, int nlotot,
@@ -236,7 +217,7 @@ int exc_launch_bmatch(const exc_dev &d, int nk, int maxngp, const kdesc *ks, hip
   }
 }
 
-// Y-stage variants: as the per-k Y stage's (exc_launch_ystage); 0 is the grouped default
+// Y-stage variants: as the per-k Y stage's (exc_launch_ystage); 4 is the grouped default at large sizes
 int exc_launch_bystage(const exc_dev &d, int nk, int maxngp, const kdesc *ks, int variant, hipStream_t s) {
   if (nk <= 0 || maxngp <= 0) return EXC_OK;
   switch (variant) {
@@ -247,20 +228,20 @@ int exc_launch_bystage(const exc_dev &d, int nk, int maxngp, const kdesc *ks, in
     case 4: return launch_bystage_dma_t<64, 64, 8, 2, 2, 4, true>(d, nk, maxngp, ks, s);   // narrow, Gauss's form
     case kYWave1: return launch_bystage_wave_t<1>(d, nk, maxngp, ks, s);
     case kYWave2: return launch_bystage_wave_t<2>(d, nk, maxngp, ks, s);
-    case kYDirect: return launch_bystage_direct(d, nk, maxngp, ks, s);
     default: return EXC_ERR_ARG;
   }
 }
 
 int exc_bmt_tile(int variant) { return variant == kMtWave1 ? 16 : variant == kMtWave2 ? 32 : 64; }
 
-// grouped MT variants: 64 x 64 tile, 8 waves; 0: BK 16, two DMA stages, Gauss's three real
-// products per complex product (the default); 1: the same with four products; 2: BK 8, four
+// grouped MT variants: 64 x 64 tile, 8 waves; 0: BK 8, two DMA stages, Gauss's three real products per
+// complex product (the default; three workgroups a CU fit its LDS, where BK 16's two wait more at their
+// barriers: 8 atoms, N = 1200, 16 k-points 2.67 ms, 2.76 with BK 16); 1: BK 16, four products; 2: BK 8, four
 // stages, three products; 3: BK 16, three stages, three products
 int exc_launch_bmt(const exc_dev &d, const kdesc *ks, const mt_item *items, int nitems, int variant, hipStream_t s) {
   if (nitems <= 0) return EXC_OK;
   switch (variant) {
-    case 0: return launch_bmt_dma_grid_t<64, 16, 2, 2, 4, true>(d, ks, items, nitems, s);
+    case 0: return launch_bmt_dma_grid_t<64, 8, 2, 2, 4, true>(d, ks, items, nitems, s);
     case 1: return launch_bmt_dma_grid_t<64, 16, 2, 2, 4>(d, ks, items, nitems, s);
     case 2: return launch_bmt_dma_grid_t<64, 8, 4, 2, 4, true>(d, ks, items, nitems, s);
     case 3: return launch_bmt_dma_grid_t<64, 16, 3, 2, 4, true>(d, ks, items, nitems, s);

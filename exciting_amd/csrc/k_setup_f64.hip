@@ -89,22 +89,6 @@ int launch_ystage_wave_t(const exc_dev &d, int ngp, const cplx *apwalm, int ldg,
   return EXC_OK;
 }
 
-__global__ __launch_bounds__(256, 2) void ystage_direct_kernel(int ngp, int naa, const cplx *__restrict__ apwalm,
-                                                               int ldg, const cplx *__restrict__ haa,
-                                                               cplx *__restrict__ yt, int ldy,
-                                                               const int *__restrict__ fperm) {
-  const int ias = blockIdx.z;
-  YTileDirect::run(ngp, naa, apwalm + (size_t)ldg * naa * ias, ldg, haa + (size_t)naa * naa * ias,
-                   yt + (size_t)ldy * naa * ias, ldy, blockIdx.x * 64, blockIdx.y * 64, fperm, 0);
-}
-
-int launch_ystage_direct(const exc_dev &d, int ngp, const cplx *apwalm, int ldg, cplx *yt, int ldy, hipStream_t s) {
-  hipLaunchKernelGGL(ystage_direct_kernel, dim3((ngp + 63) / 64, (d.naa + 63) / 64, d.natm), dim3(256), 0, s, ngp, d.naa,
-                     apwalm, ldg, d.haa, yt, ldy, d.fperm);
-  EXC_CHECK(hipGetLastError());
-  return EXC_OK;
-}
-
 template <int TB>
 __global__ __launch_bounds__(256) void mt_wave_kernel(int ngp, int ktot, const cplx *__restrict__ apwalm, int ldg,
                                                       const cplx *__restrict__ yt, int ldy,
@@ -146,7 +130,6 @@ int exc_launch_ystage(const exc_dev &d, int ngp, const cplx *apwalm, int ldg, cp
     case 4: return launch_ystage_dma_t<64, 64, 8, 2, 2, 4, true>(d, ngp, apwalm, ldg, yt, ldy, s);
     case kYWave1: return launch_ystage_wave_t<1>(d, ngp, apwalm, ldg, yt, ldy, s);
     case kYWave2: return launch_ystage_wave_t<2>(d, ngp, apwalm, ldg, yt, ldy, s);
-    case kYDirect: return launch_ystage_direct(d, ngp, apwalm, ldg, yt, ldy, s);
     default: return EXC_ERR_ARG;
   }
 }

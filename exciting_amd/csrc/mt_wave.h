@@ -203,32 +203,6 @@ struct MtTileWave {
   }
 };
 
-// one 64 x 64 tile of Yt_a with the waves 2 x 2 over the tile, each its 32 x 32 over all of k: the
-// 64-wide tile without LDS, operands shared between the waves through the CU's L1
-struct YTileDirect {
-  using C = WaveCore<2, false>;
-  __device__ static void run(int ngp, int naa, const cplx *__restrict__ A, int ldg, const cplx *__restrict__ ha,
-                             cplx *__restrict__ Y, int ldy, int row0, int col0, const int *__restrict__ fperm,
-                             int kfirst) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    row0 += 32 * (wave >> 1);
-    col0 += 32 * (wave & 1);
-    if (row0 >= ngp || col0 >= naa) return;
-    d4_t cr[2][2], ci[2][2];
-    C::sum(ha, naa, col0, naa, A, ldg, row0, ngp, naa - kfirst, 0, naa - kfirst, fperm + kfirst, cr, ci);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int e = 4 * (2 * i + j) + v;
-          const int c = col0 + C::row_of(e), r = row0 + C::col_of(e);
-          if (r < ngp && c < naa) Y[r + (size_t)c * ldy] = cplx{cr[i][j][v], ci[i][j][v]};
-        }
-  }
-};
-
 // one tile of Yt_a = A_a h_a^T, the tile's rows (basis functions) along the lanes; kfirst as in
 // YTileDMA
 template <int TB>
