@@ -456,6 +456,21 @@ int rhoir_run(exc_ctx *c, int nk, const int *ngp, const int *const *igpig, int n
   if ((rc = scf_prepare(c))) return rc;
   const exc_dev &d = c->d;
   const int N = c->dims.ngrtot;
+  if (exc_rhoir_fits(d)) {                     // the FFT below: a grid whose DFT matrices do not fit in LDS
+    if (!c->dft) {
+      std::vector<cplx> t((size_t)d.box_n[0] * d.box_n[0] + (size_t)d.box_n[1] * d.box_n[1] +
+                          (size_t)d.box_n[2] * d.box_n[2]);
+      exc_rhoir_tables(d, t.data());
+      cplx *p = nullptr;
+      if ((rc = dev_alloc(c, &p, t.size()))) return rc;
+      EXC_CHECK(hipMemcpyAsync(p, t.data(), sizeof(cplx) * t.size(), hipMemcpyHostToDevice, c->stream));
+      EXC_CHECK(hipStreamSynchronize(c->stream));
+      c->dft = p;
+    }
+    if ((rc = grow((void **)&c->zb, &c->zb_bytes, exc_rhoir_work_bytes(d, nk, nst, c->ncu)))) return rc;
+    StageTimer t(c, EXC_STAGE_SCF);
+    return exc_launch_rhoir(d, nk, ngp, igpig, nst, ldv, evec, occ, wkpt, epsocc, c->dft, c->zb, rhoir, c->ncu, c->stream);
+  }
   // states per transform: nearly equal chunks (200 states: 4 of 50, not 3 of 64 and one of 64 for 8)
   const int nch = (nst + kRhoirChunk - 1) / kRhoirChunk, B = (nst + nch - 1) / nch;
   if ((rc = grow((void **)&c->zb, &c->zb_bytes, sizeof(cplx) * (size_t)B * N))) return rc;

@@ -245,6 +245,12 @@ int exc_launch_rhoir_scatter(const exc_dev &d, int ngp, const int *igpig, const 
                              int N, cplx *z, hipStream_t s);
 int exc_launch_rhoir_accum(int N, int nb, const cplx *z, const double *occ, int j0, double wk, double eps,
                            double omega, double *rho, hipStream_t s);
+bool exc_rhoir_fits(const exc_dev &d);
+size_t exc_rhoir_work_bytes(const exc_dev &d, int nk, int nst, int ncu);
+void exc_rhoir_tables(const exc_dev &d, cplx *f);
+int exc_launch_rhoir(const exc_dev &d, int nk, const int *ngp, const int *const *igpig, int nst, const int *ldv,
+                     const double *const *evec, const double *const *occ, const double *wkpt, double eps, const cplx *tab,
+                     void *work, double *rho, int ncu, hipStream_t s);
 int exc_launch_lo(const exc_dev &d, int ngp, const cplx *apwalm, int ldg, cplx *h, cplx *o, int ldh,
                   hipStream_t s);
 int exc_launch_iora_apw(const exc_dev &d, int ngp, const cplx *apwalm, int ldg, cplx *out, int ldo, hipStream_t s);

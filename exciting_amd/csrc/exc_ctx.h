@@ -154,8 +154,9 @@ struct exc_ctx {
   // work array, Theta(r) on the grid, a staging array for V(r)
   hipfftHandle fft;
   bool have_fft, have_cfunir;
-  hipfftHandle fftb;          // batched backward FFT of genrhoir, fftb_n transforms per call
+  hipfftHandle fftb;          // batched backward FFT of genrhoir on large grids, fftb_n transforms per call
   int fftb_n;
+  cplx *dft;                  // the DFT matrices of the grid's edges (k_rhoir.hip), made at genrhoir's first call
   cplx *zb;
   size_t zb_bytes;
   cplx *fz;
