@@ -197,7 +197,8 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   const size_t o_if = o_is + (bisect ? al(4 * (size_t)n * nb) : 0);
   const size_t o_si = o_if + (bisect ? al(4 * (size_t)n * nb) : 0);
   const size_t o_tr = o_si + (bisect ? al(16 * (size_t)nb) : 0);
-  const size_t total = o_tr + (bisect ? 0 : al(exc_trd_work_bytes(n, nb)));
+  const size_t o_ch = o_tr;         // (the factorization is over before the tridiagonal reduction begins)
+  const size_t total = o_tr + (bisect ? 0 : al(std::max(exc_trd_work_bytes(n, nb), exc_chol_work_bytes(n, nb))));
   int rc;
   if ((rc = grow(&c->eg, &c->eg_bytes, total))) return rc;
   char *base = (char *)c->eg;
@@ -240,8 +241,10 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
     const rocblas_stride sw = (rocblas_stride)kBT * nev, sxx = (rocblas_stride)n * nev;
     const int ib = std::min(kBT, std::max(n - 1, 1));
     if ((rc = pin_workspace(c->ew[0], [&]() {
-           rocsolver_zpotrf_strided_batched(hb, up, n, B, n, sm, info, nb);
-           rocsolver_ztrtri_strided_batched(hb, up, nu, n, B, n, sm, info + nb, nb);
+           if (bisect) {
+             rocsolver_zpotrf_strided_batched(hb, up, n, B, n, sm, info, nb);
+             rocsolver_ztrtri_strided_batched(hb, up, nu, n, B, n, sm, info + nb, nb);
+           }
            rocblas_ztrmm_strided_batched(hb, rocblas_side_right, up, N, nu, n, n, &one, B, n, sm, A, n, sm, Z, n, sm, nb);
            rocblas_ztrmm_strided_batched(hb, rocblas_side_left, up, CT, nu, n, n, &one, B, n, sm, Z, n, sm, A, n, sm, nb);
            if (bisect)
@@ -281,14 +284,20 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   StageTimer t(c, EXC_STAGE_EIGEN);
   EXC_CHECK(hipMemcpyAsync(dkd, kd.data(), sizeof(eig_kdesc) * nb, hipMemcpyHostToDevice, c->stream));
   if ((rc = exc_launch_eig_pad(dkd, nb, n, ph, po, 1.0, c->stream))) return rc;
-  // O = U^H U for every k-point; checked before anything reads the factors
-  rocblas_status st = rocsolver_zpotrf_strided_batched(hb, up, n, B, n, sm, info, nb);
-  if (st != rocblas_status_success) return fail("zpotrf_strided_batched status", (int)st, n);
+  // O = U^H U for every k-point, checked before anything reads the factors; U^-1 in O's place (k_chol.hip;
+  // variant 7 keeps the library's, as its reduction below)
+  rocblas_status st = rocblas_status_success;
+  if (!bisect) {
+    if ((rc = exc_launch_chol_inverse(n, nb, po, info, base + o_ch, c->stream))) return rc;
+  } else {
+    st = rocsolver_zpotrf_strided_batched(hb, up, n, B, n, sm, info, nb);
+    if (st != rocblas_status_success) return fail("zpotrf_strided_batched status", (int)st, n);
+  }
   EXC_CHECK(hipMemcpyAsync(hi.data(), info, sizeof(int) * nb, hipMemcpyDeviceToHost, c->stream));
   EXC_CHECK(hipStreamSynchronize(c->stream));
   for (int b = 0; b < nb; ++b)
     if (hi[b] > 0) return hi[b] <= kd[b].n ? kd[b].n + hi[b] : fail("pad not positive definite", b, hi[b]);
-  st = rocsolver_ztrtri_strided_batched(hb, up, nu, n, B, n, sm, info + nb, nb);   // U^-1
+  if (bisect) st = rocsolver_ztrtri_strided_batched(hb, up, nu, n, B, n, sm, info + nb, nb);   // U^-1
   if (st == rocblas_status_success)   // Z = H U^-1
     st = rocblas_ztrmm_strided_batched(hb, rocblas_side_right, up, rocblas_operation_none, nu, n, n, &one, B, n, sm,
                                        A, n, sm, Z, n, sm, nb);
@@ -394,7 +403,7 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   EXC_CHECK(hipMemcpyAsync(hi.data(), info, sizeof(int) * 3 * nb, hipMemcpyDeviceToHost, c->stream));
   EXC_CHECK(hipStreamSynchronize(c->stream));
   for (int b = 0; b < nb; ++b) {
-    if (hi[nb + b] != 0) return fail("ztrtri info", b, hi[nb + b]);   // of a positive definite factor
+    if (bisect && hi[nb + b] != 0) return fail("ztrtri info", b, hi[nb + b]);   // of a positive definite factor
     if (!bisect && hi[2 * nb + b] != 0) return hi[2 * nb + b];      // eigenvalues that did not converge
   }
   if (bisect) {   // per k-point: eigenvalues found, split blocks, dstebz info, dstein info

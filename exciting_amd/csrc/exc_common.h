@@ -205,6 +205,8 @@ int exc_launch_eig_tblock(const eig_kdesc *ks, const cplx *A, const cplx *tau, i
 int exc_launch_eig_sort_r2c(const double *zr, int m, int nev, int ldr, const int *nfound, const double *w, cplx *x,
                             int ldx, double *eval, hipStream_t s);
 // tridiagonal reduction of a batch (k_trd.hip)
+size_t exc_chol_work_bytes(int n, int nb);
+int exc_launch_chol_inverse(int n, int nb, cplx *a, int *info, void *work, hipStream_t s);
 size_t exc_trd_work_bytes(int n, int nb);
 int exc_launch_trd(int n, int nb, cplx *a, double *d, double *e, cplx *tau, void *work, hipStream_t s);
 int exc_launch_eig_copyout(const eig_kdesc *ks, int nb, int n, int nev, const cplx *x, hipStream_t s);
