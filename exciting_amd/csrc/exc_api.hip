@@ -636,15 +636,15 @@ int y_narrow(const exc_ctx *c, long tiles, int wide) {
 // 16 moduli, operands as 57-bit integers of their row's scale, so that the only roundings are
 // the operands' and the result's: against 80-bit sums the error is an eighth to a third of the
 // FP64 MFMA tiles') instead of on FP64 MFMA.  Per k-point the MFMA tiles take 5.5e-8 K N^2 us, the
-// exact products 2.1e-8 K N^2 (residue GEMM) + 2.4e-5 K N (planes of both operands) + 1.3e-5 N^2
-// (reconstruction), K = natm naa: even near 700 / N + 650 / K = 1, with a margin for the tails of
+// exact products 1.7e-8 K N^2 (residue GEMM) + 2.4e-5 K N (planes of both operands) + 1.3e-5 N^2
+// (reconstruction), K = natm naa: even near 700 / N + 650 / K = 1.1, with a margin for the tails of
 // smaller grids.  Measured for the whole grouped setup, graph replays (us; MFMA, exact; the left
-// side): K = 1452, N = 1000, 16 k-points 2274, 2440 (1.15); 1936, 1200, 16 k 4149, 4015-4159 (0.92);
-// 7744, 900, 2 k 1618, 1460 (0.86); 2904, 1200, 4 k 1633, 1542 (0.81); 1452, 2000, 8 k 3794, 3271 (0.80);
-// 1936, 1600, 16 k 6519, 6033 (0.77); 2420, 1600, 8 k 4036, 3632 (0.71); 5808, 1200, 2 k 1725, 1501 (0.70); 2904,
-// 1900, 8 k 6596, 5478 (0.59); 3872, 2500, 8 k 13738, 10400 (0.45); 7744, 5000, 4 k 46263, 26800 (0.22).
+// side): K = 1936, N = 700, 8 k-points 1098, 1081-1113 (1.34); 1452, 1100, 4 k 781, 815 (1.08); 1620, 1000, 8 k
+// 1338, 1260 (1.10); 1936, 1200, 4 k 1029, 1027-1040 (0.92); 1936, 1200, 16 k 4167, 3965 (0.92); 2904, 1200, 4 k 1516,
+// 1433 (0.81); 1936, 1600, 16 k 6537, 5812 (0.77); 5808, 1200, 2 k 1898, 1430 (0.70); 2904, 1900, 8 k 6425, 4939
+// (0.59); 3872, 2500, 8 k 14299, 9601 (0.45).
 bool exact_pays(const exc_ctx *c, int maxn) {
-  return maxn > 0 && 700.0 / maxn + 650.0 / ((double)c->d.natm * c->d.naa) <= 0.88;
+  return maxn > 0 && 700.0 / maxn + 650.0 / ((double)c->d.natm * c->d.naa) <= 0.97;
 }
 
 constexpr size_t kExactPlanes = (size_t)24 << 30;   // residue planes of the k-points in the workspace at a time
@@ -904,21 +904,25 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   // defaults: the fastest variants measured on MI355X for N = 1150..5000 (grouped MT: 64x64
   // tile, 8 waves, two LDS stages filled by DMA, one item per workgroup; split: 64x64 tile,
   // LDS filled by DMA)
-  long mtiles = 0, ytiles = 0;
+  long mtiles = 0, ytiles = 0, t128 = 0, t256 = 0;
   for (int k = 0; k < nk; ++k) {
     mtiles += tri_tiles(ks[k].ngp, 64);
+    t128 += tri_tiles(ks[k].ngp, 128);
+    t256 += 4 * tri_tiles(ks[k].ngp, 256);
     ytiles += (long)((ks[k].ngp + 63) / 64) * ((c->d.naa + 127) / 128) * c->d.natm;
   }
   const int bv = split ? (c->bsplit_variant >= 0 ? c->bsplit_variant : 3)
                        : (c->bmt_variant >= 0 ? c->bmt_variant : mt_narrow(c, mtiles, 0));
   const int yv = c->y_variant >= 0 ? c->y_variant : y_narrow(c, ytiles, 4);   // 64x64 Y tiles, DMA-staged, 3 products
-  // residue GEMM: the register-pipelined 256 x 256 form from N = 2048, 128 x 128 tiles below
+  // residue GEMM: the register-pipelined 256 x 256 form from N = 800 unless its tiles cover over a quarter more
+  // than 128 x 128 ones (us of a split setup, 128, 256: K = 1936, N = 1200, 8 k-points 1234, 1204, 900, 1 k 207, 197, 500, 8 k
+  // 500, 514; 2904, 1900, 8 k 3492, 3296; 1296, 1100, 16 k, a third more, 1548, 1594)
   int maxn = 0;
   for (int k = 0; k < nk; ++k) maxn = std::max(maxn, ks[k].ngp);
   // the FP64 path by exact integer products (its O tiles take no 'iora*' terms)
   bool exact = !split && !icrt && c->bmt_variant < 0 && c->d.natm * c->d.naa <= 131000 && !(c->d.iora && !olp) &&
                exact_pays(c, maxn);
-  const int cv = c->crt_variant >= 0 ? c->crt_variant : (maxn >= 2048 ? 8 : 4);
+  const int cv = c->crt_variant >= 0 ? c->crt_variant : (maxn >= 800 && 4 * t256 <= 5 * t128 ? 8 : 4);
   const int ov = c->olp_variant >= 0 ? c->olp_variant : kOlpBcast;   // rows along lanes, columns by DPP broadcast
   int fv = c->fork_variant;
   // the modular split's Gram form: needs O_APW from the addition theorem, equal to A's Gram

@@ -366,10 +366,13 @@ __global__ __launch_bounds__(64 * WR * WC, MINW) void crt_gemm_kernel(const kdes
 // the LDS latency, the fragments of MFMA k-step s + 1 are read while the MFMAs of step s run
 // (two register sets), and the workgroup barrier that hands an LDS stage over to the DMA is
 // taken once per stage, at its last k-step, after its last fragments are in registers:
-//   wait for the next stage's DMA | barrier | read its first fragments | DMA into the stage
-//   just finished | MFMAs of the last k-step
-// so that the next stage's first fragments are in flight during those MFMAs.  Same
+//   wait for the next stage's DMA | barrier | read its first fragments | half of the DMA into the stage
+//   just finished (the other half during the next stage's first k-step) | MFMAs of the last k-step
+// so that the next stage's first fragments are in flight during those MFMAs, and a DMA follows every
+// fourth MFMA: issued together, the wave waits at the full queue of the L1 instead.  Same
 // products, same integer sums, same output layout as crt_gemm_kernel with a 2 x 2 wave grid.
+// N = 5000, 32 atoms, 8 k-points, 10 moduli: MFMA alone takes 10.3 ms (1.8 GHz: power), the DMA alone 9.1,
+// with the buffers chosen at run time both in turn 19.2, here 15.0; N = 2500, 16 atoms, 16 moduli 4.84 -> 3.70.
 // ---------------------------------------------------------------------------------------
 template <int BT, int BK, int NST, int WR, int WC>
 __device__ __forceinline__ void gemm_frags(const typename GemmCfg<BT, BK, NST, WR, WC>::Stage *st, int s,
@@ -400,7 +403,7 @@ __device__ __forceinline__ void gemm_mfma(const v4i (&af)[GemmCfg<BT, BK, NST, W
 // the L wave-wide DMAs of one stage from per-slot sources fixed for the tile (slot q: panel,
 // 16-byte chunk, 64-row quarter), `off` bytes further along k: no address arithmetic at the
 // hand-over beyond one add per slot
-template <int BT, int BK, int NST, int WR, int WC>
+template <int BT, int BK, int NST, int WR, int WC, int Q0, int Q1>
 __device__ __forceinline__ void gemm_issue_pre(typename GemmCfg<BT, BK, NST, WR, WC>::Stage *st, const unsigned char *pak,
                                                const unsigned char *pbk,
                                                const unsigned (&voff)[GemmCfg<BT, BK, NST, WR, WC>::L],
@@ -408,7 +411,7 @@ __device__ __forceinline__ void gemm_issue_pre(typename GemmCfg<BT, BK, NST, WR,
   using C = GemmCfg<BT, BK, NST, WR, WC>;
   static_assert((C::NL / 2) % C::kWaves == 0, "slot q of every wave in one panel");
 #pragma unroll
-  for (int q = 0; q < C::L; ++q)
+  for (int q = Q0; q < Q1; ++q)
     __builtin_amdgcn_global_load_lds((const void *)((q * C::kWaves >= C::NL / 2 ? pbk : pak) + voff[q]),
                                      (lds_void *)((unsigned char *)st + doff[q]), 16, 0, 0);
 }
@@ -421,7 +424,8 @@ __global__ __launch_bounds__(64 * WR * WC, 1) void crt_gemm_pipe_kernel(const kd
   using C = GemmCfg<BT, BK, NST, WR, WC>;
   using St = typename C::Stage;
   constexpr int S = BK / 32;                    // MFMA k-steps per stage
-  static_assert(S % 2 == 0 && NST >= 2 && NST <= 4, "register sets alternate within a stage; LDS size");
+  constexpr int D = C::L / S;                   // DMA slots per k-step
+  static_assert(S == 2 && C::L % S == 0 && NST >= 2 && NST <= 4, "register sets alternate within a stage; LDS size");
   EXC_DMA_STAGES(St, NST)
   const int chunk = (nwork + 7) / 8;
   const int x = blockIdx.x % 8, qb = blockIdx.x / 8;
@@ -463,14 +467,14 @@ __global__ __launch_bounds__(64 * WR * WC, 1) void crt_gemm_pipe_kernel(const kd
     }
   }
   const size_t sstride = (size_t)C::KC * chunk_stride;       // bytes of k per stage
-  // stage j's DMA is issued at the hand-over of stage j - NST (stages 0 .. NST-2 here, NST-1
-  // at the first hand-over below); stages past the end load the last one again (never read),
+  // stage j's DMA is issued from the hand-over of stage j - NST on (stages 0 .. NST-2 here, the first
+  // half of NST-1 at the first hand-over below); stages past the end load the last one again (never read),
   // so that exactly NST - 2 stages' DMA after the next one is in flight at every hand-over
   const size_t klast = (size_t)(nsteps - 1) * sstride;
 #pragma unroll
   for (int u = 0; u < NST - 1; ++u) {
     const size_t o = std::min((size_t)u * sstride, klast);
-    gemm_issue_pre<BT, BK, NST, WR, WC>(st[u], pa + o, pb + o, voff, doff);
+    gemm_issue_pre<BT, BK, NST, WR, WC, 0, C::L>(st[u], pa + o, pb + o, voff, doff);
   }
   v4i fa[2][C::MI], fb[2][C::NJ];
   // hand-over before stage 0
@@ -479,50 +483,51 @@ __global__ __launch_bounds__(64 * WR * WC, 1) void crt_gemm_pipe_kernel(const kd
   gemm_frags<BT, BK, NST, WR, WC>(st[0], 0, fa[0], fb[0], wr, wc);
   {
     const size_t o = std::min((size_t)(NST - 1) * sstride, klast);
-    gemm_issue_pre<BT, BK, NST, WR, WC>(st[NST - 1], pa + o, pb + o, voff, doff);
+    gemm_issue_pre<BT, BK, NST, WR, WC, 0, D>(st[NST - 1], pa + o, pb + o, voff, doff);
   }
-  // one stage per iteration, its LDS buffer chosen at run time, and no branch inside: the
-  // accumulators never flow through one (they would be copied between register files), and
-  // the scheduler can put one fragment read and one DMA between two MFMAs.  The last stage
-  // hands over too (its reads unused).
-  size_t koff = (size_t)(NST - 1) * sstride;    // k offset of the DMA at the next hand-over, less one stage
-#pragma unroll 1
-  for (int step = 0; step < nsteps; ++step) {
-    const int u = step % NST;
-    const int un = u + 1 < NST ? u + 1 : 0;
+  // no branch around an MFMA: the accumulators never flow through one (they would be copied between
+  // register files), and the scheduler can put one fragment read and one DMA between two MFMAs.  The
+  // last stage hands over too (its reads unused).
+  size_t koff = std::min((size_t)(NST - 1) * sstride, klast);   // k offset of stage min(step + NST - 1, nsteps - 1)
+  auto stage = [&](St *cs, St *ns, St *ps) __attribute__((always_inline)) {
+    const size_t kprev = koff;
     koff = koff + sstride < klast ? koff + sstride : klast;    // stage min(step + NST, nsteps - 1)
-    // (selects, not an indexed array: a run-time index into an array of LDS addresses would
-    // make it a static table)
-    St *const cs = u == 0 ? &s0_ : (u == 1 ? &s1_ : (u == 2 ? (St *)&s2_ : (St *)&s3_));
-    St *const ns = un == 0 ? &s0_ : (un == 1 ? &s1_ : (un == 2 ? (St *)&s2_ : (St *)&s3_));
+    // 16 MFMAs, a fragment read after each of the first eight, a DMA after every fourth
+    auto order = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      __builtin_amdgcn_sched_barrier(0);
-      if (s + 1 < S) {
-        gemm_frags<BT, BK, NST, WR, WC>(cs, s + 1, fa[(s + 1) & 1], fb[(s + 1) & 1], wr, wc);
-        gemm_mfma<BT, BK, NST, WR, WC>(fa[s & 1], fb[s & 1], acc);
-#pragma unroll
-        for (int q = 0; q < C::MI + C::NJ; ++q) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-      } else {
-        // hand-over: stage step + 1 has landed once at most the DMA of the NST - 2 stages
-        // after it is out
-        wait_vm_lgkm0<(NST - 2) * C::L>();
-        stage_barrier();
-        gemm_frags<BT, BK, NST, WR, WC>(ns, 0, fa[0], fb[0], wr, wc);
-        gemm_issue_pre<BT, BK, NST, WR, WC>(cs, pa + koff, pb + koff, voff, doff);
-        gemm_mfma<BT, BK, NST, WR, WC>(fa[s & 1], fb[s & 1], acc);
-#pragma unroll
-        for (int q = 0; q < C::MI + C::NJ; ++q) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          if (q < C::L) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-        }
+      for (int q = 0; q < C::MI * C::NJ; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (q < C::MI + C::NJ) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (q % 4 == 2 && q / 4 < D) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
       }
-    }
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    gemm_frags<BT, BK, NST, WR, WC>(cs, 1, fa[1], fb[1], wr, wc);
+    gemm_issue_pre<BT, BK, NST, WR, WC, D, C::L>(ps, pa + kprev, pb + kprev, voff, doff);
+    gemm_mfma<BT, BK, NST, WR, WC>(fa[0], fb[0], acc);
+    order();
+    __builtin_amdgcn_sched_barrier(0);
+    // hand-over: stage step + 1 has landed once at most the DMA of the NST - 2 stages after it is out
+    wait_vm_lgkm0<(NST - 2) * C::L>();
+    stage_barrier();
+    gemm_frags<BT, BK, NST, WR, WC>(ns, 0, fa[0], fb[0], wr, wc);
+    gemm_issue_pre<BT, BK, NST, WR, WC, 0, D>(cs, pa + koff, pb + koff, voff, doff);
+    gemm_mfma<BT, BK, NST, WR, WC>(fa[1], fb[1], acc);
+    order();
+  };
+  // the stages rotate by name: with a buffer chosen at run time the compiler cannot tell the fragment
+  // reads from the DMA in flight into another stage and drains it before each stage's reads
+  // (s_waitcnt vmcnt(0): load and MFMA then took turns)
+  int step = 0;
+#pragma unroll 1
+  for (; step + NST <= nsteps; step += NST) {
+#pragma unroll
+    for (int u = 0; u < NST; ++u) stage(st[u], st[(u + 1) % NST], st[(u + NST - 1) % NST]);
   }
+  // the last nsteps % NST of them
+  if (step < nsteps) stage(st[0], st[1], st[NST - 1]);
+  if (NST > 2 && step + 1 < nsteps) stage(st[1], st[2], st[0]);
+  if (NST > 3 && step + 2 < nsteps) stage(st[2], st[3], st[1]);
   wait_vm_lgkm0<0>();                            // no DMA into this workgroup's LDS outlives it
   const int m = t.m[l];
   const double mi = t.dminv[l];
