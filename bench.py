@@ -111,6 +111,15 @@ def crt_alg_ops(cr, ngps, nmod, share):
     return sum(2.0 * 2 * nmod * K * n * (n + 1) / 2 for n in ngps) * (2 * share)
 
 
+def crt_gemm_name(ngps, pinned=None):
+    """The residue GEMM that runs: variants 8 to 10 are the register-pipelined kernel on 256-wide tiles, which
+    the library takes by itself from N = 800 unless they cover over a quarter more than 128-wide ones."""
+    def tiles(t):
+        return sum(-(-n // t) * (-(-n // t) + 1) // 2 for n in ngps)
+    v = pinned if pinned is not None else (8 if max(ngps) >= 800 and 16 * tiles(256) <= 5 * tiles(128) else 4)
+    return "crt_gemm_pipe_kernel" if v in (8, 9, 10) else "crt_gemm_kernel"
+
+
 def run_split(args, ctx, batch, cr, w, fp64_value, e0, log, olpflag=0, kind="crt"):
     """The split-precision leg: the muffin-tin contraction from exact integer residue products
     (kind 'crt', EXC_BATCH_SPLIT_CRT: the library's form and moduli count unless --moduli
@@ -168,10 +177,7 @@ def run_split(args, ctx, batch, cr, w, fp64_value, e0, log, olpflag=0, kind="crt
         form, nmod, sigma = ctx.crt_form()
         ms = eager["crtgemm"][0]
         ops = crt_alg_ops(cr, ngps, nmod, share)
-        # variants 8-10 are the register-pipelined kernel; the library's default by basis size
-        # (the tuned table pins one for every workload here)
-        v = (tuned or {}).get("crtgemm", 8 if max(ngps) >= 2048 else 4)
-        gname = "crt_gemm_pipe_kernel" if v in (8, 9, 10) else "crt_gemm_kernel"
+        gname = crt_gemm_name(ngps, (tuned or {}).get("crtgemm"))
         roof = {"bound": "mfma", "kernel": f"{gname} (residue products, {nmod} moduli, int8 MFMA)",
                 "achieved": ops / (ms * 1e-3) / 1e12, "peak": PEAK_INT8 / 1e12, "unit": "TOP/s",
                 "frac": ops / (ms * 1e-3) / PEAK_INT8, "fp64_equivalent_TFLOPs": fl64 / (ms * 1e-3) / 1e12,
@@ -246,8 +252,8 @@ def run_eigen(args, ctx, batch, w, olpflag, nev, log):
     dmat = run_dmat(args, ctx, batch, w, nev, vecs, log)
     return {"value": value, "unit": "k-points/s", "nev": nev, "ms_per_step": 1000.0 * dt / steps, "steps": steps,
             "eigensolve_ms_per_k": ms_eig / max(cnt, 1),
-            "solver": "rocSOLVER: k-points padded to one order, strided-batched Cholesky, inverse, reduction and "
-                      "tridiagonalization; per-k divide and conquer on 4 streams; back-transform of "
+            "solver": "k-points padded to one order; Cholesky factor with inverse and tridiagonal reduction of the whole "
+                      "batch, rocBLAS products; per-k rocSOLVER divide and conquer on 4 streams; back-transform of "
                       "all k-points by 64-reflector blocks (strided-batched GEMMs)",
             "variants": tuned, "cpu_lapack_zhegvx_ms_per_k": cpu_ms, "density_matrix": dmat}
 
@@ -653,10 +659,21 @@ def main():
                       + (", 3 real MFMA products per complex product" if gauss else ""),
             "per_launch_flops": fl / max(mt_cnt, 1),
             "executed_mfma_frac": (0.75 if gauss else 1.0) * achieved / PEAK_FP64}
+    # large bases: the FP64 path forms the contraction from exact integer products (16 moduli, operands as 57-bit
+    # integers of their row's scale) by the residue GEMM; its error against 80-bit sums is below FP64 MFMA's
+    exact = args.path == "batched" and eager["crtgemm"][1] > 0
+    if exact:
+        ngps = [kp.ngp for kp in w.kpoints]
+        gemm_ms, ops = eager["crtgemm"][0], crt_alg_ops(cr, ngps, 16, share)
+        roof = {"bound": "mfma", "kernel": f"{crt_gemm_name(ngps)} (FP64 contraction as exact integer products, 16 "
+                                           "moduli, int8 MFMA)",
+                "achieved": ops / (gemm_ms * 1e-3) / 1e12, "peak": PEAK_INT8 / 1e12, "unit": "TOP/s",
+                "frac": ops / (gemm_ms * 1e-3) / PEAK_INT8, "traffic": None, "per_launch_ops": ops,
+                "fp64_equivalent_TFLOPs": fl / (gemm_ms * 1e-3) / 1e12}
     # HBM traffic of the dominant kernel: rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of this same
     # default command, scaled by a 1 GiB copy (committed summary); only for the profiled setup
     prof = HERE / "profiles" / f"setup_kernels_workload{args.config}.json"
-    if (args.path == "batched" and args.nk is None and not args.tune and not args.set and olpflag
+    if (args.path == "batched" and not exact and args.nk is None and not args.tune and not args.set and olpflag
             and prof.exists()):
         rec = json.loads(prof.read_text()).get("bmt_dma_grid_kernel")
         if rec:
@@ -694,6 +711,7 @@ def main():
         "config": {"workload": f"workload {args.config}: " + WORKLOAD_NAMES[args.config], "k_points": nk,
                    "path": ("FP64, all k-points grouped per stage, hipGraph replay"
                             + (", overlap MT part by the addition theorem" if olpflag else "")
+                            + (", H's MT contraction by exact integer products" if exact else "")
                             if args.path == "batched" else "FP64, per-k launches"
                             + (", host arrays (PCIe copies included)" if args.path == "host" else "")),
                    "parallelism": "single GPU", "variants": tuned},

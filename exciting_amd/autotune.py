@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import json
 import os
+import time
 from pathlib import Path
 from typing import Callable, Dict, Optional
 
@@ -61,12 +62,29 @@ def sweep(ctx, stage: str, run: Callable[[], None], reps: int = 3, log=None) -> 
     return out
 
 
+def _whole(ctx, stage, variant, run, reps) -> float:
+    """ms of a whole run with `stage` at `variant` (-1: the library's rule by size)."""
+    import torch
+    ctx.set_variant(stage, variant)
+    run()
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    for _ in range(reps):
+        run()
+    torch.cuda.synchronize()
+    return 1000.0 * (time.perf_counter() - t0) / reps
+
+
 def tune(ctx, stages, run: Callable[[], None], reps: int = 3, log=None) -> Dict[str, int]:
-    """Sweep each stage in turn (others at their current setting) and pin the fastest variant."""
+    """Sweep each stage in turn (others at their current setting) and pin the fastest variant, or leave the
+    library's own rule (-1) where the whole run is no slower with it: the rule may take another route
+    altogether (the contraction as exact integer products), which the stage's own timer does not see."""
     chosen = {}
     for st in stages:
         res = sweep(ctx, st, run, reps, log)
         best = min(res, key=res.get)
+        if _whole(ctx, st, -1, run, reps) <= _whole(ctx, st, best, run, reps):
+            best = -1
         ctx.set_variant(st, best)
         chosen[st] = best
         if log:
@@ -75,12 +93,13 @@ def tune(ctx, stages, run: Callable[[], None], reps: int = 3, log=None) -> Dict[
 
 
 def save(path: os.PathLike, key, chosen: Dict[str, int]):
-    """Merge `chosen` into the table's entry for `key` (stages it does not name are kept)."""
+    """Merge `chosen` into the table's entry for `key` (stages it does not name are kept, those left to the
+    library's rule, -1, taken out)."""
     table = {}
     if os.path.exists(path):
         with open(path) as f:
             table = json.load(f)
-    table[str(key)] = {**table.get(str(key), {}), **chosen}
+    table[str(key)] = {st: v for st, v in {**table.get(str(key), {}), **chosen}.items() if v >= 0}
     with open(path, "w") as f:
         json.dump(table, f, indent=1, sort_keys=True)
 
