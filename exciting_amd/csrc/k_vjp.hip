@@ -17,7 +17,7 @@
 // lines need D and W over pairs only through their sums per G_i - G_j = g: dw_kernel adds
 // D_ji and dp_ij D_ji + W_ji of the upper triangle into per-g sums (the other triangle is the
 // conjugate at -g), theta_kernel then walks the few 10^4 g instead of every pair for every atom.
-// Measured, 16 atoms, N = 2500, 64 states (us): U 102, back 95, h_a U 21, dw 165, theta 12, the rest 25;
+// Measured, 16 atoms, N = 2500, 64 states (us): U 90, back 95, h_a U 21, dw 165, theta 12, the rest 25;
 // with a q-scaled library product for each direction, U and V_l together 320, the contraction
 // per (atom, state) 119 and the pairs times all atoms with four atomics each 788.
 #include "setup_dev.h"
@@ -204,7 +204,9 @@ __device__ __forceinline__ void dw_add(const DwOut &o, const GTab &gt, int d0, i
   }
 }
 
-__global__ __launch_bounds__(256) void dw_kernel(int ngp, int nst, const cplx *__restrict__ ch,
+// (two workgroups a CU: left to itself the compiler takes 284 registers and one fits; a pass of the 16-atom case at
+// N = 2500, two k-points, 587 -> 577 us.  Bound by the LDS atomics of the sums.)
+__global__ __launch_bounds__(256, 2) void dw_kernel(int ngp, int nst, const cplx *__restrict__ ch,
                                                  const cplx *__restrict__ cf, const cplx *__restrict__ cg,
                                                  const int *__restrict__ perm, const int *__restrict__ igpig,
                                                  const double *__restrict__ vgpc, GTab gt, int ax, DwOut o) {
