@@ -971,6 +971,7 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   }
   if (!same) {
     // new batch: lay out the Y workspace, descriptors and the muffin-tin work list
+    c->batch_sig.clear();   // until the layout is whole: one that fails may have freed what the last batch's tables name
     EXC_CHECK(hipStreamSynchronize(c->stream));   // earlier launches may still read the old tables
     if (c->graph_exec) {
       hipGraphExecDestroy(c->graph_exec);

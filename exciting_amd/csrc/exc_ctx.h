@@ -272,7 +272,13 @@ inline int grow(void **p, size_t *have, size_t need) {
   }
   *p = nullptr;
   *have = 0;
-  EXC_CHECK(hipMalloc(p, need));
+  const hipError_t e = hipMalloc(p, need);
+  if (e != hipSuccess) {
+    hipGetLastError();                    // reported here: the next launch's check must not find it again
+    *p = nullptr;
+    fprintf(stderr, "exc_lapw: %zu bytes of workspace: %s\n", need, hipGetErrorString(e));
+    return EXC_ERR_HIP;
+  }
   *have = need;
   return EXC_OK;
 }
