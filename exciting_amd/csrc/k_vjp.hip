@@ -355,8 +355,9 @@ __global__ __launch_bounds__(256) void theta_kernel(const double *__restrict__ s
         re += s[m - 1];
         im -= s[nv + m - 1];
       }
-      dedv[2 * g] += re;
-      dedv[2 * g + 1] += im;
+      // atomic: calls on other streams may be adding their k-points to the same array
+      if (re != 0.0) atomicAdd(dedv + 2 * g, re);
+      if (im != 0.0) atomicAdd(dedv + 2 * g + 1, im);
     }
     const unsigned long long pair = rep[g];
     if (pair != ~0ull) {
