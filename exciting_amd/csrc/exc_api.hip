@@ -289,6 +289,12 @@ int exc_ctx_crt_form(const exc_ctx *c, int *form, int *nmod, double *sigma) {
   return EXC_OK;
 }
 
+int exc_ctx_exact_products(const exc_ctx *c, int *exact) {
+  if (!c || !exact) return EXC_ERR_ARG;
+  *exact = c->batch_exact ? 1 : 0;
+  return EXC_OK;
+}
+
 int exc_crt_moduli(int n, int *moduli, int *beta) {
   if (n < 8 || n > kCrtMaxUsed || !moduli || !beta) return EXC_ERR_ARG;
   CrtTab t;
@@ -580,8 +586,8 @@ int exc_match(exc_ctx *c, int ngp, int ngkmax, const double *gpc, const double *
   const size_t na = c->d.natm, lmm = c->d.lmmaxapw, ao = c->d.apwordmax, nk = ngkmax;
   const size_t b_gpc = 8 * nk, b_tp = 16 * nk, b_sf = 16 * nk * na, b_apw = 16 * nk * ao * lmm * na;
   c->apw_res_valid = false;
-  if ((rc = grow(&c->stage, &c->stage_bytes, b_gpc + b_tp + b_sf))) return rc;
-  if ((rc = grow((void **)&c->apw_res, &c->apw_res_bytes, b_apw ? b_apw : 1))) return rc;
+  if ((rc = grow(c, &c->stage, &c->stage_bytes, b_gpc + b_tp + b_sf))) return rc;
+  if ((rc = grow(c, (void **)&c->apw_res, &c->apw_res_bytes, b_apw ? b_apw : 1))) return rc;
   char *base = (char *)c->stage;
   double *d_gpc = (double *)base;
   double *d_tp = (double *)(base + b_gpc);
@@ -647,8 +653,6 @@ bool exact_pays(const exc_ctx *c, int maxn) {
   return maxn > 0 && 700.0 / maxn + 650.0 / ((double)c->d.natm * c->d.naa) <= 0.97;
 }
 
-constexpr size_t kExactPlanes = (size_t)24 << 30;   // residue planes of the k-points in the workspace at a time
-
 long tri_tiles(int ngp, int t) {
   const long n = (ngp + t - 1) / t;
   return n * (n + 1) / 2;
@@ -658,26 +662,55 @@ long tri_tiles(int ngp, int t) {
 int crt_rows(int ngp) { return (ngp + 255) / 256 * 256; }
 size_t crt_plane_bytes(int ngp, int nmod, int kp) { return (size_t)2 * nmod * kp * crt_rows(ngp); }
 
-// Whether the exact products' workspace (planes of one group of k-points, their residues) is
-// there or fits well into the free device memory; if not the batch runs on FP64 MFMA
-int exact_fits(exc_ctx *c, int nk, const exc_kpoint_dev *ks, bool olp, int cv, int nmod, int kp, bool *fits) {
+// Groups of k-points that share the residue planes and residues, as many in each as `limit` bytes
+// hold (at least one), from `ops` operands' planes and residues of `which` matrices on bt-wide
+// tiles a k-point; the largest planes and residues of a group
+void crt_group(exc_ctx *c, int nk, const exc_kpoint_dev *ks, size_t limit, int ops, int which, int bt, int nmod, int kp,
+               size_t *planes, size_t *residues) {
+  size_t q = 0, r = 0;
+  *planes = *residues = 0;
+  c->crt_groups.clear();
+  for (int k = 0; k < nk; ++k) {
+    const size_t b = ops * crt_plane_bytes(ks[k].ngp, nmod, kp);
+    const size_t t = (size_t)tri_tiles(ks[k].ngp, bt) * which * nmod * 2 * bt * bt;
+    if (k == 0 || q + r + b + t > limit) {
+      c->crt_groups.push_back({k, 0, 0, 0, 0, 0, 0});
+      q = r = 0;
+    }
+    c->crt_groups.back().nk += 1;
+    q += b;
+    r += t;
+    *planes = std::max(*planes, q);
+    *residues = std::max(*residues, r);
+  }
+}
+
+// The exact products' planes and residues: up to 4 GiB of them and an eighth of the free device
+// memory (with what the context holds of them already), but at least one k-point's.  How many
+// k-points share them does not change a bit of H; the chip is full from a few on.  Replays in ms with all
+// k-points in one group, 4, 2 and 1 GiB: 8 atoms, N = 1200, 16 k-points 3.88, 3.96, 4.07, 4.11; 16 atoms,
+// N = 2500, 8 k 9.27, 9.35, 9.61, 10.16; 32 atoms, N = 5000, 4 k 24.61, 25.09, 25.26, 25.25.  Where one
+// k-point's would be more than half of the free memory, or cannot be had, the batch runs on FP64
+// MFMA (exc_ctx_exact_products tells).  Called with crt_held set, `was` its value before.
+constexpr size_t kExactBytes = (size_t)4 << 30;
+
+int exact_workspace(exc_ctx *c, int nk, const exc_kpoint_dev *ks, bool olp, int cv, int nmod, int kp, bool was,
+                    bool *fits) {
   int bt = 0, wr = 0, wc = 0;
   *fits = false;
   if (exc_crt_shape(cv, &bt, &wr, &wc)) return EXC_OK;
-  size_t q = 0, r = 0, qmax = 0, rmax = 0;
-  for (int k = 0; k < nk; ++k) {
-    const size_t b = 2 * crt_plane_bytes(ks[k].ngp, nmod, kp);
-    if (q && q + b > kExactPlanes) q = r = 0;
-    q += b;
-    r += (size_t)tri_tiles(ks[k].ngp, bt) * (olp ? 1 : 2) * nmod * 2 * bt * bt;
-    qmax = std::max(qmax, q);
-    rmax = std::max(rmax, r);
+  const int which = olp ? 1 : 2;
+  size_t fr = 0, total = 0, q = 0, r = 0;
+  crt_group(c, nk, ks, 0, 2, which, bt, nmod, kp, &q, &r);                  // one k-point each
+  EXC_CHECK(hipMemGetInfo(&fr, &total));
+  fr += c->crt_q_bytes + c->crt_res_bytes;
+  if (q + r > fr / 2) return EXC_OK;
+  crt_group(c, nk, ks, std::min(kExactBytes, fr / 8), 2, which, bt, nmod, kp, &q, &r);
+  *fits = !grow(c, &c->crt_q, &c->crt_q_bytes, q) && !grow(c, (void **)&c->crt_res, &c->crt_res_bytes, r);
+  if (!*fits) {
+    c->crt_held = was;
+    give_back(c);
   }
-  size_t need = 0, fr = 0, total = 0;
-  if (qmax > c->crt_q_bytes) need += qmax;
-  if (rmax > c->crt_res_bytes) need += rmax;
-  if (need) EXC_CHECK(hipMemGetInfo(&fr, &total));
-  *fits = !need || need < fr - fr / 4;
   return EXC_OK;
 }
 
@@ -705,7 +738,7 @@ int setup_dev_sel(exc_ctx *c, int ngp, int ngkmax, const double *apwalm, const i
     if (h) {   // the Y stage feeds only H
       if (!ws) {
         const size_t need = sizeof(cplx) * (size_t)ngp * c->d.naa * c->d.natm;
-        if ((rc = grow((void **)&c->yt, &c->yt_bytes, need))) return rc;
+        if ((rc = grow(c, (void **)&c->yt, &c->yt_bytes, need))) return rc;
         yt = c->yt;
       }
       StageTimer t(c, untimed ? -1 : EXC_STAGE_YSTAGE);
@@ -717,7 +750,7 @@ int setup_dev_sel(exc_ctx *c, int ngp, int ngkmax, const double *apwalm, const i
       if ((c->d.iora & 1) && o) {
         // 'iora*': O's tiles take the operand A L, H's keep A (two launches)
         if (ws) return EXC_ERR_UNSUPPORTED;
-        if ((rc = grow((void **)&c->apwo, &c->apwo_bytes, sizeof(cplx) * (size_t)ngp * c->d.naa * c->d.natm)))
+        if ((rc = grow(c, (void **)&c->apwo, &c->apwo_bytes, sizeof(cplx) * (size_t)ngp * c->d.naa * c->d.natm)))
           return rc;
         rc = exc_launch_iora_apw(c->d, ngp, (const cplx *)apwalm, ngkmax, c->apwo, ngp, c->stream);
         if (!rc && h)
@@ -753,7 +786,7 @@ int setup_host_sel(exc_ctx *c, int ngp, int ngkmax, const double *apwalm, const 
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t o_ig = al(b_apw), o_vg = o_ig + al(b_ig), o_h = o_vg + al(b_vg);
   const size_t o_o = o_h + (h ? al(b_h) : 0);
-  if ((rc = grow(&c->stage, &c->stage_bytes, o_o + (o ? b_h : 0)))) return rc;
+  if ((rc = grow(c, &c->stage, &c->stage_bytes, o_o + (o ? b_h : 0)))) return rc;
   const int nout = (h ? 1 : 0) + (o ? 1 : 0);
   if ((rc = grow_host(&c->hstage, &c->hstage_bytes, std::max(b_apw, nout * b_h)))) return rc;
   char *base = (char *)c->stage;
@@ -789,7 +822,7 @@ int gram_build(exc_ctx *c) {
   // the table, scratch, then (read back together) the extremes, sigma and the infos
   const size_t o_w = al(sizeof(cplx) * nn), o_x = o_w + al(sizeof(cplx) * nn);
   const size_t b_x = 8 * (2 * (size_t)na + 1) + 4 * (size_t)na;
-  int rc = grow(&c->gram_buf, &c->gram_bytes, o_x + b_x);
+  int rc = grow(c, &c->gram_buf, &c->gram_bytes, o_x + b_x);
   if (rc) return rc;
   char *b = (char *)c->gram_buf;
   double *ext = (double *)(b + o_x);
@@ -956,14 +989,12 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   memcpy(sig.data(), ks, sizeof(exc_kpoint_dev) * nk);
   memcpy(sig.data() + sizeof(exc_kpoint_dev) * nk, tail, sizeof(tail));
   const bool same = (sig == c->batch_sig);
-  if (exact) {
-    if (same) {
-      exact = c->batch_exact;
-    } else if ((rc = exact_fits(c, nk, ks, olp, cv, ct.n, kp, &exact))) {
-      return rc;
-    }
+  if (!same) {
+    c->batch_sig.clear();   // until the layout is whole: one that fails may have freed what the last batch's tables name
+    c->batch_exact = false;
+  } else if (exact) {
+    exact = c->batch_exact;
   }
-  const bool crt = icrt || exact;
   if (same && (flags & EXC_BATCH_GRAPH) && c->graph_exec) {
     StageTimer t(c, EXC_STAGE_GRAPH);
     EXC_CHECK(hipGraphLaunch(c->graph_exec, c->stream));
@@ -971,7 +1002,6 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   }
   if (!same) {
     // new batch: lay out the Y workspace, descriptors and the muffin-tin work list
-    c->batch_sig.clear();   // until the layout is whole: one that fails may have freed what the last batch's tables name
     EXC_CHECK(hipStreamSynchronize(c->stream));   // earlier launches may still read the old tables
     if (c->graph_exec) {
       hipGraphExecDestroy(c->graph_exec);
@@ -989,10 +1019,10 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
       ptot += 2 * exc_split_plane_elems(ks[k].ngp, c->d.natm);
       etot += 2 * (size_t)ks[k].ngp * c->d.natm;
     }
-    if ((rc = grow((void **)&c->byt, &c->byt_bytes, sizeof(cplx) * (ytot ? ytot : 1)))) return rc;
+    if ((rc = grow(c, (void **)&c->byt, &c->byt_bytes, sizeof(cplx) * (ytot ? ytot : 1)))) return rc;
     if (split) {
-      if ((rc = grow((void **)&c->planes, &c->planes_bytes, 2 * (ptot ? ptot : 1)))) return rc;
-      if ((rc = grow((void **)&c->expo, &c->expo_bytes, sizeof(int) * (etot ? etot : 1)))) return rc;
+      if ((rc = grow(c, (void **)&c->planes, &c->planes_bytes, 2 * (ptot ? ptot : 1)))) return rc;
+      if ((rc = grow(c, (void **)&c->expo, &c->expo_bytes, sizeof(int) * (etot ? etot : 1)))) return rc;
     }
     // radial factors and their transposed copy (overlap variants 2 and 3: N rounded up to 64
     // rows per atom and slot, NL + 1 slots per atom: the radial factors of each l and the
@@ -1004,39 +1034,39 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
       rtpad = std::max(rtpad, (size_t)(ks[k].ngp + 63) / 64 * 64 * 2 * 4);
     }
     rttot += rtpad;
-    if (olp && (rc = grow((void **)&c->rfbuf, &c->rf_bytes, sizeof(double) * (rtot + rttot ? rtot + rttot : 1))))
+    if (olp && (rc = grow(c, (void **)&c->rfbuf, &c->rf_bytes, sizeof(double) * (rtot + rttot ? rtot + rttot : 1))))
       return rc;
-    size_t qtot = 0, xtot = 0;
+    struct Hold {                                  // the layout names the planes from here on
+      exc_ctx *c;
+      bool was;
+      ~Hold() { c->crt_held = was; }
+    } hold{c, c->crt_held};
+    c->crt_held = true;
+    if (exact && (rc = exact_workspace(c, nk, ks, olp, cv, ct.n, kp, hold.was, &exact))) return rc;
+    c->batch_exact = exact;
+    const bool crt = icrt || exact;
+    size_t qtot = 0, rtot2 = 0, xtot = 0;
     int cbt = 0, cwr = 0, cwc = 0;
     if (crt && exc_crt_shape(cv, &cbt, &cwr, &cwc)) return EXC_ERR_ARG;
     // squared row norms of A per atom (cnp each), when the grouped match runs here
     const size_t nparts = do_match ? (size_t)c->d.natm : 0;
     size_t ptot2 = 0;
-    c->crt_groups.clear();
-    c->batch_exact = exact;
     if (crt) {
-      size_t q = 0;
+      // the modular split takes all k-points at once (the Gram form splits E only)
+      if (!exact) crt_group(c, nk, ks, ~(size_t)0, gram ? 1 : 2, olp ? 1 : 2, cbt, ct.n, kp, &qtot, &rtot2);
       for (int k = 0; k < nk; ++k) {
         const size_t cnp = crt_rows(ks[k].ngp);
-        const size_t b = (gram ? 1 : 2) * crt_plane_bytes(ks[k].ngp, ct.n, kp);   // the Gram form splits E only
-        // the exact products' many planes: the k-points in groups that share the workspace
-        if (k == 0 || (exact && q && q + b > kExactPlanes)) {
-          c->crt_groups.push_back({k, 0, 0, 0, 0, 0, 0});
-          q = 0;
-        }
-        c->crt_groups.back().nk += 1;
-        q += b;
-        qtot = std::max(qtot, q);
         xtot += 2 * cnp;
         ptot2 += nparts * cnp;
       }
-      if ((rc = grow(&c->crt_q, &c->crt_q_bytes, qtot ? qtot : 1))) return rc;
-      if ((rc = grow((void **)&c->crt_x, &c->crt_x_bytes, sizeof(int) * (xtot ? xtot : 1)))) return rc;
-      if ((rc = grow((void **)&c->crt_parts, &c->crt_parts_bytes, sizeof(double) * (ptot2 ? ptot2 : 1)))) return rc;
+      if (!exact && (rc = grow(c, &c->crt_q, &c->crt_q_bytes, qtot ? qtot : 1))) return rc;
+      if (!exact && (rc = grow(c, (void **)&c->crt_res, &c->crt_res_bytes, rtot2 ? rtot2 : 1))) return rc;
+      if ((rc = grow(c, (void **)&c->crt_x, &c->crt_x_bytes, sizeof(int) * (xtot ? xtot : 1)))) return rc;
+      if ((rc = grow(c, (void **)&c->crt_parts, &c->crt_parts_bytes, sizeof(double) * (ptot2 ? ptot2 : 1)))) return rc;
     }
     std::vector<mt_item> citems;
     std::vector<int2> cwork;
-    size_t qoff = 0, xoff = 0, poff2 = 0, rmax = 0;
+    size_t qoff = 0, xoff = 0, poff2 = 0;
     size_t grp = 0;                                          // the group of k-point k
     std::vector<kdesc> kd(nk);
     std::vector<mt_item> items, oitems;
@@ -1118,7 +1148,6 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
             for (int i = first; i < (int)citems.size(); ++i) cwork.push_back(make_int2(i - g.item0, 4 * l + p));
         g.nitem = (int)citems.size() - g.item0;
         g.nwork = (int)cwork.size() - g.work0;
-        rmax = std::max(rmax, (size_t)g.nitem * ct.n * 2 * cbt * cbt);
       }
       maxngp = q.ngp > maxngp ? q.ngp : maxngp;
       const int nt = (q.ngp + T - 1) / T;
@@ -1140,25 +1169,24 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
       }
     }
     if (olp) {
-      if ((rc = grow((void **)&c->d_oitems, &c->oitems_cap, sizeof(mt_item) * (oitems.empty() ? 1 : oitems.size()))))
+      if ((rc = grow(c, (void **)&c->d_oitems, &c->oitems_cap, sizeof(mt_item) * (oitems.empty() ? 1 : oitems.size()))))
         return rc;
       if (!oitems.empty())
         EXC_CHECK(hipMemcpy(c->d_oitems, oitems.data(), sizeof(mt_item) * oitems.size(), hipMemcpyHostToDevice));
     }
     c->batch_noitems = (int)oitems.size();
     if (crt) {
-      if ((rc = grow((void **)&c->crt_res, &c->crt_res_bytes, rmax ? rmax : 1))) return rc;
-      if ((rc = grow((void **)&c->d_citems, &c->citems_cap, sizeof(mt_item) * (citems.empty() ? 1 : citems.size()))))
+      if ((rc = grow(c, (void **)&c->d_citems, &c->citems_cap, sizeof(mt_item) * (citems.empty() ? 1 : citems.size()))))
         return rc;
-      if ((rc = grow((void **)&c->d_cwork, &c->cwork_cap, sizeof(int2) * (cwork.empty() ? 1 : cwork.size()))))
+      if ((rc = grow(c, (void **)&c->d_cwork, &c->cwork_cap, sizeof(int2) * (cwork.empty() ? 1 : cwork.size()))))
         return rc;
       if (!citems.empty())
         EXC_CHECK(hipMemcpy(c->d_citems, citems.data(), sizeof(mt_item) * citems.size(), hipMemcpyHostToDevice));
       if (!cwork.empty())
         EXC_CHECK(hipMemcpy(c->d_cwork, cwork.data(), sizeof(int2) * cwork.size(), hipMemcpyHostToDevice));
     }
-    if ((rc = grow((void **)&c->d_ks, &c->ks_cap, sizeof(kdesc) * nk))) return rc;
-    if ((rc = grow((void **)&c->d_items, &c->items_cap, sizeof(mt_item) * (items.empty() ? 1 : items.size()))))
+    if ((rc = grow(c, (void **)&c->d_ks, &c->ks_cap, sizeof(kdesc) * nk))) return rc;
+    if ((rc = grow(c, (void **)&c->d_items, &c->items_cap, sizeof(mt_item) * (items.empty() ? 1 : items.size()))))
       return rc;
     EXC_CHECK(hipMemcpy(c->d_ks, kd.data(), sizeof(kdesc) * nk, hipMemcpyHostToDevice));
     if (!items.empty())
@@ -1172,8 +1200,15 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
     c->batch_nk = nk;
     c->batch_sig = sig;
   }
+  const bool crt = icrt || exact;
+  if (c->fork_variant < 0) fv = gram || exact ? 0 : 1;   // (a batch whose exact products had no room)
   const bool capture = flags & EXC_BATCH_GRAPH;
   if (capture && c->stream == nullptr) return EXC_ERR_ARG;   // the null stream cannot be captured
+  if (crt && !capture && !c->crt_held && c->stream) {   // a graph of the caller's own keeps the addresses: they stay
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    EXC_CHECK(hipStreamIsCapturing(c->stream, &st));
+    c->crt_held = st != hipStreamCaptureStatusNone;
+  }
   // inside a graph the overlap and lo kernels (they read only A, the radial factors and the
   // structure factors, and write parts of H and O the MT stage does not) can form a branch of
   // their own beside the Y and MT stages; with a persistent split-BF16 kernel (static work
@@ -1301,7 +1336,7 @@ int exc_ho_vjp_dev(exc_ctx *c, int ngp, int ngkmax, const double *apwalm, const 
   int rc = use_device(c);
   if (rc) return rc;
   const size_t need = sizeof(cplx) * exc_vjp_work_elems(c->d, ngp, nst);
-  if ((rc = grow((void **)&c->vjp_work, &c->vjp_bytes, need ? need : 1))) return rc;
+  if ((rc = grow(c, (void **)&c->vjp_work, &c->vjp_bytes, need ? need : 1))) return rc;
   StageTimer t(c, EXC_STAGE_VJP);
   const long ytiles = (long)((nst + 63) / 64) * ((c->d.naa + 127) / 128) * c->d.natm;
   return exc_launch_vjp(c->d, ngp, nst, (const cplx *)apwalm, ngkmax, igpig, vgpc, (const cplx *)sfacgp,
@@ -1327,7 +1362,7 @@ int exc_ho_vjp(exc_ctx *c, int ngp, int ngkmax, const double *apwalm, const int 
   off[0] = 0;
   const size_t sz[9] = {b_apw, b_ig, b_vg, b_sf, b_ev, b_w, b_w, b_dt, b_dv};
   for (int i = 1; i < 9; ++i) off[i] = off[i - 1] + al(sz[i - 1]);
-  if ((rc = grow(&c->stage, &c->stage_bytes, off[8] + b_dv))) return rc;
+  if ((rc = grow(c, &c->stage, &c->stage_bytes, off[8] + b_dv))) return rc;
   char *base = (char *)c->stage;
   const void *src[7] = {apwalm, igpig, vgpc, sfacgp, evec, wh, wo};
   for (int i = 0; i < 7; ++i)

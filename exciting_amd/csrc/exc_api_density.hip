@@ -29,7 +29,7 @@ int dmat_run(exc_ctx *c, int nk, const int *ngp, const int *ldg, const double *c
   const size_t b_w = al(16 * (size_t)na * naa * nst), b_x = al(16 * (size_t)na * ws * nt);
   const size_t b_t = any_sv ? al(16 * (size_t)na * ws * nst) : 0, b_p = al(16 * (size_t)na * ws * ws);
   int rc;
-  if ((rc = grow(&c->dmw, &c->dmw_bytes, nw * (b_w + b_t + b_p) + 2 * b_x))) return rc;
+  if ((rc = grow(c, &c->dmw, &c->dmw_bytes, nw * (b_w + b_t + b_p) + 2 * b_x))) return rc;
   char *base = (char *)c->dmw;
   cplx *x = (cplx *)base, *x2 = (cplx *)(base + b_x);
   char *per = base + 2 * b_x;   // per worker: W, Xt, partial
@@ -38,10 +38,7 @@ int dmat_run(exc_ctx *c, int nk, const int *ngp, const int *ldg, const double *c
     exc_ctx::EigWorker &W = c->ew[i];
     if (!W.s) EXC_CHECK(hipStreamCreateWithFlags(&W.s, hipStreamNonBlocking));   // default priority
     if (!W.done) EXC_CHECK(hipEventCreateWithFlags(&W.done, hipEventDisableTiming));
-    if (!W.blas && rocblas_create_handle(&W.blas) != rocblas_status_success) {
-      W.blas = nullptr;
-      return EXC_ERR_HIP;
-    }
+    if (int e = blas_handle(c, &W.blas)) return e;
     if (rocblas_set_stream(W.blas, W.s) != rocblas_status_success) return EXC_ERR_HIP;
   }
   const rocblas_double_complex one = {1.0, 0.0}, zero = {0.0, 0.0};
@@ -158,7 +155,7 @@ int exc_gendmatmt(exc_ctx *c, int ngp, int ngkmax, const double *apwalm, int nst
   const size_t b_d = 16 * (size_t)ws * ws * c->d.natm;
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t o_v = al(b_a), o_s = o_v + al(b_v), o_o = o_s + al(b_s), o_d = o_o + al(b_o);
-  if ((rc = grow(&c->stage, &c->stage_bytes, o_d + b_d))) return rc;
+  if ((rc = grow(c, &c->stage, &c->stage_bytes, o_d + b_d))) return rc;
   char *base = (char *)c->stage;
   EXC_CHECK(hipMemcpyAsync(base, apwalm, b_a, hipMemcpyHostToDevice, c->stream));
   EXC_CHECK(hipMemcpyAsync(base + o_v, evecfv, b_v, hipMemcpyHostToDevice, c->stream));

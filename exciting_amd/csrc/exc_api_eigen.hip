@@ -20,14 +20,14 @@ bool eig_args_ok(int nmat, int ldh, int nev, int ldv) {
 // handle's allocation could then take over that memory.  The buffer here only grows through
 // grow(), which drains the device before it frees.
 extern "C++" template <class F>
-int pin_workspace(exc_ctx::EigWorker &W, F &&calls) {
+int pin_workspace(exc_ctx *c, exc_ctx::EigWorker &W, F &&calls) {
   if (rocblas_start_device_memory_size_query(W.blas) != rocblas_status_success) return EXC_ERR_HIP;
   calls();
   size_t need = 0;
   if (rocblas_stop_device_memory_size_query(W.blas, &need) != rocblas_status_success) return EXC_ERR_HIP;
   need = std::max(need, (size_t)256);
   const bool moved = need > W.wsb;
-  int rc = grow(&W.ws, &W.wsb, need);
+  int rc = grow(c, &W.ws, &W.wsb, need);
   if (rc) return rc;
   if ((moved || !W.ws_set) && rocblas_set_workspace(W.blas, W.ws, W.wsb) != rocblas_status_success) return EXC_ERR_HIP;
   W.ws_set = true;
@@ -96,25 +96,20 @@ rocblas_status eig_calls(exc_ctx::EigWorker &W, int v, int phase, int nmat, int 
   }
 }
 
-int eig_enqueue(exc_ctx::EigWorker &W, int v, int phase, int nmat, int ldh, double *h, double *o, int nev,
+int eig_enqueue(exc_ctx *c, exc_ctx::EigWorker &W, int v, int phase, int nmat, int ldh, double *h, double *o, int nev,
                 double *eval, double *evec, int ldv, int *d_ints) {
-  if (!W.blas) {
-    if (rocblas_create_handle(&W.blas) != rocblas_status_success) {
-      W.blas = nullptr;
-      return EXC_ERR_HIP;
-    }
-  }
+  if (int e = blas_handle(c, &W.blas)) return e;
   if (rocblas_set_stream(W.blas, W.s) != rocblas_status_success) return EXC_ERR_HIP;
   // W has n slots and Z n columns: rocSOLVER's divide-and-conquer path uses the columns past
   // nev as workspace, so the caller's nev columns are filled from an internal n x n buffer
   int rc;
-  if ((rc = grow((void **)&W.w, &W.wb, sizeof(double) * nmat))) return rc;
-  if ((rc = grow((void **)&W.z, &W.zb, sizeof(cplx) * (size_t)nmat * nmat))) return rc;
-  if ((rc = grow((void **)&W.e, &W.eb, sizeof(double) * (nmat + 1)))) return rc;
+  if ((rc = grow(c, (void **)&W.w, &W.wb, sizeof(double) * nmat))) return rc;
+  if ((rc = grow(c, (void **)&W.z, &W.zb, sizeof(cplx) * (size_t)nmat * nmat))) return rc;
+  if ((rc = grow(c, (void **)&W.e, &W.eb, sizeof(double) * (nmat + 1)))) return rc;
   bool in_a = false;
   if (phase == 1) {
     // the workspace of both phases, before anything of this solve is queued
-    if ((rc = pin_workspace(W, [&]() {
+    if ((rc = pin_workspace(c, W, [&]() {
            eig_calls(W, v, 1, nmat, ldh, h, o, nev, d_ints, &in_a);
            eig_calls(W, v, 2, nmat, ldh, h, o, nev, d_ints, &in_a);
          })))
@@ -200,7 +195,7 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   const size_t o_ch = o_tr;         // (the factorization is over before the tridiagonal reduction begins)
   const size_t total = o_tr + (bisect ? 0 : al(std::max(exc_trd_work_bytes(n, nb), exc_chol_work_bytes(n, nb))));
   int rc;
-  if ((rc = grow(&c->eg, &c->eg_bytes, total))) return rc;
+  if ((rc = grow(c, &c->eg, &c->eg_bytes, total))) return rc;
   char *base = (char *)c->eg;
   cplx *ph = (cplx *)base, *po = (cplx *)(base + o_po), *pz = (cplx *)(base + o_pz), *tau = (cplx *)(base + o_tau);
   double *d = (double *)(base + o_d), *e = (double *)(base + o_e);
@@ -209,14 +204,11 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
   for (int i = 0; i <= nw; ++i) {
     exc_ctx::EigWorker &W = c->ew[i];
     if (i == 0) W.s = c->stream;
-    if (!W.blas && rocblas_create_handle(&W.blas) != rocblas_status_success) {
-      W.blas = nullptr;
-      return EXC_ERR_HIP;
-    }
+    if (int e = blas_handle(c, &W.blas)) return e;
     if (rocblas_set_stream(W.blas, W.s) != rocblas_status_success) return EXC_ERR_HIP;
     if (i > 0) {   // per worker: real eigenvectors of T (n x n), their first nev columns complex
-      if ((rc = grow((void **)&W.z, &W.zb, sizeof(double) * mat))) return rc;
-      if (!blocked && (rc = grow((void **)&W.zc, &W.zcb, sizeof(cplx) * (size_t)n * nev))) return rc;
+      if ((rc = grow(c, (void **)&W.z, &W.zb, sizeof(double) * mat))) return rc;
+      if (!blocked && (rc = grow(c, (void **)&W.zc, &W.zcb, sizeof(cplx) * (size_t)n * nev))) return rc;
     }
   }
   auto fail = [](const char *what, int a, int b) {
@@ -240,7 +232,7 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
     const rocblas_stride sv = (rocblas_stride)n * kBT, st2 = (rocblas_stride)kBT * kBT;
     const rocblas_stride sw = (rocblas_stride)kBT * nev, sxx = (rocblas_stride)n * nev;
     const int ib = std::min(kBT, std::max(n - 1, 1));
-    if ((rc = pin_workspace(c->ew[0], [&]() {
+    if ((rc = pin_workspace(c, c->ew[0], [&]() {
            if (bisect) {
              rocsolver_zpotrf_strided_batched(hb, up, n, B, n, sm, info, nb);
              rocsolver_ztrtri_strided_batched(hb, up, nu, n, B, n, sm, info + nb, nb);
@@ -260,7 +252,7 @@ int eig_grouped(exc_ctx *c, int nk, const int *nmat, const int *ldh, double *con
       return rc;
     for (int i = 1; i <= nw; ++i) {
       exc_ctx::EigWorker &W = c->ew[i];
-      if ((rc = pin_workspace(W, [&]() {
+      if ((rc = pin_workspace(c, W, [&]() {
              if (bisect) {
                double *wv = (double *)(base + o_wv);
                int *ibk = (int *)(base + o_ib), *isp = (int *)(base + o_is), *ifl = (int *)(base + o_if);
@@ -428,20 +420,20 @@ int exc_eigen_dev(exc_ctx *c, int nmat, int ldh, double *h, double *o, int nev, 
   if (!h || !o || !eval || !evec) return EXC_ERR_ARG;
   int rc = use_device(c);
   if (rc) return rc;
-  if ((rc = grow((void **)&c->eig_int, &c->eig_int_bytes, 4 * sizeof(int)))) return rc;
+  if ((rc = grow(c, (void **)&c->eig_int, &c->eig_int_bytes, 4 * sizeof(int)))) return rc;
   const int v = c->eig_variant >= 0 ? c->eig_variant : 4;
   exc_ctx::EigWorker &W = c->ew[0];
   W.s = c->stream;
   int hi[4] = {0, 0, 0, 0};
   {
     StageTimer t(c, EXC_STAGE_EIGEN);
-    if ((rc = eig_enqueue(W, v, 1, nmat, ldh, h, o, nev, eval, evec, ldv, c->eig_int))) return rc;
+    if ((rc = eig_enqueue(c, W, v, 1, nmat, ldh, h, o, nev, eval, evec, ldv, c->eig_int))) return rc;
     if (v >= 4) {
       EXC_CHECK(hipMemcpyAsync(hi, c->eig_int, sizeof(hi), hipMemcpyDeviceToHost, c->stream));
       EXC_CHECK(hipStreamSynchronize(c->stream));
       if (hi[1] > 0) return nmat + hi[1];
     }
-    if ((rc = eig_enqueue(W, v, 2, nmat, ldh, h, o, nev, eval, evec, ldv, c->eig_int))) return rc;
+    if ((rc = eig_enqueue(c, W, v, 2, nmat, ldh, h, o, nev, eval, evec, ldv, c->eig_int))) return rc;
   }
   EXC_CHECK(hipMemcpyAsync(hi, c->eig_int, sizeof(hi), hipMemcpyDeviceToHost, c->stream));
   EXC_CHECK(hipStreamSynchronize(c->stream));
@@ -459,7 +451,7 @@ int exc_eigen_batched_dev(exc_ctx *c, int nk, const int *nmat, const int *ldh, d
   if (nk == 0 || nev == 0) return EXC_OK;
   int rc = use_device(c);
   if (rc) return rc;
-  if ((rc = grow((void **)&c->eig_int, &c->eig_int_bytes, 4 * sizeof(int) * nk))) return rc;
+  if ((rc = grow(c, (void **)&c->eig_int, &c->eig_int_bytes, 4 * sizeof(int) * nk))) return rc;
   if (!c->eig_fork) EXC_CHECK(hipEventCreateWithFlags(&c->eig_fork, hipEventDisableTiming));
   const int nw = nk < exc_ctx::kEigStreams ? nk : exc_ctx::kEigStreams;
   for (int i = 1; i <= nw; ++i) {
@@ -480,9 +472,9 @@ int exc_eigen_batched_dev(exc_ctx *c, int nk, const int *nmat, const int *ldh, d
     for (int k = 0; k < nk; ++k) nmax = std::max(nmax, nmat[k]);
     for (int i = 1; i <= nw; ++i) {
       exc_ctx::EigWorker &W = c->ew[i];
-      if ((rc = grow((void **)&W.w, &W.wb, sizeof(double) * nmax))) return rc;
-      if ((rc = grow((void **)&W.z, &W.zb, sizeof(cplx) * (size_t)nmax * nmax))) return rc;
-      if ((rc = grow((void **)&W.e, &W.eb, sizeof(double) * (nmax + 1)))) return rc;
+      if ((rc = grow(c, (void **)&W.w, &W.wb, sizeof(double) * nmax))) return rc;
+      if ((rc = grow(c, (void **)&W.z, &W.zb, sizeof(cplx) * (size_t)nmax * nmax))) return rc;
+      if ((rc = grow(c, (void **)&W.e, &W.eb, sizeof(double) * (nmax + 1)))) return rc;
     }
   }
   {
@@ -501,7 +493,7 @@ int exc_eigen_batched_dev(exc_ctx *c, int nk, const int *nmat, const int *ldh, d
       for (int k = 0; k < nk && !rc; ++k) {
         if (nmat[k] == 0) continue;
         exc_ctx::EigWorker &W = c->ew[1];   // one after another (see below)
-        rc = eig_enqueue(W, v, phase, nmat[k], ldh[k], h[k], o[k], nev, eval[k], evec[k], ldv[k], c->eig_int + 4 * k);
+        rc = eig_enqueue(c, W, v, phase, nmat[k], ldh[k], h[k], o[k], nev, eval[k], evec[k], ldv[k], c->eig_int + 4 * k);
       }
       if (rc) break;
     }
@@ -530,7 +522,7 @@ int exc_eigen(exc_ctx *c, int nmat, int ldh, double *h, double *o, int nev, doub
   const size_t b_m = 16 * (size_t)ldh * nmat, b_v = 16 * (size_t)ldv * nev, b_e = 8 * (size_t)nev;
   const size_t o_o = (b_m + 255) & ~(size_t)255, o_v = o_o + ((b_m + 255) & ~(size_t)255);
   const size_t o_e = o_v + ((b_v + 255) & ~(size_t)255);
-  if ((rc = grow(&c->stage, &c->stage_bytes, o_e + b_e))) return rc;
+  if ((rc = grow(c, &c->stage, &c->stage_bytes, o_e + b_e))) return rc;
   if ((rc = grow_host(&c->hstage, &c->hstage_bytes, std::max(2 * b_m, b_v)))) return rc;
   char *base = (char *)c->stage, *hs = (char *)c->hstage;
   const size_t pitch = 16 * (size_t)ldh, width = 16 * (size_t)nmat;

@@ -113,7 +113,7 @@ int exc_ctx_hmlint(exc_ctx *c, int lmaxvr, int nrmtmax, const int *nrmt, const d
   if (c->gnt_lmaxvr != lmaxvr) {
     std::vector<cplx> g((size_t)lmm * lmm * (lmaxvr + 1) * 2);
     exc_hml_gaunt_table(d.lmaxmat, lmaxvr, g.data());
-    if ((rc = grow((void **)&c->gnt, &c->gnt_bytes, sizeof(cplx) * g.size()))) return rc;
+    if ((rc = grow(c, (void **)&c->gnt, &c->gnt_bytes, sizeof(cplx) * g.size()))) return rc;
     EXC_CHECK(hipMemcpy(c->gnt, g.data(), sizeof(cplx) * g.size(), hipMemcpyHostToDevice));
     c->gnt_lmaxvr = lmaxvr;
   }
@@ -122,7 +122,7 @@ int exc_ctx_hmlint(exc_ctx *c, int lmaxvr, int nrmtmax, const int *nrmt, const d
   const size_t n_w = H.n_w, n_apw = H.n_apw, n_lo = H.n_lo, n_v = H.n_v;
   const size_t o_spr = H.o_spr, o_apw = H.o_apw, o_lo = H.o_lo, o_v = H.o_v, o_rad = H.o_rad, o_i = H.o_i;
   c->hml_lmaxvr = -1;
-  if ((rc = grow(&c->hml, &c->hml_bytes, H.total))) return rc;
+  if ((rc = grow(c, &c->hml, &c->hml_bytes, H.total))) return rc;
   char *b = (char *)c->hml;
   std::vector<int> ints(nrmt, nrmt + ns);
   ints.insert(ints.end(), c->h_nlorb.begin(), c->h_nlorb.end());
@@ -185,7 +185,7 @@ int exc_genrhomt(exc_ctx *c, const double *dm, double *rhomt) {
   const size_t ws = c->d.naa + c->d.dm_maxlo, na = c->d.natm;
   const size_t b_d = 16 * ws * ws * na, b_r = 8 * (size_t)(c->hml_lmaxvr + 1) * (c->hml_lmaxvr + 1) * c->hml_nrmtmax * na;
   const size_t o_r = (b_d + 255) & ~(size_t)255;
-  if ((rc = grow(&c->stage, &c->stage_bytes, o_r + b_r))) return rc;
+  if ((rc = grow(c, &c->stage, &c->stage_bytes, o_r + b_r))) return rc;
   char *base = (char *)c->stage;
   EXC_CHECK(hipMemcpyAsync(base, dm, b_d, hipMemcpyHostToDevice, c->stream));
   if ((rc = exc_genrhomt_dev(c, (const double *)base, (double *)(base + o_r)))) return rc;
@@ -214,7 +214,7 @@ int exc_rhovalk_dev(exc_ctx *c, int lradstep, const double *zbshtvr, const doubl
   auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
   const size_t o_c = al(sizeof(cplx) * (size_t)ldw * nst);   // W, then evecfv evecsv, then the kernels' work
   const size_t o_k = o_c + (evecsv ? al(sizeof(cplx) * (size_t)nmat * nst) : 0);
-  if ((rc = grow(&c->rvw, &c->rvw_bytes, o_k + exc_rhovalk_work_bytes(d, lmaxvr, c->dims.nlomax, nst)))) return rc;
+  if ((rc = grow(c, &c->rvw, &c->rvw_bytes, o_k + exc_rhovalk_work_bytes(d, lmaxvr, c->dims.nlomax, nst)))) return rc;
   const HmlLayout H = hml_layout(c, lmaxvr, nrmtmax);
   const char *b = (const char *)c->hml;
   const int *di = (const int *)(b + H.o_i);
@@ -222,10 +222,7 @@ int exc_rhovalk_dev(exc_ctx *c, int lradstep, const double *zbshtvr, const doubl
   if (evecsv) {   // the states evecfv evecsv (wavefmt is linear in the coefficients)
     exc_ctx::EigWorker &W = c->ew[0];
     W.s = c->stream;
-    if (!W.blas && rocblas_create_handle(&W.blas) != rocblas_status_success) {
-      W.blas = nullptr;
-      return EXC_ERR_HIP;
-    }
+    if (int e = blas_handle(c, &W.blas)) return e;
     if (rocblas_set_stream(W.blas, W.s) != rocblas_status_success) return EXC_ERR_HIP;
     const rocblas_double_complex one = {1.0, 0.0}, zero = {0.0, 0.0};
     cplx *c2 = (cplx *)((char *)c->rvw + o_c);
@@ -272,7 +269,7 @@ int exc_rhovalk(exc_ctx *c, int lradstep, const double *zbshtvr, const double *r
   auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
   const size_t o_v = al(b_a), o_o = o_v + al(b_v), o_z = o_o + al(b_o), o_f = o_z + al(b_z), o_r = o_f + al(b_f);
   const size_t o_s = o_r + al(b_r);
-  if ((rc = grow(&c->stage, &c->stage_bytes, o_s + b_s))) return rc;
+  if ((rc = grow(c, &c->stage, &c->stage_bytes, o_s + b_s))) return rc;
   char *base = (char *)c->stage;
   EXC_CHECK(hipMemcpyAsync(base, apwalm, b_a, hipMemcpyHostToDevice, c->stream));
   EXC_CHECK(hipMemcpyAsync(base + o_v, evecfv, b_v, hipMemcpyHostToDevice, c->stream));
@@ -303,7 +300,10 @@ int scf_prepare(exc_ctx *c) {
   if (!c->fin && (rc = dev_alloc(c, &c->fin, box))) return rc;
   if (!c->have_fft) {
     // Fortran order: the first index runs fastest, so it is hipFFT's last dimension
-    if (hipfftPlan3d(&c->fft, d.box_n[2], d.box_n[1], d.box_n[0], HIPFFT_Z2Z) != HIPFFT_SUCCESS) return EXC_ERR_HIP;
+    if (!with_memory(c, [&]() {
+          return hipfftPlan3d(&c->fft, d.box_n[2], d.box_n[1], d.box_n[0], HIPFFT_Z2Z) == HIPFFT_SUCCESS;
+        }))
+      return EXC_ERR_HIP;
     c->have_fft = true;
   }
   if (hipfftSetStream(c->fft, c->stream) != HIPFFT_SUCCESS) return EXC_ERR_HIP;
@@ -380,7 +380,7 @@ int exc_gengpvec_dev(exc_ctx *c, int nk, const double *bvec, const double *vpl, 
   int rc = use_device(c);
   if (rc) return rc;
   const size_t head = gk_head(nk);
-  if ((rc = grow(&c->gk_buf, &c->gk_buf_bytes, head))) return rc;
+  if ((rc = grow(c, &c->gk_buf, &c->gk_buf_bytes, head))) return rc;
   std::vector<double> kv(6 * (size_t)nk);
   for (int k = 0; k < nk; ++k)
     for (int d = 0; d < 3; ++d) {
@@ -410,7 +410,7 @@ int exc_gengpvec(exc_ctx *c, const double *bvec, const double *vpl, const double
   if (rc) return rc;
   // device staging after the head: igpig, vgpl, vgpc, gpc, tpgpc (9 doubles + 1 int per row)
   const size_t head = gk_head(1), n = (size_t)ngkmax;
-  if ((rc = grow(&c->gk_buf, &c->gk_buf_bytes, head + 72 * n + 4 * n + 256))) return rc;
+  if ((rc = grow(c, &c->gk_buf, &c->gk_buf_bytes, head + 72 * n + 4 * n + 256))) return rc;
   char *st = (char *)c->gk_buf + head;
   double *d_vgpl = (double *)st, *d_vgpc = d_vgpl + 3 * n, *d_gpc = d_vgpc + 3 * n, *d_tp = d_gpc + n;
   int *d_ig = (int *)(d_tp + 2 * n);
@@ -435,7 +435,7 @@ int exc_gensfacgp(exc_ctx *c, int ngp, const double *vgpc, int ld, double *sfacg
   int rc = use_device(c);
   if (rc) return rc;
   const size_t head = gk_head(1), nv = 3 * (size_t)ngp, ns = (size_t)ld * c->d.natm;
-  if ((rc = grow(&c->gk_buf, &c->gk_buf_bytes, head + 8 * nv + 16 * ns + 256))) return rc;
+  if ((rc = grow(c, &c->gk_buf, &c->gk_buf_bytes, head + 8 * nv + 16 * ns + 256))) return rc;
   double *d_v = (double *)((char *)c->gk_buf + head);
   cplx *d_s = (cplx *)(d_v + nv);
   EXC_CHECK(hipMemcpyAsync(d_v, vgpc, 8 * nv, hipMemcpyHostToDevice, c->stream));
@@ -467,18 +467,20 @@ int rhoir_run(exc_ctx *c, int nk, const int *ngp, const int *const *igpig, int n
       EXC_CHECK(hipStreamSynchronize(c->stream));
       c->dft = p;
     }
-    if ((rc = grow((void **)&c->zb, &c->zb_bytes, exc_rhoir_work_bytes(d, nk, nst, c->ncu)))) return rc;
+    if ((rc = grow(c, (void **)&c->zb, &c->zb_bytes, exc_rhoir_work_bytes(d, nk, nst, c->ncu)))) return rc;
     StageTimer t(c, EXC_STAGE_SCF);
     return exc_launch_rhoir(d, nk, ngp, igpig, nst, ldv, evec, occ, wkpt, epsocc, c->dft, c->zb, rhoir, c->ncu, c->stream);
   }
   // states per transform: nearly equal chunks (200 states: 4 of 50, not 3 of 64 and one of 64 for 8)
   const int nch = (nst + kRhoirChunk - 1) / kRhoirChunk, B = (nst + nch - 1) / nch;
-  if ((rc = grow((void **)&c->zb, &c->zb_bytes, sizeof(cplx) * (size_t)B * N))) return rc;
+  if ((rc = grow(c, (void **)&c->zb, &c->zb_bytes, sizeof(cplx) * (size_t)B * N))) return rc;
   if (c->fftb_n != B) {
     if (c->fftb_n > 0) hipfftDestroy(c->fftb);
     c->fftb_n = 0;
     int dims[3] = {d.box_n[2], d.box_n[1], d.box_n[0]};   // Fortran order: first index fastest
-    if (hipfftPlanMany(&c->fftb, 3, dims, nullptr, 1, N, nullptr, 1, N, HIPFFT_Z2Z, B) != HIPFFT_SUCCESS)
+    if (!with_memory(c, [&]() {
+          return hipfftPlanMany(&c->fftb, 3, dims, nullptr, 1, N, nullptr, 1, N, HIPFFT_Z2Z, B) == HIPFFT_SUCCESS;
+        }))
       return EXC_ERR_HIP;
     c->fftb_n = B;
   }
@@ -542,7 +544,7 @@ int exc_genrhoir(exc_ctx *c, int ngp, const int *igpig, int nst, int ldv, const 
   const size_t N = c->dims.ngrtot, b_i = 4 * (size_t)ngp, b_v = 16 * (size_t)ldv * nst, b_o = 8 * (size_t)nst;
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t o_v = al(b_i), o_o = o_v + al(b_v), o_r = o_o + al(b_o);
-  if ((rc = grow(&c->stage, &c->stage_bytes, o_r + 8 * N))) return rc;
+  if ((rc = grow(c, &c->stage, &c->stage_bytes, o_r + 8 * N))) return rc;
   char *base = (char *)c->stage;
   EXC_CHECK(hipMemcpyAsync(base, igpig, b_i, hipMemcpyHostToDevice, c->stream));
   EXC_CHECK(hipMemcpyAsync(base + o_v, evecfv, b_v, hipMemcpyHostToDevice, c->stream));

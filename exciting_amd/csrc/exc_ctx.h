@@ -108,6 +108,7 @@ struct exc_ctx {
   };
   std::vector<CrtGroup> crt_groups;
   bool batch_exact;           // the FP64 batch's muffin-tin products run as exact integer products
+  bool crt_held;              // crt_q and crt_res are named by a layout under way, or by a graph of the caller's
   std::vector<char> batch_sig;   // the batch the descriptors / graph were built for
   int batch_nitems, batch_nblocks, batch_maxngp, batch_nk;
   hipGraph_t graph;
@@ -170,12 +171,53 @@ struct exc_ctx {
 
 namespace exc_impl {
 
+// Frees the residue planes and residues (gigabytes, kept for the next setup of the same batch,
+// which only lays them out again); false if there is nothing to free
+inline bool give_back(exc_ctx *c) {
+  if (c->crt_held || (!c->crt_q && !c->crt_res)) return false;
+  if (hipDeviceSynchronize() != hipSuccess) return false;
+  c->batch_sig.clear();                   // a batch that used them is laid out (and captured) again
+  if (c->crt_q) hipFree(c->crt_q);
+  if (c->crt_res) hipFree(c->crt_res);
+  c->crt_q = nullptr;
+  c->crt_res = nullptr;
+  c->crt_q_bytes = c->crt_res_bytes = 0;
+  return true;
+}
+
+// hipMalloc that gives the context's own spare memory back before it fails
+inline int device_malloc(exc_ctx *c, void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return EXC_OK;
+  if (give_back(c)) e = hipMalloc(p, bytes);
+  hipGetLastError();                      // dealt with here: the next launch's check must not find it
+  if (e == hipSuccess) return EXC_OK;
+  *p = nullptr;
+  fprintf(stderr, "exc_lapw: %zu bytes of device memory: %s\n", bytes, hipGetErrorString(e));
+  return EXC_ERR_HIP;
+}
+
+// a library object that takes device memory of its own
+template <typename F>
+inline bool with_memory(exc_ctx *c, F &&create) {
+  if (create()) return true;
+  const bool ok = give_back(c) && create();
+  hipGetLastError();
+  return ok;
+}
+inline int blas_handle(exc_ctx *c, rocblas_handle *h) {
+  if (*h || with_memory(c, [&]() { return rocblas_create_handle(h) == rocblas_status_success; })) return EXC_OK;
+  *h = nullptr;
+  return EXC_ERR_HIP;
+}
+
 template <typename T>
 inline int dev_alloc(exc_ctx *c, T **p, size_t n) {
   *p = nullptr;
   if (n == 0) return EXC_OK;
   void *q = nullptr;
-  EXC_CHECK(hipMalloc(&q, n * sizeof(T)));
+  int rc = device_malloc(c, &q, n * sizeof(T));
+  if (rc) return rc;
   c->owned.push_back(q);
   *p = (T *)q;
   return EXC_OK;
@@ -264,7 +306,7 @@ inline int d2h_cols(exc_ctx *c, char *dst, size_t dld, const char *dsrc, size_t 
 
 // A larger buffer replaces the old one; work already queued on any stream may still read or
 // write the old one, so the device drains before it is freed.
-inline int grow(void **p, size_t *have, size_t need) {
+inline int grow(exc_ctx *c, void **p, size_t *have, size_t need) {
   if (need <= *have) return EXC_OK;
   if (*p) {
     EXC_CHECK(hipDeviceSynchronize());
@@ -272,13 +314,8 @@ inline int grow(void **p, size_t *have, size_t need) {
   }
   *p = nullptr;
   *have = 0;
-  const hipError_t e = hipMalloc(p, need);
-  if (e != hipSuccess) {
-    hipGetLastError();                    // reported here: the next launch's check must not find it again
-    *p = nullptr;
-    fprintf(stderr, "exc_lapw: %zu bytes of workspace: %s\n", need, hipGetErrorString(e));
-    return EXC_ERR_HIP;
-  }
+  int rc = device_malloc(c, p, need);
+  if (rc) return rc;
   *have = need;
   return EXC_OK;
 }

@@ -108,6 +108,7 @@ SIGNATURES = {
     "exc_ctx_set_meffig": [_P, _P],
     "exc_ctx_set_iora": [_P, _P, _P, _P, _P],
     "exc_ctx_crt_form": [_P, _P, _P, _P],
+    "exc_ctx_exact_products": [_P, _P],
     "exc_ctx_set_cfdamp": [_P, C.c_double, C.c_double],
     "exc_gengpvec": [_P, _P, _P, _P, C.c_double, _I, _P, _P, _P, _P, _P, _P],
     "exc_gensfacgp": [_P, _I, _P, _I, _P],
@@ -551,6 +552,12 @@ class Context:
         f, n, s = C.c_int(), C.c_int(), C.c_double()
         self._call("exc_ctx_crt_form", self.h, C.byref(f), C.byref(n), C.byref(s))
         return f.value, n.value, s.value
+
+    def exact_products(self):
+        """Whether the last grouped setup formed its FP64 products as exact integer products."""
+        e = C.c_int()
+        self._call("exc_ctx_exact_products", self.h, C.byref(e))
+        return bool(e.value)
 
     def set_timing(self, on=True):
         self._call("exc_ctx_set_timing", self.h, 1 if on else 0)

@@ -467,6 +467,15 @@ int exc_ctx_set_moduli(exc_ctx *ctx, int n);
  * EXC_BATCH_OLP_LEGENDRE and no h1aa), the built-in choice takes the Gram form unless sigma
  * exceeds half of the largest |eigenvalue| of the h_a.  No reference counterpart. */
 int exc_ctx_crt_form(const exc_ctx *ctx, int *form, int *nmod, double *sigma);
+/* *exact = 1 if the last exc_setup_batched_dev call formed H's (without EXC_BATCH_OLP_LEGENDRE
+ * also O's) muffin-tin products as exact integer products of 57-bit row integers rather than
+ * on FP64 MFMA: what calls without a split flag do where it is faster by their sizes, unless one
+ * k-point's workspace (about 64 natm naa ngp bytes, and 16 ngp^2 for each matrix) is more than half of the free device memory.  The
+ * two differ in rounding only.  Pinning EXC_STAGE_BMT (any variant) keeps a context on FP64
+ * MFMA.  The workspace, at most 4 GiB and an eighth of the free memory (or one
+ * k-point's), is kept for the next call and given back when another allocation of the context
+ * would fail, or with the context.  No reference counterpart. */
+int exc_ctx_exact_products(const exc_ctx *ctx, int *exact);
 /* The first n moduli and beta of the modular split (for a caller's error estimate). */
 int exc_crt_moduli(int n, int *moduli, int *beta);
 
