@@ -644,13 +644,20 @@ int y_narrow(const exc_ctx *c, long tiles, int wide) {
 // FP64 MFMA tiles') instead of on FP64 MFMA.  Per k-point the MFMA tiles take 5.5e-8 K N^2 us, the
 // exact products 1.7e-8 K N^2 (residue GEMM) + 2.4e-5 K N (planes of both operands) + 1.3e-5 N^2
 // (reconstruction), K = natm naa: even near 700 / N + 650 / K = 1.1, with a margin for the tails of
-// smaller grids.  Measured for the whole grouped setup, graph replays (us; MFMA, exact; the left
-// side): K = 1936, N = 700, 8 k-points 1098, 1081-1113 (1.34); 1452, 1100, 4 k 781, 815 (1.08); 1620, 1000, 8 k
-// 1338, 1260 (1.10); 1936, 1200, 4 k 1029, 1027-1040 (0.92); 1936, 1200, 16 k 4167, 3965 (0.92); 2904, 1200, 4 k 1516,
-// 1433 (0.81); 1936, 1600, 16 k 6537, 5812 (0.77); 5808, 1200, 2 k 1898, 1430 (0.70); 2904, 1900, 8 k 6425, 4939
-// (0.59); 3872, 2500, 8 k 14299, 9601 (0.45).
-bool exact_pays(const exc_ctx *c, int maxn) {
-  return maxn > 0 && 700.0 / maxn + 650.0 / ((double)c->d.natm * c->d.naa) <= 0.97;
+// smaller grids.  Over a batch 1 / N is sum N / sum N^2, so that one large basis among small ones, whose
+// planes and tiles are mostly padding, does not take them all along.  Measured for the whole
+// grouped setup, graph replays (us; MFMA, exact; the left side): K = 1936, N = 700, 8 k-points 1098, 1081-1113 (1.34);
+// 1452, 1100, 4 k 781, 815 (1.08); 1620, 1000, 8 k 1338, 1260 (1.10); 1936, 1200, 4 k 1029, 1027-1040 (0.92); 1936,
+// 1200, 16 k 4167, 3965 (0.92); 2904, 1200, 4 k 1516, 1433 (0.81); 1936, 1600, 16 k 6537, 5812 (0.77); 5808, 1200, 2 k
+// 1898, 1430 (0.70); 2904, 1900, 8 k 6425, 4939 (0.59); 3872, 2500, 8 k 14299, 9601 (0.45); 1936, N = 1400 and twelve
+// of 300 900, 1145 (1.49; 0.84 by the largest basis), N = 1400 and sixteen of 100 638, 968 (1.33).
+bool exact_pays(const exc_ctx *c, int nk, const exc_kpoint_dev *ks) {
+  double n = 0.0, n2 = 0.0;
+  for (int k = 0; k < nk; ++k) {
+    n += ks[k].ngp;
+    n2 += (double)ks[k].ngp * ks[k].ngp;
+  }
+  return n2 > 0.0 && 700.0 * n / n2 + 650.0 / ((double)c->d.natm * c->d.naa) <= 0.97;
 }
 
 long tri_tiles(int ngp, int t) {
@@ -954,7 +961,7 @@ int exc_setup_batched_dev(exc_ctx *c, int nk, const exc_kpoint_dev *ks, int flag
   for (int k = 0; k < nk; ++k) maxn = std::max(maxn, ks[k].ngp);
   // the FP64 path by exact integer products (its O tiles take no 'iora*' terms)
   bool exact = !split && !icrt && c->bmt_variant < 0 && c->d.natm * c->d.naa <= 131000 && !(c->d.iora && !olp) &&
-               exact_pays(c, maxn);
+               exact_pays(c, nk, ks);
   const int cv = c->crt_variant >= 0 ? c->crt_variant : (maxn >= 800 && 4 * t256 <= 5 * t128 ? 8 : 4);
   const int ov = c->olp_variant >= 0 ? c->olp_variant : kOlpBcast;   // rows along lanes, columns by DPP broadcast
   int fv = c->fork_variant;
