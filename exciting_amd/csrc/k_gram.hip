@@ -14,6 +14,7 @@
 //    time on the matrix cores (1.82 ms; 2.24 with each step's update applied in the next one's
 //    pass, a read and a write of the matrix a step).
 //  * gram_chol_kernel: left-looking by panels of 16 columns.
+#include "reflector.h"
 #include "wave_sum.h"
 
 namespace {
@@ -90,15 +91,11 @@ __global__ __launch_bounds__(kGT) void gram_extremes_kernel(int n, const cplx *_
 #pragma unroll
       for (int w = 0; w < R; ++w) xn2 += buf[0][w];
       const cplx al = s_alpha;
-      cplx sc = {0.0, 0.0};
-      double beta = al.re;
-      if (xn2 != 0.0 || al.im != 0.0) {
-        beta = -copysign(sqrt(al.re * al.re + al.im * al.im + xn2), al.re);
-        const double bi = 1.0 / beta;
-        tau = cplx{(beta - al.re) * bi, -al.im * bi};
-        const double dr = al.re - beta, di = al.im, q = 1.0 / (dr * dr + di * di);
-        sc = cplx{dr * q, -di * q};
-      }
+      double rf[5];                                     // (a column below 1e-145 counts as zero)
+      reflector(al.re, al.im, xn2, rf);
+      tau = cplx{rf[1], rf[2]};
+      const cplx sc = {rf[3], rf[4]};
+      const double beta = rf[0];
       if (tid == 0) e2[j] = beta * beta;
       vn[tid] = tid == j + 1 ? cplx{1.0, 0.0} : (tid > j + 1 && tid < n) ? cmul(x, sc) : cplx{0.0, 0.0};
     }

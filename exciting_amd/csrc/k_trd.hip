@@ -17,6 +17,7 @@
 // Every kPanel columns trd_update applies V W^H + W V^H to both triangles of the rest (FP64 MFMA).
 // 4 matrices, n = 1258: 17.7 ms (14 us a column); rocSOLVER's zhetrd_strided_batched about 35 (five launches and
 // 27 us a column, 3.4 ms of updates).
+#include "reflector.h"
 #include "wave_sum.h"
 
 namespace {
@@ -175,15 +176,10 @@ __global__ __launch_bounds__(256) void trd_mv_kernel(TrdArgs args, int c, int p)
   xn2 = wave_sum(xn2);
   s0 = cplx{wave_sum(s0.re), wave_sum(s0.im)};
   s1 = cplx{wave_sum(s1.re), wave_sum(s1.im)};
-  cplx tau = {0.0, 0.0}, sc = {0.0, 0.0};
-  double beta = al.re;
-  if (xn2 != 0.0 || al.im != 0.0) {
-    beta = -copysign(sqrt(al.re * al.re + al.im * al.im + xn2), al.re);
-    const double bi = 1.0 / beta;
-    tau = cplx{(beta - al.re) * bi, -al.im * bi};
-    const double dr = al.re - beta, di = al.im, q = 1.0 / (dr * dr + di * di);
-    sc = cplx{dr * q, -di * q};
-  }
+  double rf[5];                                            // (a column below 1e-145 counts as zero)
+  reflector(al.re, al.im, xn2, rf);
+  const cplx tau = {rf[1], rf[2]}, sc = {rf[3], rf[4]};
+  const double beta = rf[0];
   double vav = 0.0;                                        // of v^H A v: conj(v_k) y_k, real part
   __shared__ double sv[4];
   if (work) {
