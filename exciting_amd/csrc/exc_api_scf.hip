@@ -456,7 +456,10 @@ int rhoir_run(exc_ctx *c, int nk, const int *ngp, const int *const *igpig, int n
   if ((rc = scf_prepare(c))) return rc;
   const exc_dev &d = c->d;
   const int N = c->dims.ngrtot;
-  if (exc_rhoir_fits(d)) {                     // the FFT below: a grid whose DFT matrices do not fit in LDS
+  int maxngp = 0;
+  for (int k = 0; k < nk; ++k) maxngp = std::max(maxngp, ngp[k]);
+  // the FFT below: a grid whose DFT matrices do not fit in LDS, or a large one with few states
+  if (exc_rhoir_fits(d) && exc_rhoir_pays(d, maxngp, nst)) {
     if (!c->dft) {
       std::vector<cplx> t((size_t)d.box_n[0] * d.box_n[0] + (size_t)d.box_n[1] * d.box_n[1] +
                           (size_t)d.box_n[2] * d.box_n[2]);
@@ -489,7 +492,7 @@ int rhoir_run(exc_ctx *c, int nk, const int *ngp, const int *const *igpig, int n
   for (int k = 0; k < nk; ++k)
     for (int j0 = 0; j0 < nst; j0 += B) {
       const int nb = std::min(B, nst - j0);
-      EXC_CHECK(hipMemsetAsync(c->zb, 0, sizeof(cplx) * (size_t)B * N, c->stream));
+      if ((rc = exc_launch_rhoir_zero((size_t)B * N, c->zb, c->stream))) return rc;
       if ((rc = exc_launch_rhoir_scatter(d, ngp[k], igpig[k], (const cplx *)evec[k], ldv[k], j0, nb, N, c->zb,
                                          c->stream)))
         return rc;

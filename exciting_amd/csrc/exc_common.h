@@ -243,11 +243,13 @@ int exc_launch_gensfacgp(const exc_dev &d, int ngp, const double *vgpc, int ld, 
 int exc_launch_scf_real(int n, const cplx *z, double *out, hipStream_t s);
 int exc_launch_scf_product(int n, const double *a, const double *b, cplx *z, hipStream_t s);
 int exc_launch_scf_gather(const exc_dev &d, int ngvec, double scale, const cplx *z, cplx *out, hipStream_t s);
+int exc_launch_rhoir_zero(size_t n, cplx *z, hipStream_t s);
 int exc_launch_rhoir_scatter(const exc_dev &d, int ngp, const int *igpig, const cplx *evec, int ldv, int j0, int nb,
                              int N, cplx *z, hipStream_t s);
 int exc_launch_rhoir_accum(int N, int nb, const cplx *z, const double *occ, int j0, double wk, double eps,
                            double omega, double *rho, hipStream_t s);
 bool exc_rhoir_fits(const exc_dev &d);
+bool exc_rhoir_pays(const exc_dev &d, int ngp, int nst);
 size_t exc_rhoir_work_bytes(const exc_dev &d, int nk, int nst, int ncu);
 void exc_rhoir_tables(const exc_dev &d, cplx *f);
 int exc_launch_rhoir(const exc_dev &d, int nk, const int *ngp, const int *const *igpig, int nst, const int *ldv,

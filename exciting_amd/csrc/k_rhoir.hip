@@ -62,8 +62,11 @@ __global__ __launch_bounds__(256) void rhoir_clear_kernel(RhoArgs p) {
   if (i < 6) p.rng[6 * k + i] = i < 3 ? 0x7fffffff : -1;
 }
 
-__global__ __launch_bounds__(256) void rhoir_map_kernel(RhoArgs p) {
-  const int i = blockIdx.x * 256 + threadIdx.x, k = blockIdx.y, n = p.n[0] * p.n[1] * p.n[2];
+// (the ranges by workgroups of 1024: atomics of every wave on the six words took 30 us at 26000 functions)
+constexpr int kMap = 1024;
+__global__ __launch_bounds__(kMap) void rhoir_map_kernel(RhoArgs p) {
+  __shared__ int r[kMap / 64][6];
+  const int i = blockIdx.x * kMap + threadIdx.x, k = blockIdx.y, n = p.n[0] * p.n[1] * p.n[2];
   const int g = i < p.k[k].ngp ? p.k[k].igpig[i] - 1 : -1;
   const bool in = g >= 0 && g < n;
   int s[3] = {0x7fffffff, 0x7fffffff, 0x7fffffff}, h[3] = {-1, -1, -1};
@@ -79,11 +82,19 @@ __global__ __launch_bounds__(256) void rhoir_map_kernel(RhoArgs p) {
       s[q] = min(s[q], __shfl_xor(s[q], o));
       h[q] = max(h[q], __shfl_xor(h[q], o));
     }
-    if ((threadIdx.x & 63) == 0 && h[q] >= 0) {
-      atomicMin(p.rng + 6 * k + q, s[q]);
-      atomicMax(p.rng + 6 * k + 3 + q, h[q]);
+    if ((threadIdx.x & 63) == 0) {
+      r[threadIdx.x >> 6][q] = s[q];
+      r[threadIdx.x >> 6][3 + q] = h[q];
     }
   }
+  __syncthreads();
+  if (threadIdx.x >= 6) return;
+  const bool low = threadIdx.x < 3;
+  int v = r[0][threadIdx.x];
+#pragma unroll
+  for (int w = 1; w < kMap / 64; ++w) v = low ? min(v, r[w][threadIdx.x]) : max(v, r[w][threadIdx.x]);
+  if (low) atomicMin(p.rng + 6 * k + threadIdx.x, v);
+  else atomicMax(p.rng + 6 * k + threadIdx.x, v);
 }
 
 // a wave: 16 columns (s2, s3) of one item, all x
@@ -238,6 +249,24 @@ bool exc_rhoir_fits(const exc_dev &d) {
   return d.box_n[0] <= 16 * kTMax && d.box_n[1] <= 16 * kTMax && d.box_n[2] <= 16 * kTMax;
 }
 
+// Whether the products beat the FFT for nst states of a basis of ngp functions.  A workgroup of
+// rhoir_yz takes a state a wave: with a few states most of it idles behind its loads of the DFT matrices,
+// where the FFT of one state is a short job.  In us, W the complex multiply-adds of a state in
+// millions (edges padded to 16, the basis a ball in the box), G the points in millions: products
+// about 23 + 1.4 W + 0.16 W nst, FFT 28 + 28 G nst; below W = 3 both are mostly launches.  Measured (products, FFT):
+// 48^3 points, N = 5898, 1 state 33, 25, 8 states 40, 57; 60^3, 13335, 1 44, 26, 8 56, 62; 60^3, 2000, 1 31, 27, 8 35, 60;
+// 72^3 (the most padding, and the FFT's best edge), 18688, 8 104, 83, 40 286, 285; 75^3, 26046, 1 88, 46, 8 119, 113, 40
+// 316, 563; 18 x 75 x 75, 5840, 1 42, 28, 8 54, 59; below the line 18 x 18 x 75, 1347, 1 32, 23, 8 40, 32, 16 40, 43.
+bool exc_rhoir_pays(const exc_dev &d, int ngp, int nst) {
+  auto pad = [](int n) { return (n + 15) / 16 * 16.0; };
+  const double n1 = d.box_n[0], n2 = d.box_n[1], n3 = d.box_n[2], g = n1 * n2 * n3;
+  const double f = std::min(1.0, cbrt(ngp / (g * (M_PI / 6.0))));
+  const int m1 = (int)ceil(f * n1), m2 = (int)ceil(f * n2), m3 = (int)ceil(f * n3);
+  const double w = 1e-6 * (pad(d.box_n[0]) * m1 * m2 * m3 +
+                           n1 * pad(d.box_n[1]) * (m2 * pad(m3) + pad(d.box_n[2]) * pad(m3)));
+  return w < 3.0 || nst * (28e-6 * g - 0.16 * w) >= 1.4 * w - 5.0;
+}
+
 // the items (states of all k-points) that z holds at a time: 256 MB, or the 64 states that the batched FFT takes
 static long rho_chunk(size_t n, long items) {
   const long c = std::max((long)((size_t(256) << 20) / (sizeof(cplx) * n)), 64l);
@@ -301,7 +330,7 @@ int exc_launch_rhoir(const exc_dev &d, int nk, const int *ngp, const int *const 
     p.part = (double *)(p.inv + ((size_t)std::min(nk, kKMax) * n + 1) / 2 * 2);
     hipLaunchKernelGGL(rhoir_clear_kernel, dim3((unsigned)((n + 255) / 256), kc), dim3(256), 0, s, p);
     EXC_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(rhoir_map_kernel, dim3((maxngp + 255) / 256, kc), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(rhoir_map_kernel, dim3((maxngp + kMap - 1) / kMap, kc), dim3(kMap), 0, s, p);
     EXC_CHECK(hipGetLastError());
     for (long i0 = 0; i0 < items; i0 += chunk) {
       p.i0 = (int)i0;

@@ -9,6 +9,8 @@
 // zfftifc.f90's convention: forward (sign -1) scaled by 1/N, backward (+1) unscaled.
 #include <math.h>
 
+#include <algorithm>
+
 #include "exc_common.h"
 
 namespace {
@@ -87,6 +89,11 @@ __global__ __launch_bounds__(kST) void scf_gather_kernel(exc_dev d, int ngvec, d
   out[g] = {v.re * scale, v.im * scale};
 }
 
+// (a kernel, not a memset: the caller may be capturing the stream)
+__global__ __launch_bounds__(kST) void rhoir_zero_kernel(size_t n, cplx *z) {
+  for (size_t i = (size_t)blockIdx.x * kST + threadIdx.x; i < n; i += (size_t)gridDim.x * kST) z[i] = cplx{0.0, 0.0};
+}
+
 // z[b N + grid(G_igk)] = evec(igk, j0 + b): the plane-wave coefficients of state j0 + b
 __global__ __launch_bounds__(kST) void rhoir_scatter_kernel(exc_dev d, int ngp, const int *igpig, const cplx *evec,
                                                             int ldv, int j0, int N, cplx *z) {
@@ -98,10 +105,12 @@ __global__ __launch_bounds__(kST) void rhoir_scatter_kernel(exc_dev d, int ngp, 
 }
 
 // rho(r) += sum_b t_b |z_b(r)|^2, t_b = wk occ(j0 + b) / Omega, over the states of the chunk (at
-// most 64) with |wk occ| > eps.  64 points a workgroup, each of its 4 waves every fourth of those
-// states with 4 loads in flight: the grid alone gives about a hundred waves, too few to hide a load
-// (N = 24300, 64 states, 25 MB: 17 us with a thread per point, 5.6 here).
+// most 64) with |wk occ| > eps, 4 loads in flight a wave.  SPLIT waves share 64 points, each every SPLIT-th of
+// those states: a grid of 24300 points alone gives about a hundred waves, too few to hide a load (64 states,
+// 25 MB: 17 us with a thread per point, 5.6 with 4 waves); from 2^17 points a thread per point does (75^3 points,
+// 12 states, the whole density 171 us with 4 waves a point, 163 here).
 constexpr int kAccStates = 64;
+template <int SPLIT>
 __global__ __launch_bounds__(kST) void rhoir_accum_kernel(int N, int nb, const cplx *z, const double *occ, int j0,
                                                           double wk, double eps, double omega, double *rho) {
   __shared__ double t2[kAccStates];
@@ -121,17 +130,21 @@ __global__ __launch_bounds__(kST) void rhoir_accum_kernel(int N, int nb, const c
     if (lane == 0) cnt = __popcll(m);
   }
   __syncthreads();
-  const int n = cnt, r = blockIdx.x * 64 + lane;
+  const int n = cnt, r = SPLIT == 1 ? blockIdx.x * kST + threadIdx.x : blockIdx.x * 64 + lane;
   const cplx *zr = z + min(r, N - 1);
   double s = 0.0;
 #pragma unroll 4
-  for (int i = wave; i < n; i += 4) {
+  for (int i = SPLIT == 1 ? 0 : wave; i < n; i += SPLIT) {
     const cplx v = zr[(size_t)st[i] * N];
     s += t2[i] * (v.re * v.re + v.im * v.im);
   }
-  part[wave][lane] = s;
-  __syncthreads();
-  if (wave == 0 && r < N) rho[r] += ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+  if constexpr (SPLIT == 1) {
+    if (r < N) rho[r] += s;
+  } else {
+    part[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && r < N) rho[r] += ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane];
+  }
 }
 
 inline unsigned blocks(int n) { return (unsigned)((n + kST - 1) / kST); }
@@ -172,6 +185,13 @@ int exc_launch_scf_gather(const exc_dev &d, int ngvec, double scale, const cplx 
   return EXC_OK;
 }
 
+int exc_launch_rhoir_zero(size_t n, cplx *z, hipStream_t s) {
+  if (n == 0) return EXC_OK;
+  hipLaunchKernelGGL(rhoir_zero_kernel, dim3((unsigned)std::min((n + kST - 1) / kST, (size_t)8192)), dim3(kST), 0, s, n, z);
+  EXC_CHECK(hipGetLastError());
+  return EXC_OK;
+}
+
 int exc_launch_rhoir_scatter(const exc_dev &d, int ngp, const int *igpig, const cplx *evec, int ldv, int j0, int nb,
                              int N, cplx *z, hipStream_t s) {
   if (ngp <= 0 || nb <= 0) return EXC_OK;
@@ -185,7 +205,10 @@ int exc_launch_rhoir_accum(int N, int nb, const cplx *z, const double *occ, int 
                            double omega, double *rho, hipStream_t s) {
   if (nb <= 0) return EXC_OK;
   if (nb > kAccStates) return EXC_ERR_ARG;
-  hipLaunchKernelGGL(rhoir_accum_kernel, dim3((N + 63) / 64), dim3(kST), 0, s, N, nb, z, occ, j0, wk, eps, omega, rho);
+  if (N < 1 << 17)
+    hipLaunchKernelGGL(rhoir_accum_kernel<4>, dim3((N + 63) / 64), dim3(kST), 0, s, N, nb, z, occ, j0, wk, eps, omega, rho);
+  else
+    hipLaunchKernelGGL(rhoir_accum_kernel<1>, dim3(blocks(N)), dim3(kST), 0, s, N, nb, z, occ, j0, wk, eps, omega, rho);
   EXC_CHECK(hipGetLastError());
   return EXC_OK;
 }
