@@ -111,6 +111,12 @@ def crt_alg_ops(cr, ngps, nmod, share):
     return sum(2.0 * 2 * nmod * K * n * (n + 1) / 2 for n in ngps) * (2 * share)
 
 
+def pinned(tuned, stage):
+    """The variant `tuned` pins for a stage; None where the library's own rule decides (no entry, or -1)."""
+    v = (tuned or {}).get(stage, -1)
+    return v if v >= 0 else None
+
+
 def crt_gemm_name(ngps, pinned=None):
     """The residue GEMM that runs: variants 8 to 10 are the register-pipelined kernel on 256-wide tiles, which
     the library takes by itself from N = 800 unless they cover over a quarter more than 128-wide ones."""
@@ -177,7 +183,7 @@ def run_split(args, ctx, batch, cr, w, fp64_value, e0, log, olpflag=0, kind="crt
         form, nmod, sigma = ctx.crt_form()
         ms = eager["crtgemm"][0]
         ops = crt_alg_ops(cr, ngps, nmod, share)
-        gname = crt_gemm_name(ngps, (tuned or {}).get("crtgemm"))
+        gname = crt_gemm_name(ngps, pinned(tuned, "crtgemm"))
         roof = {"bound": "mfma", "kernel": f"{gname} (residue products, {nmod} moduli, int8 MFMA)",
                 "achieved": ops / (ms * 1e-3) / 1e12, "peak": PEAK_INT8 / 1e12, "unit": "TOP/s",
                 "frac": ops / (ms * 1e-3) / PEAK_INT8, "fp64_equivalent_TFLOPs": fl64 / (ms * 1e-3) / 1e12,
@@ -648,10 +654,9 @@ def main():
         mt_ms, mt_cnt = tim["mt"]
         fl = sum(mt_flops(cr, kp.ngp) for kp in w.kpoints) * args.steps
     achieved = fl / (mt_ms * 1e-3) if mt_ms > 0 else 0.0
-    # the grouped MT variants 0, 2, 3 (0 is the default) form each complex product from three
-    # real MFMA products (Gauss's form) instead of four: they execute 6 of the 8 algorithmic flops
-    bmt_v = (tuned or {}).get("bmt", 0)
-    gauss = args.path == "batched" and bmt_v in (0, 2, 3)
+    # the grouped MT tiles but variant 1 (the library's own choices among them) form each complex product
+    # from three real MFMA products (Gauss's form) instead of four: they execute 6 of the 8 algorithmic flops
+    gauss = args.path == "batched" and pinned(tuned, "bmt") != 1
     roof = {"bound": "mfma", "achieved": achieved / 1e12, "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
             "frac": achieved / PEAK_FP64, "traffic": None,
             "kernel": ("bmt_dma_grid_kernel (grouped, all k)" if args.path == "batched" else "mt_dma_kernel (per k)")
@@ -665,10 +670,10 @@ def main():
     if exact:
         ngps = [kp.ngp for kp in w.kpoints]
         gemm_ms, ops = eager["crtgemm"][0], crt_alg_ops(cr, ngps, 16, share)
-        roof = {"bound": "mfma", "kernel": f"{crt_gemm_name(ngps)} (FP64 contraction as exact integer products, 16 "
+        roof = {"bound": "mfma", "kernel": f"{crt_gemm_name(ngps, pinned(tuned, "crtgemm"))} (FP64 contraction as exact integer products, 16 "
                                            "moduli, int8 MFMA)",
                 "achieved": ops / (gemm_ms * 1e-3) / 1e12, "peak": PEAK_INT8 / 1e12, "unit": "TOP/s",
-                "frac": ops / (gemm_ms * 1e-3) / PEAK_INT8, "traffic": None, "per_launch_ops": ops,
+                "frac": ops / (gemm_ms * 1e-3) / PEAK_INT8, "traffic": None, "per_launch_ops": ops / eager["crtgemm"][1],
                 "fp64_equivalent_TFLOPs": fl / (gemm_ms * 1e-3) / 1e12}
     # HBM traffic of the dominant kernel: rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of this same
     # default command, scaled by a 1 GiB copy (committed summary); only for the profiled setup
