@@ -197,9 +197,12 @@ inline int device_malloc(exc_ctx *c, void **p, size_t bytes) {
   return EXC_ERR_HIP;
 }
 
-// a library object that takes device memory of its own
+// A library object that takes device memory of its own.  hipBLASLt ends the process when its handle's
+// memory cannot be had, so the spare memory is given back before it comes to that.
 template <typename F>
 inline bool with_memory(exc_ctx *c, F &&create) {
+  size_t fr = 0, total = 0;
+  if (hipMemGetInfo(&fr, &total) == hipSuccess && fr < (size_t)1 << 30) give_back(c);
   if (create()) return true;
   const bool ok = give_back(c) && create();
   hipGetLastError();

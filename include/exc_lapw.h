@@ -474,7 +474,8 @@ int exc_ctx_crt_form(const exc_ctx *ctx, int *form, int *nmod, double *sigma);
  * two differ in rounding only.  Pinning EXC_STAGE_BMT (any variant) keeps a context on FP64
  * MFMA.  The workspace, at most 4 GiB and an eighth of the free memory (or one
  * k-point's), is kept for the next call and given back when another allocation of the context
- * would fail, or with the context.  No reference counterpart. */
+ * would fail (unless a graph of the caller's has recorded a call that used it), or with the
+ * context.  No reference counterpart. */
 int exc_ctx_exact_products(const exc_ctx *ctx, int *exact);
 /* The first n moduli and beta of the modular split (for a caller's error estimate). */
 int exc_crt_moduli(int n, int *moduli, int *beta);

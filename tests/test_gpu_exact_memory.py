@@ -101,9 +101,6 @@ def test_workspace_given_back(load):
     ref = [torch.linalg.eigvalsh(h.cpu())[:nev] for h in H]
     with torch.cuda.stream(s):
         b = lapw.DeviceBatch(cr, kps)
-    small = [torch.eye(20, dtype=torch.complex128, device="cuda")] * 2       # the libraries' own memory
-    ctx.eigen_batched_dev([20], small[:1], small[1:], nev, ev[:1], [torch.zeros((nev, 20), dtype=torch.complex128,
-                                                                               device="cuda")])
     _run(ctx, b)
     first = [t.clone() for t in b.H + b.O]
     assert ctx.exact_products()
@@ -121,4 +118,48 @@ def test_workspace_given_back(load):
     assert ctx.exact_products()
     for x, y in zip(b.H + b.O, first):
         assert torch.equal(x, y)
+    ctx.close()
+
+
+def test_workspace_in_a_graph_of_the_callers(load):
+    """A graph the caller records around an eager call holds the workspace's addresses: an allocation
+    that does not fit then fails, and the graph's replays keep their bits."""
+    import torch
+    from exciting_amd import lapw
+    cr, kps = load
+    s = torch.cuda.Stream()
+    ctx = lapw.Context(cr, stream=s)
+    flags = lapw.EXC_BATCH_MATCH | lapw.EXC_BATCH_OLP_LEGENDRE
+    with torch.cuda.stream(s):
+        b = lapw.DeviceBatch(cr, kps)
+        ctx.setup_batched_dev(b, flags)
+        torch.cuda.synchronize()
+        assert ctx.exact_products()
+        first = [t.clone() for t in b.H + b.O]
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        ctx.setup_batched_dev(b, flags)
+    # the adjoint's workspace, 16 (2 nst natm naa + 3 nst ngp) bytes, is allocated at its first call
+    d, nst = b.dks[0], 4000
+    C = torch.zeros((nst, b.nmat[0]), dtype=torch.complex128, device="cuda")
+    wt = torch.zeros(nst, dtype=torch.float64, device="cuda")
+    dt = torch.zeros((cr.natm, 3), dtype=torch.float64, device="cuda")
+    dv = torch.zeros(cr.ngvec, dtype=torch.complex128, device="cuda")
+    hog = _leave(100 << 20)
+    print("an adjoint that does not fit, beside a recorded graph", flush=True)
+    with pytest.raises(lapw.ExcError) as ei:
+        ctx.vjp_dev(d.ngp, d.ngkmax, b.apw[0], d.igpig, d.vgpc, d.sfacgp, C, b.nmat[0], nst, wt, wt, dt, dv)
+    assert ei.value.code == lapw.EXC_ERR_HIP
+    del hog
+    torch.cuda.empty_cache()
+    for i in range(3):
+        for t in b.H + b.O:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        print(f"replay {i}", flush=True)
+        g.replay()
+        torch.cuda.synchronize()
+        for x, y in zip(b.H + b.O, first):
+            assert torch.equal(x, y)
     ctx.close()
