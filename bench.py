@@ -670,8 +670,8 @@ def main():
     if exact:
         ngps = [kp.ngp for kp in w.kpoints]
         gemm_ms, ops = eager["crtgemm"][0], crt_alg_ops(cr, ngps, 16, share)
-        roof = {"bound": "mfma", "kernel": f"{crt_gemm_name(ngps, pinned(tuned, "crtgemm"))} (FP64 contraction as exact integer products, 16 "
-                                           "moduli, int8 MFMA)",
+        name = crt_gemm_name(ngps, pinned(tuned, "crtgemm"))
+        roof = {"bound": "mfma", "kernel": f"{name} (FP64 contraction as exact integer products, 16 moduli, int8 MFMA)",
                 "achieved": ops / (gemm_ms * 1e-3) / 1e12, "peak": PEAK_INT8 / 1e12, "unit": "TOP/s",
                 "frac": ops / (gemm_ms * 1e-3) / PEAK_INT8, "traffic": None, "per_launch_ops": ops / eager["crtgemm"][1],
                 "fp64_equivalent_TFLOPs": fl / (gemm_ms * 1e-3) / 1e12}
