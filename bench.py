@@ -678,14 +678,17 @@ def main():
     # HBM traffic of the dominant kernel: rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of this same
     # default command, scaled by a 1 GiB copy (committed summary); only for the profiled setup
     prof = HERE / "profiles" / f"setup_kernels_workload{args.config}.json"
-    if (args.path == "batched" and not exact and args.nk is None and not args.tune and not args.set and olpflag
-            and prof.exists()):
-        rec = json.loads(prof.read_text()).get("bmt_dma_grid_kernel")
+    if args.path == "batched" and args.nk is None and not args.tune and not args.set and olpflag and prof.exists():
+        rec = json.loads(prof.read_text()).get("crt_gemm_pipe_kernel, 16 moduli" if exact else "bmt_dma_grid_kernel")
         if rec:
             roof["traffic"] = rec["fetch_bytes"] + rec["write_bytes"]
             roof["traffic_source"] = str(prof.relative_to(HERE))
-            roof["algorithmic_bytes"] = sum(32.0 * kp.ngp * cr.natm * cr.maxaa + 16.0 * kp.ngp ** 2
-                                            for kp in w.kpoints)
+            # both operands and the written triangle and mirror; the exact products': both operands' planes
+            # and the residues, a launch each k-point
+            K = cr.natm * cr.maxaa
+            each = [64.0 * n * K + 16.0 * n * n if exact else 32.0 * n * K + 16.0 * n * n for n in
+                    (kp.ngp for kp in w.kpoints)]
+            roof["algorithmic_bytes"] = sum(each) / (eager["crtgemm"][1] if exact else 1)
     stages = {k: {"ms_per_launch": (ms / cnt if cnt else None), "launches": cnt} for k, (ms, cnt) in tim.items() if cnt}
     if eager:
         stages["grouped_eager_pass"] = {k: ms for k, (ms, cnt) in eager.items() if cnt}

@@ -2,10 +2,16 @@
 //
 // H_MT = conj(A) Yt^T (and O_MT = conj(A) A^T) from exact integer products instead of FP64
 // MFMA, the other terms of the setup staying FP64.  The plain FP64 path takes the same route at
-// large sizes with 16 moduli (beta = 57, exc_setup_batched_dev's exact_pays): every element down
-// to 2^-4 of its row's 2-norm then enters with all its 53 bits, and rows the integers cannot
+// large sizes with 16 moduli (beta = 57, exc_setup_batched_dev's exact_pays); rows the integers cannot
 // represent (not finite, norms outside 1e-125 .. 1e145) are marked and their tiles left to
-// FP64 MFMA (bmt_fix_kernel):
+// FP64 MFMA (bmt_fix_kernel).  An element then enters with an absolute error of 2^-58 of the power of
+// two above its row's norm: with all its 53 bits down to 2^-4 of the norm, with 45 at 2^-12, about the
+// median element of an lmax 10 basis.  The sums are exact, so H_ij is within 2^-56 sqrt(2K) |A_i| |Yt_j|
+// and one rounding: a bound relative to the rows' norms, not to H_ij.  (8 atoms, lmax 10, N = 260, against 80-bit
+// sums, per |A_i| |Yt_j|: rms 7e-18, largest 2.3e-17; FP64 products 3.3e-17, 1.4e-16; 5 of 100
+// elements come out further off than by FP64, the smallest of a row by up to a digit of their own.)
+//
+// The steps:
 //
 //  scale : per row i of an operand X (N x K complex, K = natm naa) the exponent e_i with
 //          |X_i|_2 < 2^e_i and s_i = beta - e_i, beta the largest with 2^(2 beta + 2) <= P,
@@ -13,13 +19,13 @@
 //  split : X'_ik = rint(Re X_ik 2^s_i) + i rint(Im X_ik 2^s_i), exact integers below 2^beta.
 //          Every modulus m is odd with prime factors 1 mod 4, so it has a square root iota of
 //          -1 and Z_m[i] splits into two copies of Z_m by the ring maps x + iy -> x +- iota y.
-//          Per modulus the two planes of an operand are those maps, as symmetric int8
-//          residues: Re X' - iota Im X' and Re X' + iota Im X' for the conjugated left operand,
+//          Per modulus the two planes of an operand are those maps, as int8 residues (within
+//          m / 2 + 2 of zero, lowres): Re X' - iota Im X' and Re X' + iota Im X' for the conjugated left operand,
 //          Re X' + iota Im X' and Re X' - iota Im X' for the right one; layout
 //          [m][plane][K/16][row][16 bytes]: one 16-byte k-chunk of 64 consecutive rows is one
 //          1 KiB wave-wide DMA.
 //  gemm  : per modulus, tile and map, U = u_a u_b^T or V = v_a v_b^T by
-//          v_mfma_i32_32x32x32_i8 with exact int32 accumulation (|P| <= K 120^2 < 2^31),
+//          v_mfma_i32_32x32x32_i8 with exact int32 accumulation (|P| <= K 122^2 < 2^31),
 //          reduced modulo m to int8 residues: two real products per modulus, where Gauss's
 //          form needs three.
 //  merge : per tile element Re = (U + V)/2, Im = (U - V)/(2 iota) modulo each m, then
@@ -45,14 +51,12 @@
 namespace {
 
 using setup_dev::GTab;
-using setup_dev::lookup_g;
 using setup_dev::stage_barrier;
 using setup_dev::wait_vm_lgkm0;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void;
-
 
 // symmetric residue of an exact integer held in a double, |x| < 2^52, modulo an odd m
 // (|x/m| is never within 1/(2m) of a half-integer, far above the rounding of x/m)

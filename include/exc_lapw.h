@@ -243,8 +243,11 @@ typedef struct exc_kpoint_dev {
                                  /* rounded differently); H is unchanged                         */
 
 /* match (optional) + H and O of nk k-points, each with its own basis size, in one grouped
- * launch per stage on the context's stream; the muffin-tin stage is a persistent kernel over
- * a work list of (k, tile, H/O) items.  Results equal nk calls of the per-k entry points. */
+ * launch per stage on the context's stream; the muffin-tin stage takes a work list of (k, tile,
+ * H/O) items.  Results equal nk calls of the per-k entry points to rounding: the tiles, and
+ * whether H's products run as exact integers (exc_ctx_exact_products), go by what the whole
+ * batch holds, so that a k-point's last bits can depend on the k-points beside it.  Pinned
+ * variants (exc_ctx_set_variant) do not. */
 int exc_setup_batched_dev(exc_ctx *ctx, int nk, const exc_kpoint_dev *ks, int flags);
 
 /* Adjoint of the setup (forcek.f90:13, the IBS force term of one k-point).
