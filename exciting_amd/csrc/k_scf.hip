@@ -1,7 +1,7 @@
 // Per-SCF producers of the interstitial tables the setup reads: Theta(G) and Theta(r)
 // (gencfun.f90:52-96, cfdamp = 0) and V(G) (genveffig.f90:23-33); and the interstitial
-// density of the occupied states (genrhoir.f90:28-89) on grids with an edge above 80 points (the smaller
-// ones: k_rhoir.hip): a chunk of states is scattered to the grid, transformed backward in one batched FFT and
+// density of the occupied states (genrhoir.f90:28-89) on grids with an edge above 80 points and on large ones with
+// few states (the others: k_rhoir.hip): a chunk of states is scattered to the grid, transformed backward in one batched FFT and
 // |psi|^2 accumulated per grid point.
 // The FFT grid is the G box of the context (ngrid(i) = box extent, every grid point one G);
 // position of G on the grid j1 + n1 (j2 + n2 j3) with negative components wrapped to n + i

@@ -367,7 +367,9 @@ int exc_rhovalk(exc_ctx *ctx, int lradstep, const double *zbshtvr, const double 
  * on the FFT grid of exc_ctx_gencfun (the G box), rhoir(ngrtot) accumulated.  _dev: device
  * arrays (evecfv(ldv, nst), occ(nst), igpig(ngp) 1-based), on the context's stream; the
  * batched form takes ngp and igpig from ks[k] and one evecfv, occ, wkpt per k-point, with the
- * states of every k-point transformed in batches of 64; without _dev: host arrays. */
+ * states of every k-point transformed by products with the grid's DFT matrices, or, on grids
+ * with an edge above 80 points and large ones with few states, by FFTs of up to 64 states at
+ * a time; without _dev: host arrays. */
 int exc_genrhoir_dev(exc_ctx *ctx, int ngp, const int *igpig, int nst, int ldv, const double *evecfv,
                      const double *occ, double wkpt, double epsocc, double *rhoir);
 int exc_genrhoir_batched_dev(exc_ctx *ctx, int nk, const exc_kpoint_dev *ks, int nst, const int *ldv,
