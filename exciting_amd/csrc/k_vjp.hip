@@ -22,7 +22,7 @@
 // per (atom, state) 119 and the pairs times all atoms with four atomics each 788.
 // U and the product back take three real products per complex one (Gauss), which round the imaginary
 // parts more than the library's four did; dE/dtau as a whole came closer to 64-bit values all the same (16 atoms, N = 2500:
-// 4.0e-15 -> 3.2e-15 relative), since the derivative's factor enters once instead of in three products.
+// 4.0e-15 -> 3.2e-15 relative).
 #include "setup_dev.h"
 #include "mt_dma.h"
 
